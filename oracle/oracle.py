@@ -19,13 +19,14 @@ _DVODE = None
 # by `make ref` wherever the reference's sources are present
 DVODE_REF = os.path.join(_HERE, "_ref", "libdvode_ref.so")
 REFERENCE = "/root/reference"
+DVODE_F = os.path.join("store", "therm_lib", "chemkin", "core", "dvode.f")
 
 
 def build(force: bool = False) -> str:
     so = os.path.join(_HERE, "liboracle.so")
     if force or not os.path.exists(so):
         subprocess.run(["make", "-s", "-C", _HERE] + (["-B"] if force else []), check=True)
-    if os.path.isdir(REFERENCE) and (force or not os.path.exists(DVODE_REF)):
+    if os.path.exists(os.path.join(REFERENCE, DVODE_F)) and (force or not os.path.exists(DVODE_REF)):
         subprocess.run(["make", "-s", "-C", _HERE, "ref", "REF=" + REFERENCE] + (["-B"] if force else []),
                        check=True)
     return so
