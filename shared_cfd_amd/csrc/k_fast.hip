@@ -16,7 +16,9 @@
 //
 // Layout: a "quad strip" is 16 rows of one block owned by one wavefront;
 // lane L = 4r+c holds component c of row r.  Row r processes column
-// i = d-r+1 at step d, so the 16 rows of a step lie on an anti-diagonal.
+// i = d-r-floor(r/4)+1 at step d: the rows of a step lie on an anti-diagonal,
+// with one extra step between the groups of four rows that share a 16-lane
+// row of the wavefront (see the sweep schedule below).
 // Per-cell coefficients are stored by (strip, d, lane) -- the "skewed
 // layout" -- so every step of both sweeps reads 64 consecutive slots.
 //
@@ -33,12 +35,14 @@
 namespace shcfd {
 
 constexpr int QR = 16;  // rows per quad strip
-constexpr int CH = 16;  // steps per unrolled sweep chunk (padding unit)
+constexpr int CH = 16;  // steps a strip is padded to (padding unit)
+constexpr int GD = 1;   // extra steps between the four-row groups of a strip
+constexpr int SPAN = QR - 1 + 3 * GD;  // steps row 15 runs behind row 0
 
 struct QStrip {
     int b, j0, prev, next;
     long long base;  // slot of (step 0, lane 0); multiple of 128
-    int nch, pad;    // chunks of CH steps covering the ni + QR - 1 steps
+    int nch, pad;    // chunks of CH steps covering the ni + SPAN steps
 };
 
 // slot of the one-double arrays for (step dd, lane L): pair-interleaved
@@ -94,7 +98,7 @@ __device__ inline PostScal post_scal(const DevCtx& d, long long c) {
 
 // cell of slot (strip S, step d, row r)
 __device__ inline bool slot_cell(const QStrip& S, const DevBlock& B, int d, int r, int& i, int& j) {
-    i = d - r + 1;
+    i = d - r - GD * (r >> 2) + 1;
     j = S.j0 + r;
     return i >= 1 && i <= B.ni && j <= B.nj;
 }
@@ -111,8 +115,11 @@ constexpr unsigned long long SENTINEL = 0x7FF4DEADBEEFCAFEULL;
 constexpr int HOFF = 48;
 
 // Operator arrays G = (GA, GB) and H = (HA, HB): per step a 4 KB block of
-// four 1 KB parts, part p holding doubles (2p', 2p'+1) of every lane's row,
+// four 1 KB parts, part p holding elements (2p', 2p'+1) of every lane's row,
 // p = 2*(0 for A, 1 for B) + p'; lane L's pair sits at 16 L in its part.
+// Element m of lane 4r+k is that of column (k + m) mod 4: the lane's own
+// component comes first and needs no broadcast, the others come by one DPP
+// quad rotation each.
 // Each 16-byte load of a sweep step then reads 1 KB of consecutive bytes.
 __device__ inline long long op_index(const QStrip& S, int dd, int L, int p, int e) {
     return (S.base / 64 + dd) * 512 + p * 128 + 2 * L + e;
@@ -135,7 +142,8 @@ __device__ inline void prep_ops(const DevCtx& d, const QStrip& S, int dd, int r,
     if (Dn)
         *reinterpret_cast<double2*>(&Dn[(S.base / 64 + dd) * 32 + 2 * r]) =
             make_double2(-(fa * J.nuA), -(fb * J.nuB));
-    // rows of the operators: lane 4r+k holds row k (4 doubles)
+    // rows of the operators: lane 4r+k holds row k (4 doubles), element m the
+    // one of column (k + m) mod 4
     const double* mats[4] = {J.Ap, J.Bp, J.Am, J.Bm};
     const double fs[2] = {fa, fb};
 #pragma unroll
@@ -143,13 +151,13 @@ __device__ inline void prep_ops(const DevCtx& d, const QStrip& S, int dd, int r,
         double* o = m < 2 ? G : H;
         if (!o) continue;
         mm4(mats[m], Sm, T);
-        // doubles (2p', 2p'+1) of a lane's row are adjacent: one 16-byte store
+        // elements (2p', 2p'+1) of a lane's row are adjacent: one 16-byte store
 #pragma unroll
         for (int k = 0; k < 4; k++)
 #pragma unroll
             for (int lp = 0; lp < 2; lp++)
                 *reinterpret_cast<double2*>(&o[op_index(S, dd, 4 * r + k, 2 * (m & 1) + lp, 0)]) =
-                    make_double2(fs[m & 1] * T[k + 4 * (2 * lp)], fs[m & 1] * T[k + 4 * (2 * lp + 1)]);
+                    make_double2(fs[m & 1] * T[k + 4 * ((k + 2 * lp) & 3)], fs[m & 1] * T[k + 4 * ((k + 2 * lp + 1) & 3)]);
     }
 }
 
@@ -232,35 +240,14 @@ __global__ void __launch_bounds__(256) k_fast_rhs_prep(DevCtx d, const QStrip* s
 }
 
 // ---------------------------------------------------------------------------
-// Hand-off between quad strips.  The producer's boundary row stores its
-// outgoing contribution with an agent-coherent 64-bit store into a slot that
-// holds a signalling-NaN sentinel (filled by k_fast_rhs_prep before every
-// sweep); the consumer polls the slot until the sentinel is gone.  No flag
-// and no store-completion wait is needed, so the producer never drains its
-// load pipeline.  Arithmetic never produces this NaN payload.
+// Hand-off between quad strips.  The producer stores the outgoing
+// contribution of its boundary row with agent-coherent 64-bit stores into a
+// row whose slots hold a signalling-NaN sentinel (filled before every sweep);
+// the consumer polls the slots until the sentinel is gone.  No flag and no
+// store-completion wait is needed.  Arithmetic never produces this NaN
+// payload.
 // ---------------------------------------------------------------------------
 __device__ inline bool is_sentinel(double x) { return (unsigned long long)__double_as_longlong(x) == SENTINEL; }
-
-// wave-uniform: poll until the lanes `mine` read a non-sentinel value from
-// their slot.  Past the bound it raises SHCFD_E_SPIN and goes on with zero,
-// so the sweep still runs to its end (no early exit from the step loop).
-__device__ inline void handoff_wait(double& x, const double* slotp, bool mine, long long spin_limit, int* iflag) {
-    long long it = 0;
-    while (__ballot(mine && is_sentinel(x)) != 0ULL) {
-        if (it++ >= spin_limit) {
-            atomicCAS(iflag + IFLAG_ERR, 0, SHCFD_E_SPIN);
-            x = 0.0;
-            break;
-        }
-        __builtin_amdgcn_s_sleep(2);
-        x = load_agent(slotp);
-    }
-}
-
-// wait for every outstanding vector memory access of the wave (vmcnt(0),
-// other counters left alone)
-__device__ inline void wait_all_vmem() { __builtin_amdgcn_s_waitcnt(0x0F70); }
-
 
 // Buffer views.  Each sweep addresses its strip through buffer resources
 // (base in scalar registers, 32-bit lane offset, per-step offsets in scalar
@@ -288,9 +275,9 @@ __device__ inline void st_pair(__amdgpu_buffer_rsrc_t r, double2 x, int voff, in
     const shcfd_u32x4 v = {(unsigned)a, (unsigned)(a >> 32), (unsigned)b, (unsigned)(b >> 32)};
     __builtin_amdgcn_raw_buffer_store_b128(v, r, voff, soff, 0);
 }
-__device__ inline double ld_agent(__amdgpu_buffer_rsrc_t r, int voff, int soff) {
-    const shcfd_u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, AUX_AGENT);
-    return u2d(v.x, v.y);
+__device__ inline double2 ld_agent2(__amdgpu_buffer_rsrc_t r, int voff, int soff) {
+    const shcfd_u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, AUX_AGENT);
+    return make_double2(u2d(v.x, v.y), u2d(v.z, v.w));
 }
 __device__ inline void st_agent(__amdgpu_buffer_rsrc_t r, double x, int voff, int soff) {
     const unsigned long long a = (unsigned long long)__double_as_longlong(x);
@@ -305,25 +292,46 @@ __device__ inline int pair_off(int dd) { return (dd + CH) * 512; }
 __device__ inline int dn_off(int dd) { return (dd + CH) * 256; }
 __device__ inline int col_off(int col) { return (col + HOFF) * 32; }
 
-// Sweep schedule.  A sweep workgroup has two wavefronts on one CU: wave 0
-// computes, wave 1 streams the strip's operator blocks and R/X pairs into LDS
-// with LDS-DMA loads (buffer_load ... lds), CS steps per chunk, NSLOT chunk
-// slots.  The vector-memory path of a CU moves about 64 bytes per cycle, and
-// a step needs 4.5 KB of operators: issued by the computing wave, those loads
-// stall its dependency chain; issued by a second wave they overlap it.  The
-// waves meet at one s_barrier per chunk: before it the loader has waited for
-// the chunk the compute wave reads next, and the compute wave has finished
-// reading the slot the loader refills next.  The compute wave keeps the
-// hand-off ring (PH steps of device-coherent loads), its V/Z stores and the
-// hand-off stores.  Its step body is straight-line code; a hand-off miss takes
-// a rare uniform branch that polls the one column and then drains all
-// outstanding accesses, so it leaves no pending state for the common path.
+// Sweep schedule.  A sweep workgroup has four wavefronts, one per SIMD of its
+// CU, that meet at one s_barrier per chunk of CS steps:
+//   * wave 0 computes.  It touches global memory only to store V/Z, so it
+//     never waits for a vector-memory access: operators, right-hand sides and
+//     hand-offs all come from LDS;
+//   * wave 1 streams the strip's operator blocks and R/X pairs into LDS with
+//     LDS-DMA loads (buffer_load ... lds), three chunk slots ahead.  A step
+//     needs 4.5 KB of operators, and a CU's vector-memory path moves about 64
+//     bytes per cycle;
+//   * wave 2 takes the neighbour strip's hand-off row: it polls device memory
+//     and puts each chunk's columns into an LDS ring;
+//   * wave 3 stores the strip's own outgoing columns from that ring.
+// In one wave the polling loads and the stores share the in-order vmcnt: each
+// ring load then waits for the stores before it, which cost the compute wave
+// a third of its time.
+//
+// What bounds the sweep is the issue of the compute wave: 9 FP64 operations
+// (about 8 cycles each), 8 DPP moves and 7 LDS accesses per step, 148 cycles
+// in isolation and 170 beside the loader, against a dependent chain of about
+// 105 (v -> quad rotations -> four multiply-adds -> the neighbour row's lanes
+// -> next v).  So the operator rows are stored rotated (own component first:
+// 6 moves instead of 8 broadcasts), the next right-hand side opens the chain
+// of a, and the neighbour value is read before the operators, which the step
+// after next needs.  Within a 16-lane row of the wavefront (four grid rows)
+// the hop to the next row is one DPP row shift.  Between those groups it would
+// take a chain of whole-wave shifts, so the groups run GD = 1 step apart and
+// the value crosses through LDS: 3 more steps per strip against 3 dependent
+// DPP moves per step.
+//
+// Measured, forward / backward us per launch: 258,048-cell forward step 167 /
+// 152 -> 130 / 118; 512x128 C-mesh 84 / 87 -> 65 / 66; 400x4 tube 46 / 47 ->
+// 32 / 32 (one strip: 112 -> 75 ns per step).  A hop between strips costs 18
+// steps of skew, up to 5 of chunk granularity and 1.3 us from the producer's
+// store to the consumer's look.
 constexpr int CS = 4;                                   // steps per LDS chunk
-constexpr int NSLOT = 3;                                // LDS chunk slots
 constexpr int SLOT_G = CS * 4096;                       // operator bytes per slot
 constexpr int SLOT_DN = SLOT_G + (CS / 2) * 1024;       // + R/X step pairs
 constexpr int SLOT_BYTES = SLOT_DN + CS * 256;          // + diagonal terms (backward sweep with S = I)
 constexpr int LD_PER_CHUNK = 4 * CS + CS / 2;           // LDS-DMA loads per chunk, + 1 with Dn
+static_assert(3 * CS <= CH, "chunks read past a strip's end fall in its guard steps");
 static_assert(CS * 256 == 1024, "one LDS-DMA load carries a chunk's diagonal terms");
 
 typedef __attribute__((address_space(3))) void lds_void;
@@ -331,8 +339,13 @@ typedef __attribute__((address_space(3))) void lds_void;
 __device__ inline void lds_dma(__amdgpu_buffer_rsrc_t r, char* lds, int voff, int soff) {
     __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void*)lds, 16, voff, soff, 0, 0);
 }
-// s_barrier that the compiler may not move memory accesses across
+// the compiler keeps LDS accesses on their side of this point (everything
+// else may cross)
+__device__ inline void ds_order() { __builtin_amdgcn_sched_barrier(0x7F); }
+// s_barrier that the compiler may not move memory accesses across; the second
+// form first waits until the last LDS access of the wave alone is outstanding
 __device__ inline void wg_barrier() { asm volatile("s_barrier" ::: "memory"); }
+__device__ inline void chunk_barrier() { asm volatile("s_waitcnt lgkmcnt(1)\n\ts_barrier" ::: "memory"); }
 // wait until at most N vector memory accesses of this wave are outstanding
 template <int N>
 __device__ inline void wait_vmcnt() {
@@ -342,11 +355,10 @@ __device__ inline void wait_vmcnt() {
 __device__ inline void wait_lgkm0() { __builtin_amdgcn_s_waitcnt(0xC07F); }
 
 // loader wave: chunk j = aligned block m of CS steps (steps CS*m .. CS*m+CS-1)
-// into slot j % NSLOT; the caller orders blocks (ascending or descending)
+// into an LDS slot; the caller orders blocks (ascending or descending)
 template <bool DN>
 __device__ inline void load_block(__amdgpu_buffer_rsrc_t rop, __amdgpu_buffer_rsrc_t rpair, __amdgpu_buffer_rsrc_t rdn,
-                                  char* lds, int j, int m, int vl) {
-    char* slot = lds + (j % NSLOT) * SLOT_BYTES;
+                                  char* slot, int m, int vl) {
 #pragma unroll
     for (int t = 0; t < CS; t++)
 #pragma unroll
@@ -356,174 +368,299 @@ __device__ inline void load_block(__amdgpu_buffer_rsrc_t rop, __amdgpu_buffer_rs
     if constexpr (DN) lds_dma(rdn, slot + SLOT_DN, vl, dn_off(CS * m));
 }
 
-// loader side of the chunk protocol: nck chunks, block of chunk j = blk(j);
-// DN: the chunks also carry the backward sweep's diagonal terms
-template <bool DN, typename BLK>
-__device__ inline void loader(__amdgpu_buffer_rsrc_t rop, __amdgpu_buffer_rsrc_t rpair, __amdgpu_buffer_rsrc_t rdn,
-                              char* lds, int nck, int vl, BLK blk) {
+// wave 1: NS chunk slots, block of chunk j = blk(j); DN: the chunks also carry
+// the backward sweep's diagonal terms.  Chunk j's last operators are read
+// during chunk j, the others during chunk j - 1, so chunk j + NS - 1 takes the
+// slot of chunk j - 1 while chunk j is computed.
+template <int NS, bool DN, typename BLK>
+__device__ inline void sweep_loader(__amdgpu_buffer_rsrc_t rop, __amdgpu_buffer_rsrc_t rpair,
+                                    __amdgpu_buffer_rsrc_t rdn, char* lds, int nck, int vl, BLK blk) {
     constexpr int LD = LD_PER_CHUNK + (DN ? 1 : 0);
-    load_block<DN>(rop, rpair, rdn, lds, 0, blk(0), vl);
-    load_block<DN>(rop, rpair, rdn, lds, 1, blk(1), vl);
-    load_block<DN>(rop, rpair, rdn, lds, 2, blk(2), vl);
-    wait_vmcnt<2 * LD>();  // chunk 0 in LDS
+    static_assert(NS >= 4 && (NS - 2) * LD < 64, "vmcnt range");
+#pragma unroll
+    for (int k = 0; k < NS - 1; k++) load_block<DN>(rop, rpair, rdn, lds + k * SLOT_BYTES, blk(k), vl);
+    wait_vmcnt<(NS - 2) * LD>();  // chunk 0 in LDS
     wg_barrier();
-    wait_vmcnt<LD>();      // chunk 1
+    wait_vmcnt<(NS - 3) * LD>();  // chunk 1
     wg_barrier();
+    int slot = (NS - 1) * SLOT_BYTES;
     for (int j = 0; j < nck; j++) {
-        // chunk j+3 takes the slot of chunk j, read before the last barrier;
         // the blocks past the strip's end fall in its guard steps
-        load_block<DN>(rop, rpair, rdn, lds, j + 3, blk(j + 3), vl);
-        wait_vmcnt<LD>();  // chunk j+2
+        load_block<DN>(rop, rpair, rdn, lds + slot, blk(j + NS - 1), vl);
+        slot = slot == (NS - 1) * SLOT_BYTES ? 0 : slot + SLOT_BYTES;
+        wait_vmcnt<(NS - 3) * LD>();  // chunk j + 2
         wg_barrier();
     }
+    wg_barrier();
 }
 
-// compute side: one chunk's operators and R/X pair(s) from LDS
-struct Chunk {
-    double2 g[CS][4];
-    double2 r[CS / 2];
-    double2 dn[CS];  // diagonal terms of the lane's row (DN only)
+// ---- the LDS ring between the rows -----------------------------------------
+// Slot e % RS belongs to sweep step e: the 64 lanes' outgoing terms of step
+// e - 1 - GD (what the next group's edge row takes at step e) and, at RIN, the
+// four components the strip's edge row takes from the neighbour strip (nothing
+// reads the terms of those four lanes, which go four places further).  A lane
+// reads the slot of step e + 1 during step e.
+//
+// With RS = 4 CS slots the outgoing courier may run one step behind the chunk
+// barrier, so that the barrier need not wait for the last step's ring write
+// (its own slot is rewritten two chunks later); with RS = 2 CS the barrier
+// waits for it.
+constexpr int RING = 64;                     // doubles per slot
+constexpr int RIN = 4;
+template <int RS>
+constexpr bool late_out() { return RS >= 4 * CS; }
+
+template <int NS, int RS>
+struct SweepLds {
+    char chunk[NS * SLOT_BYTES];
+    double ring[RS * RING];
 };
-template <bool DN = false>
-__device__ inline void read_chunk(Chunk& c, const char* lds, int j, int vl) {
-    const char* base = lds + (j % NSLOT) * SLOT_BYTES;
-    const char* slot = base + vl;
+
+// one row shift of a 64-bit value within the 16-lane rows (row_shr:4 towards
+// higher lanes, row_shl:4 towards lower); the lanes with no source keep `old`
+template <bool UP>
+__device__ inline double row_shift4(double old, double x) {
+    constexpr int ctrl = UP ? 0x114 : 0x104;
+    const int lo = __builtin_amdgcn_update_dpp(__double2loint(old), __double2loint(x), ctrl, 0xF, 0xF, false);
+    const int hi = __builtin_amdgcn_update_dpp(__double2hiint(old), __double2hiint(x), ctrl, 0xF, 0xF, false);
+    return __hiloint2double(hi, lo);
+}
+
+// lane 4r+c receives lane 4r + (c + K) mod 4
+template <int K>
+__device__ inline double quad_rot(double x) {
+    constexpr int ctrl = (K & 3) | (((K + 1) & 3) << 2) | (((K + 2) & 3) << 4) | (((K + 3) & 3) << 6);
+    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(x), ctrl, 0xF, 0xF, true);
+    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(x), ctrl, 0xF, 0xF, true);
+    return __hiloint2double(hi, lo);
+}
+
+// a step's operators (A and B rows of the lane) and, with DN, its diagonal
+// terms
+struct StepOps {
+    double2 g[4], dn;
+};
+template <bool DN>
+__device__ inline void read_ops(StepOps& o, const char* slot, int ts, int vl) {
+    const char* p = slot + vl + ts * 4096;
 #pragma unroll
-    for (int t = 0; t < CS; t++)
+    for (int k = 0; k < 4; k++) o.g[k] = *reinterpret_cast<const double2*>(p + k * 1024);
+    // row r = lane/4: 16 bytes at 16 r (four lanes share it)
+    if constexpr (DN) o.dn = *reinterpret_cast<const double2*>(slot + SLOT_DN + ts * 256 + 4 * (vl / 16 & ~3));
+}
+__device__ inline double2 read_pair(const char* slot, int q, int vl) {
+    return *reinterpret_cast<const double2*>(slot + SLOT_G + q * 1024 + vl);
+}
+
+// wave 0: the sweep over nck chunks.  BWD: steps descend and v = R - (a + b);
+// DN: the operators are (GA, GB) and the diagonal terms are subtracted from
+// their diagonal elements (HA = GA - dsci alpha nuA I).  The next step's
+// right-hand side opens the multiply-add chain of a.
+template <int NS, int RS, bool BWD, bool DN>
+__device__ inline void sweep_compute(SweepLds<NS, RS>& lds, __amdgpu_buffer_rsrc_t rv, int nck, int L) {
+    const int vl = 16 * L;
+    // where the lane's neighbour value comes from in a ring slot: the edge row
+    // of its group takes the last row of the group before it in sweep order,
+    // the strip's own edge row the neighbour strip's columns
+    const int gr = L >> 4, c = L & 3;
+    const int src = BWD ? (gr == 3 ? RIN + c : 16 * (gr + 1) + c) : (gr == 0 ? RIN + c : 16 * (gr - 1) + 12 + c);
+    const double* rd = lds.ring + src;
+    double* wr = lds.ring + ((L & ~3) == RIN ? L + 4 : L);
+    StepOps o[CS];
+    double2 r[CS / 2];
+    auto pair_q = [](int q) { return BWD ? CS / 2 - 1 - q : q; };
+    // R/X of step t of a chunk from its pairs
+    auto rhs = [&](int t) { return ((BWD ? CS - 1 - t : t) & 1) ? r[t >> 1].y : r[t >> 1].x; };
+    wg_barrier();  // chunk 0 and the neighbour's columns of steps 0..CS in LDS
 #pragma unroll
-        for (int p = 0; p < 4; p++) c.g[t][p] = *reinterpret_cast<const double2*>(slot + t * 4096 + p * 1024);
+    for (int t = 0; t < CS; t++) read_ops<DN>(o[t], lds.chunk, BWD ? CS - 1 - t : t, vl);
 #pragma unroll
-    for (int q = 0; q < CS / 2; q++) c.r[q] = *reinterpret_cast<const double2*>(slot + SLOT_G + q * 1024);
-    if constexpr (DN) {
-        // row r = lane/4 of step t: 16 bytes at t*256 + 16 r (four lanes share it)
-        const char* dn = base + SLOT_DN + 4 * (vl / 16 & ~3);
+    for (int q = 0; q < CS / 2; q++) r[q] = read_pair(lds.chunk, pair_q(q), vl);
+    double nb = rd[0];
+    wait_lgkm0();
+    wg_barrier();  // chunk 1 in LDS
+    // a: the step's right-hand side with the term of the row's previous column
+    double a = rhs(0), b = 0.0, keep = 0.0;
+    const char* cur = lds.chunk;  // slot of chunk j
+    for (int j = 0; j < nck; j += RS / CS) {
 #pragma unroll
-        for (int t = 0; t < CS; t++) c.dn[t] = *reinterpret_cast<const double2*>(dn + t * 256);
+        for (int h = 0; h < RS / CS; h++) {
+            const char* next = cur == lds.chunk + (NS - 1) * SLOT_BYTES ? lds.chunk : cur + SLOT_BYTES;
+#pragma unroll
+            for (int t = 0; t < CS; t++) {
+                const int e = h * CS + t;                  // step modulo RS
+                const int ts = BWD ? CS - 1 - t : t;       // step within the stored chunk
+                const double bin = row_shift4<!BWD>(nb, b);
+                // the neighbour value of the next step is read first, then the
+                // operators that the step before has used: LDS returns in
+                // order, so the next step waits for this value alone
+                nb = rd[((e + 1) & (RS - 1)) * RING];
+                ds_order();
+                const double v = BWD ? a - bin : a + bin;
+                const double v1 = quad_rot<1>(v), v2 = quad_rot<2>(v), v3 = quad_rot<3>(v);
+                const double2 a01 = o[t].g[0], a23 = o[t].g[1], b01 = o[t].g[2], b23 = o[t].g[3];
+                const double a0 = DN ? a01.x + o[t].dn.x : a01.x, b0 = DN ? b01.x + o[t].dn.y : b01.x;
+                const double R = rhs((t + 1) & (CS - 1));
+                if (t > 0)
+                    read_ops<DN>(o[t - 1], next, BWD ? CS - t : t - 1, vl);
+                else
+                    read_ops<DN>(o[CS - 1], cur, BWD ? 0 : CS - 1, vl);
+                b = fma(b23.y, v3, fma(b23.x, v2, fma(b01.y, v1, b0 * v)));
+                a = BWD ? fma(-a23.y, v3, fma(-a23.x, v2, fma(-a01.y, v1, fma(-a0, v, R))))
+                        : fma(a23.y, v3, fma(a23.x, v2, fma(a01.y, v1, fma(a0, v, R))));
+                if (!(t & 1)) {
+                    keep = v;
+                    r[t >> 1] = read_pair(next, pair_q(t >> 1), vl);
+                } else {
+                    const int m = BWD ? nck - 1 - (j + h) : j + h;  // stored chunk
+                    st_pair(rv, BWD ? make_double2(v, keep) : make_double2(keep, v), vl,
+                            pair_off(CS * m + (ts & ~1)));
+                }
+                wr[((e + 1 + GD) & (RS - 1)) * RING] = b;
+                ds_order();
+            }
+            cur = next;
+            if (late_out<RS>()) {
+                chunk_barrier();
+            } else {
+                wait_lgkm0();
+                wg_barrier();
+            }
+        }
+    }
+    wait_lgkm0();
+    wg_barrier();  // the last step's outgoing terms
+}
+
+// wave 2: columns of the neighbour strip's hand-off row (view rin) into the
+// ring, those of steps CS j + 1 .. CS j + CS before chunk j is computed.  Step
+// e takes column col0 + e (forward) or col0 - e (backward).  One load covers
+// LK = 32 steps (lane l: components 2 (l & 1) and the next of step l/2).  The
+// next one is issued, from the step then wanted, before the last is looked
+// at: a look costs no more than the rest of its latency (about 0.7 us, since
+// the loads queue behind the loader's), and a look that delivers several
+// chunks lets the strip catch up.  More loads in flight slowed the loader by
+// more than they saved.  Past spin_limit looks without progress it raises
+// SHCFD_E_SPIN and goes on with zeros, so that the sweep still runs to its
+// end.
+constexpr int LK = 32;
+template <int RS, bool BWD>
+__device__ inline void courier_in(double* ring, __amdgpu_buffer_rsrc_t rin, bool present, int col0, int nck, int L,
+                                  long long spin_limit, int* iflag) {
+    if (!present) {
+        for (int j = 0; j < nck + 3; j++) wg_barrier();
+        return;
+    }
+    const int c = 2 * (L & 1), k = L >> 1;
+    auto poll = [&](int e) {  // steps e .. e + LK - 1
+        asm volatile("" ::: "memory");  // a poll is a new load
+        return ld_agent2(rin, 8 * c + col_off(col0 + (BWD ? -1 : 1) * (e + k)), 0);
+    };
+    int e = 0, n = CS + 1, met = 0;  // steps e .. e + n - 1 are wanted; barriers met
+    long long it = 0;
+    bool dead = false;
+    int f1 = 0;
+    double2 x1 = poll(0);
+    while (met < nck + 2) {
+        const double2 x = x1;
+        const int f = f1;
+        f1 = e;
+        x1 = poll(e);
+        const unsigned long long got = __ballot(dead || !(is_sentinel(x.x) || is_sentinel(x.y)));
+        while (met < nck + 2) {
+            const unsigned long long want = (1ULL << (2 * n)) - 1;
+            if (e + n - f > LK || (~(got >> (2 * (e - f))) & want) != 0ULL) break;
+            const int q = k - (e - f);
+            if (q >= 0 && q < n)
+                *reinterpret_cast<double2*>(&ring[((e + q) & (RS - 1)) * RING + RIN + c]) =
+                    make_double2(is_sentinel(x.x) ? 0.0 : x.x, is_sentinel(x.y) ? 0.0 : x.y);
+            wait_lgkm0();
+            wg_barrier();
+            if (met == 0) {  // chunk 1 of the operators
+                wg_barrier();
+                met = 1;
+            }
+            met++;
+            e += n;
+            n = CS;
+            it = -1;
+        }
+        if (!dead && it++ >= spin_limit + 1) {
+            atomicCAS(iflag + IFLAG_ERR, 0, SHCFD_E_SPIN);
+            dead = true;
+        }
+    }
+    wg_barrier();
+}
+
+// wave 3: the strip's outgoing columns (lanes at `edge` of the ring) to its
+// hand-off row after chunk j's barrier (late_out: up to the step before the
+// chunk's last, whose terms follow with the next chunk's).  Step e gives column col0 + e (forward) or col0 - e (backward).
+template <int RS, bool BWD>
+__device__ inline void courier_out(const double* ring, __amdgpu_buffer_rsrc_t rout, bool present, int col0, int edge,
+                                   int nck, int L) {
+    constexpr int DIR = BWD ? -1 : 1;
+    const int c = L & 3, k = L >> 2;
+    wg_barrier();
+    wg_barrier();
+    for (int j = 0; j <= nck; j++) {
+        wg_barrier();  // chunk j is computed (j = nck: nothing is left to compute)
+        const int e = CS * j - (late_out<RS>() ? 1 : 0) + (k & (CS - 1));
+        const double x = ring[((e + 1 + GD) & (RS - 1)) * RING + edge + c];
+        const bool live = present && k < CS && e >= 0 && e < CS * nck;
+        st_agent(rout, x, live ? 8 * c + col_off(col0 + DIR * e) : BUF_DROP, 0);
+        wait_lgkm0();
     }
 }
 
-constexpr int PH = 4;   // hand-off prefetch depth (steps); divides 2*CS
-constexpr int HM = 4;   // extra hand-off lead (columns) awaited before the start
-
-__shared__ __attribute__((aligned(16))) char sweep_lds[NSLOT * SLOT_BYTES];
-
-// one forward step (lane L: component L&3 of row L>>2): step dd, slot step t
-// of chunk c, ring position u (compile-time after unrolling)
-__device__ inline void fwd_step(const Chunk& c, int t, int u, int dd, double& a, double& bo, double& vlo,
-                                double (&hb)[PH],
-                                bool cons, const double* hin, __amdgpu_buffer_rsrc_t rin,
-                                __amdgpu_buffer_rsrc_t rv, __amdgpu_buffer_rsrc_t rout, int vl, int vc, int vo,
-                                long long spin_limit, int* iflag) {
-    const double2 ga01 = c.g[t][0], ga23 = c.g[t][1], gb01 = c.g[t][2], gb23 = c.g[t][3];
-    const double Rc = (t & 1) ? c.r[t >> 1].y : c.r[t >> 1].x;
-    const int i0 = dd + 1;  // column of row 0
-    double x = hb[u % PH];
-    if (__builtin_expect((__builtin_amdgcn_ballot_w64(is_sentinel(x)) & 0xFULL) != 0ULL, 0)) {
-        // the producer fell behind after the start: poll this column only
-        // (a ring refill here would make the compiler copy the ring on the
-        // common path), then drain so the common path inherits no pending
-        // loads
-        handoff_wait(x, hin + 4LL * i0, cons, spin_limit, iflag);
-        wait_all_vmem();
-    }
-    double bin = shift_up4(bo);
-    if (cons) bin = x;
-    const double v = (Rc + a) + bin;
-    // refill the ring slot once x is dead, so the load lands in place
-    hb[u % PH] = ld_agent(rin, vc, col_off(i0 + PH));
-    if (t & 1)
-        st_pair(rv, make_double2(vlo, v), vl, pair_off(dd - 1));
-    else
-        vlo = v;
-    const double v0 = quad_bcast<0>(v), v1 = quad_bcast<1>(v), v2 = quad_bcast<2>(v), v3 = quad_bcast<3>(v);
-    a = fma(ga23.y, v3, fma(ga23.x, v2, fma(ga01.y, v1, ga01.x * v0)));
-    bo = fma(gb23.y, v3, fma(gb23.x, v2, fma(gb01.y, v1, gb01.x * v0)));
-    // row 15 hands column dd-14 to the strip below
-    st_agent(rout, bo, vo, col_off(dd - (QR - 2)));
+// clear the ring: the steps before the first values, and the columns of a
+// strip that has no neighbour, are zero
+template <int RS>
+__device__ inline void clear_ring(double* ring) {
+    for (int k = (int)threadIdx.x; k < RS * RING; k += 256) ring[k] = 0.0;
+    wait_lgkm0();
+    wg_barrier();
 }
 
 // ---------------------------------------------------------------------------
-// forward sweep: one workgroup (compute wave + loader wave) per quad strip
+// forward sweep: one workgroup per quad strip
 // ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(1, 1)))
+template <int NS, int RS>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2)))
 k_fast_fwd(DevCtx d, const QStrip* strips, int nstrips, const double* R_sl, const double* G, double* V_sl,
            double* hand, long long hstride, long long spin_limit, const int2* work, int nwork, double* H) {
     if ((int)blockIdx.x >= nstrips) {
         // workgroups past the strips form the backward operators (HA, HB) of
         // the work items, concurrently with the sweep: 16 steps x 16 rows per
-        // item, two cells per thread.  They wait on nothing, and the strips
-        // (lower workgroup ids) are dispatched before them.
+        // item.  They wait on nothing, and the strips (lower workgroup ids)
+        // are dispatched before them.
         const int nh = (int)gridDim.x - nstrips;
         for (int w = (int)blockIdx.x - nstrips; w < nwork; w += nh) {
             const int2 wk = work[w];
             const QStrip S = strips[wk.x];
             const DevBlock B = d.blk[S.b];
-#pragma unroll 1
-            for (int h = 0; h < 2; h++) {
-                const int t = (int)threadIdx.x + 128 * h;
-                prep_cell_h(d, S, B, wk.y + (t & 15), t >> 4, H);
-            }
+            prep_cell_h(d, S, B, wk.y + ((int)threadIdx.x & 15), (int)threadIdx.x >> 4, H);
         }
         return;
     }
     const int s = blockIdx.x;
-    const int L = threadIdx.x & 63;
+    const int L = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const QStrip S = strips[s];
-    const int ni = d.blk[S.b].ni;
     const int nck = S.nch * (CH / CS);  // chunks, processed in ascending order
     const long long nstep = (long long)(S.nch + 2) * CH;
-    const int vl = 16 * L;
-    if (threadIdx.x >= 64) {
+    __shared__ __attribute__((aligned(16))) SweepLds<NS, RS> lds;
+    clear_ring<RS>(lds.ring);
+    if (wave == 0) {
+        sweep_compute<NS, RS, false, false>(lds, view(V_sl + S.base - 64 * CH, nstep * 64), nck, L);
+    } else if (wave == 1) {
         const __amdgpu_buffer_rsrc_t rg = view(G + (S.base / 64 - CH) * 512, nstep * 512);
         const __amdgpu_buffer_rsrc_t rr = view(R_sl + S.base - 64 * CH, nstep * 64);
-        loader<false>(rg, rr, rr, sweep_lds, nck, vl, [](int j) { return j; });
-        return;
-    }
-    const bool cons = L < 4;  // lanes of row 0: they take the hand-off
-    const __amdgpu_buffer_rsrc_t rv = view(V_sl + S.base - 64 * CH, nstep * 64);
-    // a strip with no neighbour above reads the row of zeros
-    const long long prow = S.prev >= 0 ? S.prev : nstrips;
-    const __amdgpu_buffer_rsrc_t rin = view(hand + prow * hstride, hstride);
-    const __amdgpu_buffer_rsrc_t rout = view(hand + (long long)s * hstride, hstride);
-    const double* hin = hand + prow * hstride + 4 * HOFF + (L & 3);  // for polling
-    const int vc = 8 * (L & 3);
-    const int vo = (S.next >= 0 && L >= 60) ? vc : BUF_DROP;  // row 15 hands off
-    // start once the strip above is PH+HM columns ahead, so that the ring
-    // loads find their columns already written
-    {
-        const int ahead = min(PH + HM, ni);
-        double y = load_agent(hin + 4LL * ahead);
-        handoff_wait(y, hin + 4LL * ahead, cons, spin_limit, d.iflag);
-        wait_all_vmem();
-    }
-    double hb[PH];
-#pragma unroll
-    for (int q = 0; q < PH; q++) hb[q] = ld_agent(rin, vc, col_off(q + 1));
-    // drain before the loop: the wait counts at the loop head then follow the
-    // back edge alone (in-order vmcnt: with these loads still in flight on
-    // entry, every step would also wait for the stores of the last steps)
-    wait_all_vmem();
-    double a = 0.0, bo = 0.0, vlo = 0.0;
-    Chunk A, B;
-    wg_barrier();  // chunk 0 in LDS
-    read_chunk(A, sweep_lds, 0, vl);
-    wait_lgkm0();
-    wg_barrier();  // chunk 1 in LDS
-    for (int j = 0; j < nck; j += 2) {
-        read_chunk(B, sweep_lds, j + 1, vl);
-#pragma unroll
-        for (int t = 0; t < CS; t++)
-            fwd_step(A, t, t, CS * j + t, a, bo, vlo, hb, cons, hin, rin, rv, rout, vl, vc, vo, spin_limit,
-                     d.iflag);
-        wait_lgkm0();
-        wg_barrier();
-        read_chunk(A, sweep_lds, j + 2, vl);
-#pragma unroll
-        for (int t = 0; t < CS; t++)
-            fwd_step(B, t, CS + t, CS * (j + 1) + t, a, bo, vlo, hb, cons, hin, rin, rv, rout, vl, vc, vo,
-                     spin_limit, d.iflag);
-        wait_lgkm0();
-        wg_barrier();
+        sweep_loader<NS, false>(rg, rr, rr, lds.chunk, nck, 16 * L, [](int j) { return j; });
+    } else if (wave == 2) {  // row 0 of step e is at column e + 1
+        const long long prow = S.prev >= 0 ? S.prev : nstrips;
+        courier_in<RS, false>(lds.ring, view(hand + prow * hstride, hstride), S.prev >= 0, 1, nck, L, spin_limit, d.iflag);
+    } else {  // row 15 of step e is at column e - SPAN + 1
+        courier_out<RS, false>(lds.ring, view(hand + (long long)s * hstride, hstride), S.next >= 0, 1 - SPAN, 60, nck, L);
     }
 }
 
@@ -569,107 +706,32 @@ __global__ void __launch_bounds__(256) k_fast_mid(DevCtx d, const QStrip* strips
 // backward sweep: workgroup g handles strip (n-1-g), so the strip it waits
 // for (the one above) has a lower workgroup id
 // ---------------------------------------------------------------------------
-// one backward step: step dd, slot step t of chunk c, ring position u.  DN:
-// the operators are (GA, GB) and the step subtracts the diagonal terms
-// (HA z = GA z - dsci alpha nuA z, the term entering as the first addend)
-template <bool DN>
-__device__ inline void bwd_step(const Chunk& c, int t, int u, int dd, double& a, double& bo, double& zhi,
-                                double (&hb)[PH], bool cons, const double* hin, __amdgpu_buffer_rsrc_t rin,
-                                __amdgpu_buffer_rsrc_t rz, __amdgpu_buffer_rsrc_t rout, int vl, int vc, int vo,
-                                long long spin_limit, int* iflag) {
-    const double2 ha01 = c.g[t][0], ha23 = c.g[t][1], hb01 = c.g[t][2], hb23 = c.g[t][3];
-    const double Xc = (t & 1) ? c.r[t >> 1].y : c.r[t >> 1].x;
-    const int i15 = dd - (QR - 2);  // column of row 15
-    double x = hb[u % PH];
-    if (__builtin_expect((__builtin_amdgcn_ballot_w64(is_sentinel(x)) >> 60) != 0ULL, 0)) {
-        // the producer fell behind: poll this column only
-        handoff_wait(x, hin + 4LL * i15, cons, spin_limit, iflag);
-        wait_all_vmem();
-    }
-    double bin = shift_down4(bo);
-    if (cons) bin = x;
-    const double z = Xc - (a + bin);
-    hb[u % PH] = ld_agent(rin, vc, col_off(i15 - PH));
-    if (t & 1)
-        zhi = z;
-    else
-        st_pair(rz, make_double2(z, zhi), vl, pair_off(dd));
-    const double z0 = quad_bcast<0>(z), z1 = quad_bcast<1>(z), z2 = quad_bcast<2>(z), z3 = quad_bcast<3>(z);
-    if constexpr (DN) {
-        const double pa = c.dn[t].x * z, pb = c.dn[t].y * z;
-        a = fma(ha23.y, z3, fma(ha23.x, z2, fma(ha01.y, z1, fma(ha01.x, z0, pa))));
-        bo = fma(hb23.y, z3, fma(hb23.x, z2, fma(hb01.y, z1, fma(hb01.x, z0, pb))));
-    } else {
-        a = fma(ha23.y, z3, fma(ha23.x, z2, fma(ha01.y, z1, ha01.x * z0)));
-        bo = fma(hb23.y, z3, fma(hb23.x, z2, fma(hb01.y, z1, hb01.x * z0)));
-    }
-    // row 0 hands column dd+1 to the strip above
-    st_agent(rout, bo, vo, col_off(dd + 1));
-}
-
 // DN: H holds (GA, GB) and Dn the diagonal terms (schemes with S = I)
-template <bool DN>
-__global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(1, 1)))
+template <int NS, int RS, bool DN>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2)))
 k_fast_bwd(DevCtx d, const QStrip* strips, int nstrips, const double* X_sl, const double* H, const double* Dn,
            double* Z_sl, double* hand, long long hstride, long long spin_limit) {
     const int s = nstrips - 1 - (int)blockIdx.x;
-    const int L = threadIdx.x & 63;
+    const int L = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const QStrip S = strips[s];
     const int nck = S.nch * (CH / CS);  // chunk j holds block nck-1-j (steps descend)
     const long long nstep = (long long)(S.nch + 2) * CH;
-    const int vl = 16 * L;
-    if (threadIdx.x >= 64) {
+    const int top = nck * CS - 1;  // stored step of sweep step 0
+    __shared__ __attribute__((aligned(16))) SweepLds<NS, RS> lds;
+    clear_ring<RS>(lds.ring);
+    if (wave == 0) {
+        sweep_compute<NS, RS, true, DN>(lds, view(Z_sl + S.base - 64 * CH, nstep * 64), nck, L);
+    } else if (wave == 1) {
         const __amdgpu_buffer_rsrc_t rh = view(H + (S.base / 64 - CH) * 512, nstep * 512);
         const __amdgpu_buffer_rsrc_t rx = view(X_sl + S.base - 64 * CH, nstep * 64);
         const __amdgpu_buffer_rsrc_t rd = DN ? view(Dn + (S.base / 64 - CH) * 32, nstep * 32) : rx;
-        loader<DN>(rh, rx, rd, sweep_lds, nck, vl, [nck](int j) { return nck - 1 - j; });
-        return;
-    }
-    const bool cons = L >= 60;  // lanes of row 15: they take the hand-off
-    const __amdgpu_buffer_rsrc_t rz = view(Z_sl + S.base - 64 * CH, nstep * 64);
-    // a strip with no neighbour below reads the row of zeros
-    const long long nrow = S.next >= 0 ? S.next : nstrips;
-    const __amdgpu_buffer_rsrc_t rin = view(hand + nrow * hstride, hstride);
-    const __amdgpu_buffer_rsrc_t rout = view(hand + (long long)s * hstride, hstride);
-    const double* hin = hand + nrow * hstride + 4 * HOFF + (L & 3);  // for polling
-    const int vc = 8 * (L & 3);
-    const int vo = (S.prev >= 0 && L < 4) ? vc : BUF_DROP;  // row 0 hands off
-    const int top = nck * CS - 1;  // first step of the sweep
-    // start once the strip below is PH+HM columns ahead (columns descend
-    // from ni; the padded columns above ni are zero)
-    {
-        const int ahead = max(d.blk[S.b].ni - PH - HM, 1);
-        double y = load_agent(hin + 4LL * ahead);
-        handoff_wait(y, hin + 4LL * ahead, cons, spin_limit, d.iflag);
-        wait_all_vmem();
-    }
-    // row 15's column at step dd is dd-14
-    double hb[PH];
-#pragma unroll
-    for (int q = 0; q < PH; q++) hb[q] = ld_agent(rin, vc, col_off(top - q - (QR - 2)));
-    wait_all_vmem();  // as in the forward sweep
-    double a = 0.0, bo = 0.0, zhi = 0.0;
-    Chunk A, B;
-    wg_barrier();
-    read_chunk<DN>(A, sweep_lds, 0, vl);
-    wait_lgkm0();
-    wg_barrier();
-    for (int j = 0; j < nck; j += 2) {
-        read_chunk<DN>(B, sweep_lds, j + 1, vl);
-        const int m0 = nck - 1 - j;  // block of chunk j
-#pragma unroll
-        for (int u = 0; u < CS; u++)
-            bwd_step<DN>(A, CS - 1 - u, u, CS * m0 + CS - 1 - u, a, bo, zhi, hb, cons, hin, rin, rz, rout, vl, vc, vo,
-                     spin_limit, d.iflag);
-        wait_lgkm0();
-        wg_barrier();
-        read_chunk<DN>(A, sweep_lds, j + 2, vl);
-#pragma unroll
-        for (int u = 0; u < CS; u++)
-            bwd_step<DN>(B, CS - 1 - u, CS + u, CS * (m0 - 1) + CS - 1 - u, a, bo, zhi, hb, cons, hin, rin, rz, rout, vl,
-                     vc, vo, spin_limit, d.iflag);
-        wait_lgkm0();
-        wg_barrier();
+        sweep_loader<NS, DN>(rh, rx, rd, lds.chunk, nck, 16 * L, [nck](int j) { return nck - 1 - j; });
+    } else if (wave == 2) {  // row 15 of stored step dd is at column dd - SPAN + 1
+        const long long nrow = S.next >= 0 ? S.next : nstrips;
+        courier_in<RS, true>(lds.ring, view(hand + nrow * hstride, hstride), S.next >= 0, top - SPAN + 1, nck, L, spin_limit,
+                         d.iflag);
+    } else {  // row 0 of stored step dd is at column dd + 1
+        courier_out<RS, true>(lds.ring, view(hand + (long long)s * hstride, hstride), S.prev >= 0, top + 1, 0, nck, L);
     }
 }
 
@@ -759,8 +821,8 @@ __device__ inline void put_transposed(double* o, const QStrip& S, int dd, int r,
 #pragma unroll
     for (int k = 0; k < 4; k++)
 #pragma unroll
-        for (int l = 0; l < 4; l++)
-            o[op_index(S, dd, 4 * r + k, pbase + (l >> 1), l & 1)] = present ? -(fs * M[l + 4 * k]) : 0.0;
+        for (int m = 0; m < 4; m++)
+            o[op_index(S, dd, 4 * r + k, pbase + (m >> 1), m & 1)] = present ? -(fs * M[((k + m) & 3) + 4 * k]) : 0.0;
 }
 
 __global__ void __launch_bounds__(256) k_fast_adj_prep(DevCtx d, const QStrip* strips, const int2* work, int nwork,
@@ -903,7 +965,7 @@ int FastPath::init(Ctx& c) {
     for (int s = 0; s < total; s++) {
         const int b = order[s].x, k = order[s].y;
         const DevBlock& B = c.hblk[b];
-        const int nd = B.ni + QR - 1;
+        const int nd = B.ni + SPAN;
         const int nch = (nd + CH - 1) / CH;
         maxcols = std::max(maxcols, nch * CH);
         QStrip S{};
@@ -921,8 +983,9 @@ int FastPath::init(Ctx& c) {
     nstrips = (int)hs.size();
     nwork = (int)hw.size();
     nslots = base;
-    // columns -HOFF .. maxcols + PH + HM of every hand-off row
-    hstride = 4LL * (HOFF + maxcols + PH + HM + 2);
+    // columns -HOFF .. maxcols + 9 of every hand-off row (the views' range
+    // check returns zero beyond, and drops stores)
+    hstride = 4LL * (HOFF + maxcols + 10);
     auto al = [&](void** p, size_t bytes) {
         if (hipMalloc(p, bytes) != hipSuccess) return false;
         return hipMemset(*p, 0, bytes) == hipSuccess;
@@ -948,6 +1011,35 @@ void FastPath::release() {
     *this = FastPath();
 }
 
+// With more strips than CUs a CU holds two strips: 80 KB of LDS each
+static_assert(sizeof(SweepLds<4, 2 * CS>) <= 81920, "two sweep workgroups per CU");
+constexpr int SWEEP_NS = 4, RS_ALONE = 4 * CS, RS_SHARED = 2 * CS;
+
+void FastPath::sweep_fwd(Ctx& c, const DevCtx& d, int nhwg, const double* Rp, const double* Gp, double* Vp, double* hp,
+                         double* Hp) {
+    if (ncu > 0 && nstrips > ncu)
+        hipLaunchKernelGGL((k_fast_fwd<SWEEP_NS, RS_SHARED>), dim3(nstrips + nhwg), dim3(256), 0, c.stream, d, strips,
+                           nstrips, Rp, Gp, Vp, hp, hstride, c.spin_limit, work, nhwg ? nwork : 0, Hp);
+    else
+        hipLaunchKernelGGL((k_fast_fwd<SWEEP_NS, RS_ALONE>), dim3(nstrips + nhwg), dim3(256), 0, c.stream, d, strips,
+                           nstrips, Rp, Gp, Vp, hp, hstride, c.spin_limit, work, nhwg ? nwork : 0, Hp);
+}
+
+void FastPath::sweep_bwd(Ctx& c, const DevCtx& d, bool diag, const double* Xp, const double* Hp, const double* Dp,
+                         double* Zp, double* hp) {
+#define SHCFD_BWD(RS, DN)                                                                                     \
+    hipLaunchKernelGGL((k_fast_bwd<SWEEP_NS, RS, DN>), dim3(nstrips), dim3(256), 0, c.stream, d, strips, nstrips, Xp, Hp, \
+                       Dp, Zp, hp, hstride, c.spin_limit)
+    if (ncu > 0 && nstrips > ncu) {
+        if (diag) SHCFD_BWD(RS_SHARED, true);
+        else SHCFD_BWD(RS_SHARED, false);
+    } else {
+        if (diag) SHCFD_BWD(RS_ALONE, true);
+        else SHCFD_BWD(RS_ALONE, false);
+    }
+#undef SHCFD_BWD
+}
+
 int FastPath::implicit(Ctx& c, int step_internal, int dqdt_inline, int abpm_inline, void (*pb)(Ctx*, int),
                        void (*pe)(Ctx*, int)) {
     DevCtx d = c.dev();
@@ -959,28 +1051,25 @@ int FastPath::implicit(Ctx& c, int step_internal, int dqdt_inline, int abpm_inli
     // the forward ones less diagonal terms: the backward sweep streams (GA,
     // GB) and the 16 bytes of those terms per cell that prep writes, instead
     // of 256 bytes of (HA, HB).  In dual time, when the strips leave CUs idle,
-    // workgroups of the forward launch past the strips form (HA, HB) there,
-    // and the launch asks for 28 KB of dynamic LDS beside the sweep's 57 KB
-    // so that no CU holds two of its workgroups: an operator workgroup next
-    // to a strip would take issue slots and vector-memory bandwidth from the
-    // strip's waves (measured on the 258k-cell forward step: 195 us per
-    // forward sweep with them side by side, 178 us apart, 167 us with (HA,
-    // HB) formed in prep instead, where prep costs 14 us more).  With more
+    // workgroups of the forward launch past the strips form (HA, HB) there.
+    // The sweep's LDS (86 KB) keeps a CU to one of the launch's workgroups: an
+    // operator workgroup next to a strip would take issue slots and
+    // vector-memory bandwidth from the strip's waves.  128 of them spread the
+    // work over the sweep's time; 512 finish sooner and slow the first strips
+    // (258k-cell forward step, whole steps: 1 % slower).  With more
     // strips than CUs (batches of many blocks) no CU is idle: prep forms (HA,
     // HB) from the same cell Jacobians as (GA, GB), and the forward launch
     // holds the strips alone.
     const bool diag = !dual;
     const bool busy = ncu > 0 && nstrips > ncu;
-    const unsigned FWD_PAD_LDS = busy ? 0u : 28672u;
-    const int nhwg = (busy || diag) ? 0 : std::min(nwork, 512);
+    const int nhwg = (busy || diag) ? 0 : std::min(nwork, 128);
     pb(&c, PROF_PREP);
     hipLaunchKernelGGL(k_fast_rhs_prep, dim3(xcd_groups(nwork)), dim3(256), 0, st, d, strips, work, nwork, dqdt_inline,
                        abpm_inline, R, G,
                        (busy && !diag) ? H : nullptr, diag ? Dn : nullptr, hand, nstrips, hstride);
     pe(&c, PROF_PREP);
     pb(&c, PROF_SWEEP_FWD);
-    hipLaunchKernelGGL(k_fast_fwd, dim3(nstrips + nhwg), dim3(128), FWD_PAD_LDS, st, d, strips, nstrips, R, G, V,
-                       hand_f, hstride, c.spin_limit, work, nwork, H);
+    sweep_fwd(c, d, nhwg, R, G, V, hand_f, H);
     pe(&c, PROF_SWEEP_FWD);
     const double* Xin = V;
     if (dual) {
@@ -990,12 +1079,7 @@ int FastPath::implicit(Ctx& c, int step_internal, int dqdt_inline, int abpm_inli
         Xin = X;
     }
     pb(&c, PROF_SWEEP_BWD);
-    if (diag)
-        hipLaunchKernelGGL(k_fast_bwd<true>, dim3(nstrips), dim3(128), 0, st, d, strips, nstrips, Xin, G, Dn, Z,
-                           hand_b, hstride, c.spin_limit);
-    else
-        hipLaunchKernelGGL(k_fast_bwd<false>, dim3(nstrips), dim3(128), 0, st, d, strips, nstrips, Xin, H, nullptr, Z,
-                           hand_b, hstride, c.spin_limit);
+    sweep_bwd(c, d, diag, Xin, diag ? G : H, diag ? Dn : nullptr, Z, hand_b);
     pe(&c, PROF_SWEEP_BWD);
     pb(&c, PROF_UPDATE);
     hipLaunchKernelGGL(k_fast_post, dim3(xcd_groups(nwork)), dim3(256), 0, st, d, strips, work, nwork, Z, part);
@@ -1041,10 +1125,8 @@ int FastPath::adjoint_apply(Ctx& c, const double* r_cell, double* lam) {
     hipStream_t st = c.stream;
     hipLaunchKernelGGL(k_fast_adj_rhs, dim3(xcd_groups(nwork)), dim3(256), 0, st, d, strips, work, nwork, r_cell, aR,
                        ahand, nstrips, hstride);
-    hipLaunchKernelGGL(k_fast_fwd, dim3(nstrips), dim3(128), 0, st, d, strips, nstrips, aR, aG, aV, ahand, hstride,
-                       c.spin_limit, work, 0, nullptr);
-    hipLaunchKernelGGL(k_fast_bwd<false>, dim3(nstrips), dim3(128), 0, st, d, strips, nstrips, aV, aH, nullptr, aZ,
-                       ahand + hstride * (nstrips + 1), hstride, c.spin_limit);
+    sweep_fwd(c, d, 0, aR, aG, aV, ahand, nullptr);
+    sweep_bwd(c, d, false, aV, aH, nullptr, aZ, ahand + hstride * (nstrips + 1));
     hipLaunchKernelGGL(k_fast_adj_post, dim3(xcd_groups(nwork)), dim3(256), 0, st, d, strips, work, nwork, aZ, lam);
     return hipGetLastError() == hipSuccess ? SHCFD_OK : SHCFD_E_HIP;
 }

@@ -26,6 +26,10 @@ struct FastPath {
     // operators, both sweeps and the update
     int implicit(Ctx& c, int step_internal, int dqdt_inline, int abpm_inline, void (*prof_begin)(Ctx*, int),
                  void (*prof_end)(Ctx*, int));
+    void sweep_fwd(Ctx& c, const DevCtx& d, int nhwg, const double* Rp, const double* Gp, double* Vp, double* hp,
+                   double* Hp);
+    void sweep_bwd(Ctx& c, const DevCtx& d, bool diag, const double* Xp, const double* Hp, const double* Dp, double* Zp,
+                   double* hp);
     int adjoint_prep(Ctx& c);                                      // transposed operators at the current state
     int adjoint_apply(Ctx& c, const double* r_cell, double* lam);  // lam += M^-T r
 };
