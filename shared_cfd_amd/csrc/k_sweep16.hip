@@ -327,25 +327,60 @@ k_sweep16_bwd(DevCtx d, const Strip16* strips, int nstrips, double* hand, long l
 //     (Atilde x)_nY   = U X + u e + n_x dp
 //     (Atilde x)_nY+1 = U V + v e + n_y dp
 //     (Atilde x)_nY+2 = U E + H e + U dp
-// with U = n_x u + n_y v, s = sum_k x_k, e = n_x X + n_y V - U s and
+// with U = n_x u + n_y v, s = sum_k x_k, e = n_x (X - u s) + n_y (V - v s) and
 // dp = sum_k DHi_k x_k + (gamma-1) ((u^2+v^2)/2 s - u X - v V + E).
-// A step therefore needs the cell's state (2 nY + 13 numbers) instead of
-// the 2 dq^2 entries of the two matrices: every lane reads one pair (c1, DHi)
-// (c1 = Y_k, u, v or H for its component) and the 13 cell scalars come
-// through LDS, written by the lanes of components 0..7 from their prefetched
-// share.  The sums s and dp are taken in the same order by every lane.  The
-// algebra is exact; the rounding differs from the matrix products
-// (agreement with them to ~1e-13 relative per sweep).
+// Each term is thus a diagonal part and three dot products with x: eA and eB
+// (e with n = dsci alpha n_i / 2 and dscj alpha n_j / 2) and dp.  alpha is
+// folded in as in k_fast.hip: the forward sweep computes
+// v = R + GA v(i-1) + GB v(j-1) with GA = dsci alpha A+, the backward sweep
+// z = v - (HA z(i+1) + HB z(j+1)), and dq = alpha z.  The record of a cell
+// holds the coefficients of the dot products and of the terms per component.
+//
+// Layout and schedule.  Lane 4r + c of compute wave w holds component 4w + c
+// of row r; the groups of four rows run one step apart (row r works on column
+// t - r - floor(r/4) + 1 at step t), so that within a group the hop to the
+// next row is one DPP row shift and between groups the value crosses through
+// an LDS ring.  The records are stored by (strip, step, wave, lane): a step's
+// loads and its store share one address, each is one run of consecutive bytes,
+// and slots of no cell hold zeros (no masks); v and z replace R in place.  A
+// step has one workgroup barrier: before it each quad puts its partial sums of
+// the three dot products into LDS (lane c the c-th, from a transposing
+// reduction), after it lane c adds the waves' and the quad exchanges the
+// totals.  Two more waves move the hand-off: wave C polls the neighbour
+// strip's row, wave C + 1 stores the strip's own, so a compute wave waits for
+// no store and no other strip except at the barrier.
+//
+// Bound by the chain of one step, 240 ns: 17 FP64 operations (about 8 cycles
+// each from one wave), the DPP moves and two LDS round trips, beside 5 loads of
+// 64 x 16 bytes per wave; then by the hand-off, a strip running 18 steps plus
+// about 4 us behind its neighbour.  Measured at nY = 9: 575 us forward and
+// 545 us backward on 1024 x 512 (before 1285 and 986), 109 and 110 us on
+// 223 x 99 (before 200 and 210); forming the records and the right-hand side
+// in one pass, 195 us on 1024 x 512 (before, cell data 104 us and right-hand
+// side 78 us in two), the update 56 us.  Before, dq was read and written in
+// place: 64 lanes in 64 different cache lines per access, with the hand-off
+// polls and stores in the same in-order vmcnt.  Looking at the hand-off more
+// often than when a step needs it costs more than it gains, since a look waits
+// for its load and the barrier for the look: 612 us forward with a look every
+// second step.
 // ---------------------------------------------------------------------------
 
 namespace {
-constexpr int JPD = 11;   // prefetch distance of the cell data, in steps (JPD + 1 = 12 steps per round)
-// a round of JPD + 1 steps must cycle whole rings: the hand-off loads (PH),
-// the scalar slots (3) and the LDS exchange buffers (2)
-static_assert((JPD + 1) % PH == 0 && (JPD + 1) % 6 == 0, "round length");
-constexpr int JSC = 16;   // cell scalars per (step, row): u v g H nxi nyi nxj nyj nuA/2 nuB/2 alpha dsci dscj
-constexpr int JST = 17;   // their row stride in LDS (odd: the 16 rows of a read fall in distinct banks)
-enum { JS_U = 0, JS_V, JS_G, JS_H, JS_NXI, JS_NYI, JS_NXJ, JS_NYJ, JS_HNA, JS_HNB, JS_AL, JS_DSCI, JS_DSCJ };
+constexpr int JU = 8;          // steps per unrolled round; prefetch runs JU - 1 steps ahead
+constexpr int JGD = 1;         // extra steps between the four-row groups
+constexpr int JSPAN = 15 + 3 * JGD;  // steps row 15 runs behind row 0
+constexpr int JRS = 8;         // ring slots
+constexpr int JRIN = 4;        // ring lanes of the neighbour strip's components
+
+// Cell records by (strip, step, wave), in bytes: (c1, cP) and R per lane, the
+// sweeps' diagonal pairs per row, (cA, cB) per row in waves of species alone,
+// per lane in the others, which also hold (pA, pB); c1 = Y_k, u, v or H, cA,
+// cB and cP the dot products' coefficients of the component, pA and pB the
+// factors of dp
+constexpr int JO_R = 1024, JO_LF = 1536, JO_LB = 1792, JO_E = 2048, JO_P = 3072;
+template <int NY>
+constexpr int jrec_step() { return jrec_off(NY, (NY + 6) / 4); }
+static_assert(JO_E + 16 * 16 == JREC_S && JO_P + 16 * 64 == JREC_M && JU - 1 <= JPAD, "cell records");
 
 template <int CTRL>
 __device__ inline double quad_perm(double v) {
@@ -354,93 +389,88 @@ __device__ inline double quad_perm(double v) {
     hi = __builtin_amdgcn_mov_dpp(hi, CTRL, 0xF, 0xF, true);
     return __hiloint2double(hi, lo);
 }
-// (x0 + x1) + (x2 + x3) of the four lanes of each quad, in every lane
-__device__ inline double quad_sum(double x) {
-    const double y = x + quad_perm<1 | (0 << 2) | (3 << 4) | (2 << 6)>(x);   // quad_perm [1,0,3,2]
-    return y + quad_perm<2 | (3 << 2) | (0 << 4) | (1 << 6)>(y);             // quad_perm [2,3,0,1]
+constexpr int QP_X1 = 1 | (0 << 2) | (3 << 4) | (2 << 6), QP_X2 = 2 | (3 << 2) | (0 << 4) | (1 << 6);
+// sums over the four lanes of each quad: of f0 in lane 0, f1 in lane 1, f2 in
+// lanes 2 and 3; odd: lane 1 or 3, up: lane 2 or 3
+__device__ inline double quad_sums(double f0, double f1, double f2, bool odd, bool up) {
+    const double g01 = (odd ? f1 : f0) + quad_perm<QP_X1>(odd ? f0 : f1);
+    const double g2 = f2 + quad_perm<QP_X1>(f2);
+    return (up ? g2 : g01) + quad_perm<QP_X2>(up ? g01 : g2);
 }
 
-// Buffer views: base in scalar registers, a per-lane byte offset fixed for
-// the sweep and a per-step byte offset in a scalar register, so an access
-// costs one instruction; a lane that must not store gives an offset beyond
-// the view (the hardware's range check drops it).
-typedef unsigned int jv_u32x4 __attribute__((ext_vector_type(4)));
+// Buffer views of the hand-off rows: the hardware's range check returns zero
+// for loads beyond a row and drops stores there
 typedef unsigned int jv_u32x2 __attribute__((ext_vector_type(2)));
 constexpr int JV_DROP = 0x7FFFFF00;
 constexpr int JV_AGENT = 16;   // sc1: device-coherent access
 __device__ inline __amdgpu_buffer_rsrc_t jview(const void* base, long long bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, (int)bytes, 0x00020000);
 }
-__device__ inline double jv_d(unsigned lo, unsigned hi) {
-    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+__device__ inline double jv_ld(__amdgpu_buffer_rsrc_t r, int voff) {
+    const jv_u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(r, voff, 0, JV_AGENT);
+    return __longlong_as_double((long long)(((unsigned long long)v.y << 32) | v.x));
 }
-__device__ inline double2 jv_ld2(__amdgpu_buffer_rsrc_t r, int voff, int soff) {
-    const jv_u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0);
-    return make_double2(jv_d(v.x, v.y), jv_d(v.z, v.w));
-}
-template <int AUX = 0>
-__device__ inline double jv_ld(__amdgpu_buffer_rsrc_t r, int voff, int soff) {
-    const jv_u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, AUX);
-    return jv_d(v.x, v.y);
-}
-template <int AUX = 0>
-__device__ inline void jv_st(__amdgpu_buffer_rsrc_t r, double x, int voff, int soff) {
+__device__ inline void jv_st(__amdgpu_buffer_rsrc_t r, double x, int voff) {
     const unsigned long long a = (unsigned long long)__double_as_longlong(x);
     const jv_u32x2 v = {(unsigned)a, (unsigned)(a >> 32)};
-    __builtin_amdgcn_raw_buffer_store_b64(v, r, voff, soff, AUX);
+    __builtin_amdgcn_raw_buffer_store_b64(v, r, voff, 0, JV_AGENT);
 }
+__device__ inline void jbarrier() { asm volatile("s_barrier" ::: "memory"); }
 
-// per-lane inputs of one step of the Jacobian-free sweeps
-struct JStepIn {
-    double2 cp;    // (c1, DHi) of the lane's component
-    double2 sp;    // the lane's share of the next step's cell scalars
-    double r, q;
+template <int NY>
+struct JLds {
+    static constexpr int C = (NY + 6) / 4;
+    double ring[JRS][C * 64];  // slot t % JRS: the terms the edge rows take at step t
+    double f[2][16][3][(C + 1) / 2 * 2];  // the waves' partial sums of each row's dot products
 };
 
-// the lane's outgoing terms dsci A+-(x) and dscj B+-(x) (sgn = +1 forward,
-// -1 backward) from its row's sums s = sum_k x_k and qd = sum_k DHi_k x_k,
-// the momentum and energy components X, V, E, its own component xk and the
-// cell scalars sc (LDS, row stride JST)
-template <int NY, bool FWD>
-__device__ inline void jvp_out(double s, double qd, double X, double V, double E, double xk, const double* sc, int k,
-                               double c1, double& a_out, double& b_out) {
-#pragma clang fp contract(fast)
-    const double u = sc[JS_U], v = sc[JS_V], g = sc[JS_G];
-    const double nxi = sc[JS_NXI], nyi = sc[JS_NYI], nxj = sc[JS_NXJ], nyj = sc[JS_NYJ];
-    const double Ui = (nxi * u) + (nyi * v), Uj = (nxj * u) + (nyj * v);
-    const double ei = ((nxi * X) + (nyi * V)) - (Ui * s);
-    const double ej = ((nxj * X) + (nyj * V)) - (Uj * s);
-    const double dp = qd + g * ((((0.5 * ((u * u) + (v * v))) * s) - ((u * X) + (v * V))) + E);
-    const double cai = k < NY ? 0.0 : (k == NY ? nxi : (k == NY + 1 ? nyi : Ui));
-    const double caj = k < NY ? 0.0 : (k == NY ? nxj : (k == NY + 1 ? nyj : Uj));
-    const double oA = ((Ui * xk) + (c1 * ei)) + (cai * dp);
-    const double oB = ((Uj * xk) + (c1 * ej)) + (caj * dp);
-    if (FWD) {
-        a_out = sc[JS_DSCI] * ((0.5 * oA) + (sc[JS_HNA] * xk));
-        b_out = sc[JS_DSCJ] * ((0.5 * oB) + (sc[JS_HNB] * xk));
-    } else {
-        a_out = sc[JS_DSCI] * ((0.5 * oA) - (sc[JS_HNA] * xk));
-        b_out = sc[JS_DSCJ] * ((0.5 * oB) - (sc[JS_HNB] * xk));
-    }
+// cell of (strip, step t, row r)
+__device__ inline bool jslot_cell(const Strip16& S, const DevBlock& B, int t, int r, int& i, int& j) {
+    i = t - r - JGD * (r >> 2) + 1;
+    j = S.j0 + r;
+    return i >= 1 && i <= B.ni && j <= B.nj;
 }
 }  // namespace
 
-// the cell data of the Jacobian-free sweeps, in their strip-step layout:
-// the pair (c1, DHi) of (global step g, wave w, lane L) at cp[(g C + w) 64 + L]
-// and scalar p of (step g, row r) at sc[(g 16 + r) JSC + p].  Slots of no
-// cell stay zero (the arrays are cleared once at allocation).  Also stores
-// alpha, as set_ABpm does.
+// The right-hand side of the update (k_rhs) and the cell data of the sweeps in
+// one pass: workgroup = 16 steps x 16 rows of one strip, a wave taking 4 rows x
+// 16 steps so that each load of a cell field reads four runs of 16 cells.
+// Also stores alpha, as set_ABpm does, and refills the hand-off rows.
 template <int NY>
-__global__ void __launch_bounds__(256) k_set_jd16(DevCtx d, const Strip16* strips, double2* cp, double* sc) {
+__global__ void __launch_bounds__(256) k_rhs_jd16(DevCtx d, const Strip16* strips, int nstrips, int nsteps16,
+                                                  int dqdt_inline, char* recs, double* hand, long long hstride) {
     using D = Dims<NY>;
-    constexpr int dq = D::dq, C = (dq + 3) / 4;
-    const Strip16 S = strips[blockIdx.x];
-    const int t = (int)blockIdx.y * 16 + (int)(threadIdx.x >> 4), r = (int)(threadIdx.x & 15);
+    constexpr int dq = D::dq, C = (dq + 3) / 4, W0 = NY / 4;
+    {
+        const long long n = 2LL * (nstrips + 1) * hstride;
+        const double sv = __longlong_as_double((long long)SENT16);
+        for (long long e = (long long)blockIdx.x * 256 + threadIdx.x; e < n; e += (long long)gridDim.x * 256) {
+            const int row = (int)((e / hstride) % (nstrips + 1));
+            const long long col = (e % hstride) / dq - HO;
+            const bool live = row < nstrips && col >= 1 && col <= d.blk[strips[row].b].ni;
+            hand[e] = live ? sv : 0.0;
+        }
+    }
+    const int s = (int)blockIdx.x / nsteps16;
+    const Strip16 S = strips[s];
+    const int t = 16 * ((int)blockIdx.x % nsteps16) + (int)(threadIdx.x & 15), r = (int)(threadIdx.x >> 4);
     const DevBlock B = d.blk[S.b];
-    if (t >= B.ni + 15) return;
-    const int i = t - r + 1, j = S.j0 + r;
-    if (i < 1 || i > B.ni || j > B.nj) return;
-    const long long c = cidx(B, i, j), g = S.base + t;
+    int i, j;
+    char* rec = recs + (JPAD + S.base + t) * jrec_step<NY>();
+    if (!jslot_cell(S, B, t, r, i, j)) {
+        if (t < (B.ni + JSPAN + JU - 1) / JU * JU) {  // the sweeps left their v and z here
+#pragma unroll
+            for (int w = 0; w < C; w++) {
+                double2* R = reinterpret_cast<double2*>(rec + jrec_off(NY, w) + JO_R) + 2 * r;
+                R[0] = R[1] = make_double2(0.0, 0.0);
+            }
+        }
+        return;
+    }
+    const long long c = cidx(B, i, j);
+    double bal[dq], x[dq];
+    flux_balance<NY>(d, B, c, bal);
+    rhs_of_cell<NY>(d, c, bal, dqdt_inline != 0, [](int) { return 0.0; }, [](int) { return 0.0; }, []() { return 0.0; }, x);
     // the scalars of cell_jacobian for the non-preconditioned schemes
     // (sch_lusgs.raw.f90:26-38, :131-133; sch_NR.raw.f90:134-136)
     const double rho = FLD(d, SHCFD_F_W, 0, c), u = FLD(d, SHCFD_F_W, IW_U, c), v = FLD(d, SHCFD_F_W, IW_V, c);
@@ -457,291 +487,251 @@ __global__ void __launch_bounds__(256) k_set_jd16(DevCtx d, const Strip16* strip
                              ? 1.0 / ((((3.0 * vol) / (2.0 * dtv)) + (dsci * nuA)) + (dscj * nuB))
                              : 1.0 / (((vol / dtv) + (dsci * nuA)) + (dscj * nuB));
     FLD(d, SHCFD_F_ALPHA, 0, c) = alpha;
+    const double fa = (0.5 * dsci) * alpha, fb = (0.5 * dscj) * alpha;
+    const double g1 = gamm - 1.0, ke = 0.5 * ((u * u) + (v * v));
+    const double2 lf = make_double2(fa * (unA + nuA), fb * (unB + nuB));
+    const double2 lb = make_double2(fa * (unA - nuA), fb * (unB - nuB));
+    const double2 es = make_double2(-(fa * unA), -(fb * unB));
 #pragma unroll
-    for (int w = 0; w < C; w++)
+    for (int w = 0; w < C; w++) {
+        char* o = rec + jrec_off(NY, w);
+        double2* o1 = reinterpret_cast<double2*>(o) + 4 * r;
+        double2* oE = reinterpret_cast<double2*>(o + JO_E) + 4 * r;
+        double2* oP = reinterpret_cast<double2*>(o + JO_P) + 4 * r;
+        double rv[4];
 #pragma unroll
         for (int cc = 0; cc < 4; cc++) {
-            const int k = 4 * w + cc;
-            double c1 = 0.0, dh = 0.0;
-            if (k < NY) {
-                c1 = FLD(d, SHCFD_F_W, 4 + k, c);
-                dh = FLD(d, SHCFD_F_DHI, k, c);
-            } else if (k == NY) {
-                c1 = u;
-            } else if (k == NY + 1) {
-                c1 = v;
-            } else if (k == NY + 2) {
-                c1 = H;
+            const int k = 4 * w + cc, m = k - NY;
+            rv[cc] = k < dq ? x[k < dq ? k : 0] : 0.0;
+            if (k < NY) o1[cc] = make_double2(FLD(d, SHCFD_F_W, 4 + k, c), FLD(d, SHCFD_F_DHI, k, c) + g1 * ke);
+            else o1[cc] = m == 0 ? make_double2(u, -(g1 * u)) : m == 1 ? make_double2(v, -(g1 * v))
+                        : m == 2 ? make_double2(H, g1) : make_double2(0.0, 0.0);
+            if (w >= W0) {
+                oE[cc] = m < 0 ? es : m == 0 ? make_double2(fa * n1a, fb * n1b)
+                       : m == 1 ? make_double2(fa * n2a, fb * n2b) : make_double2(0.0, 0.0);
+                oP[cc] = m == 0 ? make_double2(fa * n1a, fb * n1b) : m == 1 ? make_double2(fa * n2a, fb * n2b)
+                       : m == 2 ? make_double2(fa * unA, fb * unB) : make_double2(0.0, 0.0);
             }
-            cp[(g * C + w) * 64 + 4 * r + cc] = make_double2(c1, dh);
         }
-    double* o = sc + (g * 16 + r) * JSC;
-    o[JS_U] = u;
-    o[JS_V] = v;
-    o[JS_G] = gamm - 1.0;
-    o[JS_H] = H;
-    o[JS_NXI] = n1a;
-    o[JS_NYI] = n2a;
-    o[JS_NXJ] = n1b;
-    o[JS_NYJ] = n2b;
-    o[JS_HNA] = nuA * 0.5;
-    o[JS_HNB] = nuB * 0.5;
-    o[JS_AL] = alpha;
-    o[JS_DSCI] = dsci;
-    o[JS_DSCJ] = dscj;
-}
-
-// One step of a Jacobian-free sweep, per lane: x of its component from the
-// incoming terms and alpha (read one step ahead); then x, the quad partial
-// sums of x_k and DHi_k x_k over the species lanes, and the next step's cell
-// scalars go to LDS; after the barrier the lane reads X, V, E, the partial
-// sums of its row and the scalars, and forms its outgoing terms.  LDS rows
-// have odd strides, so the 16 rows of a wave's read fall in distinct banks.
-
-// forward sweep, Jacobian-free: x = alpha (R + A+(i-1) x(i-1) dsci + B+(j-1) x(j-1) dscj)
-template <int NY>
-__global__ void __launch_bounds__(NY + 3 <= 16 ? 256 : 320) __attribute__((amdgpu_waves_per_eu(1, 1)))
-k_sweep16j_fwd(DevCtx d, const Strip16* strips, int nstrips, double* hand, long long hstride, long long spin_limit,
-               const double2* __restrict__ jcp, const double* __restrict__ jsc) {
-    constexpr int dq = NY + 3, C = (dq + 3) / 4, XST = (4 * C) | 1, PST = 2 * C + 1;
-    constexpr int CP_STEP = C * 64 * 16, SC_STEP = 16 * JSC * 8;
-    __shared__ double xs[2][16][XST];
-    __shared__ double pq[2][16][PST];
-    __shared__ double scs[3][16][JST];
-    const int s = blockIdx.x;
-    const int w = (int)(threadIdx.x >> 6), L = (int)(threadIdx.x & 63), r = L >> 2, k = 4 * w + (L & 3);
-    const Strip16 S = strips[s];
-    const DevBlock B = d.blk[S.b];
-    const int ni = B.ni, nj = B.nj, j = S.j0 + r;
-    const bool rowok = j <= nj, kok = k < dq;
-    const bool has_next = S.next >= 0;
-    const bool mine = r == 0 && kok;
-    const int nsteps = ni + 15;
-    const int sp_slot = 4 * w + (L & 3);   // the scalar pair this lane carries (< 8 only)
-    const bool carrier = sp_slot < 8;
-    const int kk = kok ? k : 0;
-    const long long prow = S.prev >= 0 ? S.prev : nstrips;
-    const double* hpoll = hand + prow * hstride + (long long)HO * dq + kk;
-    const __amdgpu_buffer_rsrc_t vin = jview(hand + prow * hstride, hstride * 8);
-    const __amdgpu_buffer_rsrc_t vout = jview(hand + (long long)s * hstride, hstride * 8);
-    const int h_lane = (HO * dq + kk) * 8;                                     // column c at + c dq 8
-    const int h_store = (has_next && r == 15 && kok) ? h_lane - 14 * dq * 8 : JV_DROP;  // column t - 14
-    const __amdgpu_buffer_rsrc_t vcp = jview(jcp + S.base * C * 64, (long long)nsteps * CP_STEP);
-    const int cp_lane = (w * 64 + L) * 16;
-    const __amdgpu_buffer_rsrc_t vsc = jview(jsc + S.base * 16 * JSC, (long long)nsteps * SC_STEP);
-    const int sc_lane = (r * JSC + 2 * (carrier ? sp_slot : 0)) * 8;
-    // one view of all dq components (uniform across the wave: a per-lane base
-    // would make every access a loop over the lanes' distinct bases); the
-    // lane's component and cell in the lane offset
-    const __amdgpu_buffer_rsrc_t vdq = jview(d.f[SHCFD_F_DQ], (long long)dq * d.NC * 8);
-    const int dq_lane = (int)((kk * d.NC + cidx(B, 0, rowok ? j : nj) + 1 - r) * 8);  // the cell of step t at + 8 t
-    auto load = [&](int t, JStepIn& in) {
-        const int tc = t < nsteps ? t : nsteps - 1;  // past the end: re-read the last step
-        const int tn = t + 1 < nsteps ? t + 1 : nsteps - 1;
-        in.cp = jv_ld2(vcp, cp_lane, tc * CP_STEP);
-        in.sp = jv_ld2(vsc, sc_lane, tn * SC_STEP);
-        in.r = jv_ld(vdq, dq_lane, tc * 8);
-    };
-    {
-        const double2 v0 = jv_ld2(vsc, sc_lane, 0);
-        if (carrier) {
-            scs[0][r][2 * sp_slot] = v0.x;
-            scs[0][r][2 * sp_slot + 1] = v0.y;
-        }
-    }
-    JStepIn buf[JPD + 1];
-    double hr[PH];
-#pragma unroll
-    for (int p = 0; p < PH; p++) hr[p] = jv_ld<JV_AGENT>(vin, h_lane, (p + 1) * dq * 8);  // columns 1..PH
-#pragma unroll
-    for (int p = 0; p < JPD; p++) load(p, buf[p]);
-    lds_barrier();
-    double al = scs[0][r][JS_AL];
-    double a_in = 0.0, bo = 0.0;
-    bool dead = false;
-    const int tend = ((nsteps + JPD) / (JPD + 1)) * (JPD + 1);  // whole rounds; the extra steps are idle
-    for (int t0 = 0; t0 < tend; t0 += JPD + 1) {
-#pragma unroll
-        for (int u = 0; u <= JPD; u++) {
-            const int t = t0 + u;
-            double hv = hr[u % PH];
-            hr[u % PH] = jv_ld<JV_AGENT>(vin, h_lane, (t + 1 + PH) * dq * 8);
-            load(t + JPD, buf[(u + JPD) % (JPD + 1)]);
-            const JStepIn& in = buf[u];
-            const int i = t - r + 1;
-            const bool act = rowok && i >= 1 && i <= ni;
-            double b_in = shift_up4(bo);
-            if (__builtin_expect(__ballot(mine && is_sent16(hv)) != 0ULL, 0))
-                hv = poll16(hpoll + (long long)(t + 1) * dq, hv, mine, spin_limit, d.iflag, dead);
-            if (r == 0) b_in = kok ? hv : 0.0;
-            const double xc = al * (in.r + (a_in + b_in));
-            const double x = (act && kok) ? xc : 0.0;
-            jv_st(vdq, x, (act && kok) ? dq_lane : JV_DROP, t * 8);
-            xs[u & 1][r][k] = x;
-            const double ps = quad_sum(k < NY ? x : 0.0);
-            const double pd = quad_sum(in.cp.y * x);
-            if ((L & 3) == 0) {
-                pq[u & 1][r][2 * w] = ps;
-                pq[u & 1][r][2 * w + 1] = pd;
-            }
-            if (carrier) {
-                scs[(u + 1) % 3][r][2 * sp_slot] = in.sp.x;
-                scs[(u + 1) % 3][r][2 * sp_slot + 1] = in.sp.y;
-            }
-            lds_barrier();
-            const double* sct = scs[u % 3][r];
-            const double* xr = xs[u & 1][r];
-            const double* pr = pq[u & 1][r];
-            double sx = pr[0], qd = pr[1];
-#pragma unroll
-            for (int q = 1; q < C; q++) {
-                sx = sx + pr[2 * q];
-                qd = qd + pr[2 * q + 1];
-            }
-            double ao, bn;
-            jvp_out<NY, true>(sx, qd, xr[NY], xr[NY + 1], xr[NY + 2], x, sct, kk, in.cp.x, ao, bn);
-            al = scs[(u + 1) % 3][r][JS_AL];
-            a_in = act ? ao : a_in;
-            bo = act ? bn : 0.0;
-            jv_st<JV_AGENT>(vout, bo, act ? h_store : JV_DROP, t * dq * 8);
-        }
+        double2* oR = reinterpret_cast<double2*>(o + JO_R) + 2 * r;
+        oR[0] = make_double2(rv[0], rv[1]);
+        oR[1] = make_double2(rv[2], rv[3]);
+        reinterpret_cast<double2*>(o + JO_LF)[r] = lf;
+        reinterpret_cast<double2*>(o + JO_LB)[r] = lb;
+        if (w < W0) reinterpret_cast<double2*>(o + JO_E)[r] = es;
     }
 }
 
-// backward sweep, Jacobian-free: x = x* - alpha (A-(i+1) x(i+1) dsci + B-(j+1) x(j+1) dscj),
-// and the (res, omega) partials (NR); LU-SGS's q += x is k_add_dq's pass
-// after the sweep (the scattered q accesses of each step, 16 rows x 4
-// components of 8 bytes, cost more than the pass)
-template <int NY>
-__global__ void __launch_bounds__(NY + 3 <= 16 ? 256 : 320) __attribute__((amdgpu_waves_per_eu(1, 1)))
-k_sweep16j_bwd(DevCtx d, const Strip16* strips, int nstrips, double* hand, long long hstride, double* part,
-               long long spin_limit, const double2* __restrict__ jcp, const double* __restrict__ jsc) {
-    constexpr int dq = NY + 3, C = (dq + 3) / 4, XST = (4 * C) | 1, PST = 2 * C + 1;
-    constexpr int CP_STEP = C * 64 * 16, SC_STEP = 16 * JSC * 8;
-    __shared__ double xs[2][16][XST];
-    __shared__ double pq[2][16][PST];
-    __shared__ double scs[3][16][JST];
-    __shared__ double red[2][4];
-    const int s = nstrips - 1 - (int)blockIdx.x;
-    const int w = (int)(threadIdx.x >> 6), L = (int)(threadIdx.x & 63), r = L >> 2, k = 4 * w + (L & 3);
+// the sweep's compute wave w, rec its record of the strip's step 0; BWD: stored
+// steps descend
+template <int NY, bool BWD, bool PURE>
+__device__ inline void jsweep_compute(JLds<NY>& lds, char* rec, int nt, int w, int L) {
+    constexpr int C = (NY + 6) / 4;
+    constexpr long long STEP = BWD ? -jrec_step<NY>() : jrec_step<NY>();
+    const int r = L >> 2, c = L & 3, gr = L >> 4;
+    const bool odd = (c & 1) != 0, up = c >= 2;
+    const int src = 64 * w + (BWD ? (gr == 3 ? JRIN + c : 16 * (gr + 1) + c)
+                                  : (gr == 0 ? JRIN + c : 16 * (gr - 1) + 12 + c));
+    const int dst = 64 * w + ((L & ~3) == JRIN ? L + 4 : L);
+    const int fc = min(c, 2);
+    const unsigned o16 = 16u * L, o8 = 8u * L + JO_R, ol = 16u * r + (BWD ? JO_LB : JO_LF),
+                   oe = (PURE ? 16u * r : 16u * L) + JO_E;
+    if (BWD) rec += (long long)(nt - 1) * jrec_step<NY>();
+    auto ld16 = [](const char* u, unsigned o) { return *reinterpret_cast<const double2*>(u + o); };
+    // a step's inputs, JU - 1 steps ahead
+    double2 b1[JU], bE[JU], bP[JU], bL[JU];
+    double bR[JU];
+    const char* in = rec;
+#define JLOAD(Q)                                                 \
+    {                                                            \
+        b1[Q] = ld16(in, o16);                                   \
+        bE[Q] = ld16(in, oe);                                    \
+        if constexpr (!PURE) bP[Q] = ld16(in + JO_P, o16);       \
+        bL[Q] = ld16(in, ol);                                    \
+        bR[Q] = *reinterpret_cast<const double*>(in + o8);       \
+        in += STEP;                                              \
+    }
+#pragma unroll
+    for (int q = 0; q < JU - 1; q++) JLOAD(q)
+    wait_vmem();  // so that the waits in the loop follow its own accesses alone
+    jbarrier();  // ring cleared, the neighbour's column of step 0 there
+    double nb = lds.ring[0][src], a = bR[0], b = 0.0;
+    for (int t0 = 0; t0 < nt; t0 += JU) {
+#pragma unroll
+        for (int q = 0; q < JU; q++) {
+            JLOAD((q + JU - 1) % JU)
+            const double bin = row_shift4<!BWD>(nb, b);
+            const double v = BWD ? a - bin : a + bin;
+            const double f = quad_sums(bE[q].x * v, bE[q].y * v, b1[q].y * v, odd, up);
+            if (c < 3) lds.f[q & 1][r][c][w] = f;
+            *reinterpret_cast<double*>(rec + o8) = v;
+            rec += STEP;
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            double tot = lds.f[q & 1][r][fc][0];
+#pragma unroll
+            for (int m = 1; m < C; m++) tot = tot + lds.f[q & 1][r][fc][m];
+            nb = lds.ring[(q + 1) & (JRS - 1)][src];
+            const double eB = quad_perm<0x55>(tot), eA = quad_perm<0x00>(tot);
+            const double rn = bR[(q + 1) % JU];
+            b = fma(b1[q].x, eB, bL[q].y * v);
+            a = BWD ? fma(-b1[q].x, eA, fma(-bL[q].x, v, rn)) : fma(b1[q].x, eA, fma(bL[q].x, v, rn));
+            if constexpr (!PURE) {
+                const double dp = quad_perm<0xAA>(tot);
+                b = fma(bP[q].y, dp, b);
+                a = fma(BWD ? -bP[q].x : bP[q].x, dp, a);
+            }
+            lds.ring[(q + 1 + JGD) & (JRS - 1)][dst] = b;
+        }
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+#undef JLOAD
+}
+
+// forward and backward sweeps: one workgroup of C compute waves and two
+// hand-off waves per strip.  Backward, workgroup g handles strip nstrips-1-g,
+// so the strip it waits on (the one above) has a lower workgroup id.
+template <int NY, bool BWD>
+__global__ void __launch_bounds__(64 * ((NY + 6) / 4 + 2)) __attribute__((amdgpu_waves_per_eu(1, 2)))
+k_sweep16j(DevCtx d, const Strip16* strips, int nstrips, double* hand, long long hstride, long long spin_limit,
+           char* recs) {
+    constexpr int dq = NY + 3, C = (dq + 3) / 4;
+    __shared__ __attribute__((aligned(16))) JLds<NY> lds;
+    const int s = BWD ? nstrips - 1 - (int)blockIdx.x : (int)blockIdx.x;
+    const int L = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const Strip16 S = strips[s];
+    const int nt = (d.blk[S.b].ni + JSPAN + JU - 1) / JU * JU;  // steps, whole rounds
+    for (int e = (int)threadIdx.x; e < JRS * C * 64; e += 64 * (C + 2)) lds.ring[e / (C * 64)][e % (C * 64)] = 0.0;
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    jbarrier();
+    if (wave < C) {
+        char* rec = recs + (JPAD + S.base) * jrec_step<NY>() + jrec_off(NY, wave);
+        if (wave < NY / 4) jsweep_compute<NY, BWD, true>(lds, rec, nt, wave, L);
+        else jsweep_compute<NY, BWD, false>(lds, rec, nt, wave, L);
+    } else if (wave == C) {
+        // the neighbour strip's columns: step e takes column col0 + e (forward)
+        // or col0 - e (backward), in the ring before the barrier of step e - 1.
+        // Two loads cover 2 NQ steps; the next pair is issued, from the step
+        // then wanted, before the last is looked at
+        constexpr int NQ = 64 / dq;
+        const int from = BWD ? S.next : S.prev;
+        if (from < 0) {
+            for (int t = 0; t < nt + 2; t++) jbarrier();
+            return;
+        }
+        const __amdgpu_buffer_rsrc_t rin = jview(hand + (long long)from * hstride, hstride * 8);
+        const int col0 = BWD ? nt - JSPAN : 1;
+        const int q0 = L / dq, k = L % dq;
+        const bool used = q0 < NQ;
+        auto poll = [&](int e, double& x0, double& x1) {
+            asm volatile("" ::: "memory");  // a poll is a new load
+            const int c0 = col0 + (BWD ? -(e + q0) : e + q0), c1 = c0 + (BWD ? -NQ : NQ);
+            x0 = jv_ld(rin, ((HO + c0) * dq + k) * 8);
+            x1 = jv_ld(rin, ((HO + c1) * dq + k) * 8);
+        };
+        int have = 0, f1 = 0;  // steps below `have` are in the ring
+        double x0, x1;
+        poll(0, x0, x1);
+        long long it = 0;
+        bool dead = false;
+        // looks at the loads in flight; steps up to `last` may enter the ring
+        auto look = [&](int last) {
+            const double v0 = x0, v1 = x1;
+            const int f = f1;
+            f1 = have;
+            poll(have, x0, x1);
+            const unsigned long long m0 = __ballot(dead || !used || !is_sent16(v0));
+            const unsigned long long m1 = __ballot(dead || !used || !is_sent16(v1));
+            int ready = m0 == ~0ULL ? NQ : __builtin_ctzll(~m0) / dq;
+            if (ready == NQ) ready += m1 == ~0ULL ? NQ : __builtin_ctzll(~m1) / dq;
+            const int upto = min(f + ready - 1, last);
+            const int e0 = f + q0, e1 = e0 + NQ;
+            const int lane = 64 * (k >> 2) + JRIN + (k & 3);
+            if (used && e0 >= have && e0 <= upto) lds.ring[e0 & (JRS - 1)][lane] = is_sent16(v0) ? 0.0 : v0;
+            if (used && e1 >= have && e1 <= upto) lds.ring[e1 & (JRS - 1)][lane] = is_sent16(v1) ? 0.0 : v1;
+            if (upto >= have) {
+                have = upto + 1;
+                it = 0;
+            } else if (!dead && it++ >= spin_limit + 1) {
+                atomicCAS(d.iflag + IFLAG_ERR, 0, SHCFD_E_SPIN);
+                dead = true;  // no further waits in this sweep: it runs to its end with zeros
+            }
+        };
+        while (have < 1) look(0);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        jbarrier();
+        for (int t = 0; t < nt; t++) {
+            while (have < t + 2) look(t + JRS - 1);
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            jbarrier();
+        }
+        jbarrier();
+    } else {
+        // the strip's own columns: the terms of step t are in the ring after
+        // the barrier of step t + 1.  Step e gives column col0 + e (forward)
+        // or col0 - e (backward)
+        const bool present = (BWD ? S.prev : S.next) >= 0 && L < dq;
+        const __amdgpu_buffer_rsrc_t rout = jview(hand + (long long)s * hstride, hstride * 8);
+        const int col0 = BWD ? nt : 1 - JSPAN;
+        const int k = L < dq ? L : 0, lane = 64 * (k >> 2) + (BWD ? 0 : 60) + (k & 3);
+        jbarrier();
+        for (int t = 0; t <= nt; t++) {
+            jbarrier();
+            if (t == 0) continue;
+            const double x = lds.ring[(t + JGD) & (JRS - 1)][lane];
+            const int col = col0 + (BWD ? -(t - 1) : t - 1);
+            jv_st(rout, x, present ? ((HO + col) * dq + k) * 8 : JV_DROP);
+        }
+    }
+}
+
+// after the sweeps: dq = alpha z into the natural field; LU-SGS: q += dq over
+// the active blocks; NR: (res, omega) partials per workgroup
+template <int NY>
+__global__ void __launch_bounds__(256) k_post16j(DevCtx d, const Strip16* strips, int nsteps16, const char* recs,
+                                                 double* part) {
+    constexpr int dq = NY + 3, C = (dq + 3) / 4;
+    __shared__ double shr[4], sho[4];
+    const int s = (int)blockIdx.x / nsteps16;
+    const Strip16 S = strips[s];
+    const int t = 16 * ((int)blockIdx.x % nsteps16) + (int)(threadIdx.x & 15), r = (int)(threadIdx.x >> 4);
     const DevBlock B = d.blk[S.b];
-    const int ni = B.ni, nj = B.nj, j = S.j0 + r;
-    const bool rowok = j <= nj, kok = k < dq;
-    const bool has_prev = S.prev >= 0;
-    const bool mine = r == 15 && kok;
     const bool inner = inner_loop_scheme(d.p.scheme);
-    const double dqmax = d.p.dqmax;
-    const int nsteps = ni + 15;
-    const int sp_slot = 4 * w + (L & 3);
-    const bool carrier = sp_slot < 8;
-    const int kk = kok ? k : 0;
-    const long long nrow = S.next >= 0 ? S.next : nstrips;
-    const double* hpoll = hand + nrow * hstride + (long long)HO * dq + kk;
-    const __amdgpu_buffer_rsrc_t vin = jview(hand + nrow * hstride, hstride * 8);
-    const __amdgpu_buffer_rsrc_t vout = jview(hand + (long long)s * hstride, hstride * 8);
-    const int h_lane = (HO * dq + kk) * 8;
-    const int h_store = (has_prev && r == 0 && kok) ? h_lane : JV_DROP;   // column ni + 15 - t
-    // backward step t of row r visits the cell of forward step ni + 14 - t
-    const __amdgpu_buffer_rsrc_t vcp = jview(jcp + S.base * C * 64, (long long)nsteps * CP_STEP);
-    const int cp_lane = (w * 64 + L) * 16;
-    const __amdgpu_buffer_rsrc_t vsc = jview(jsc + S.base * 16 * JSC, (long long)nsteps * SC_STEP);
-    const int sc_lane = (r * JSC + 2 * (carrier ? sp_slot : 0)) * 8;
-    // views of all dq and q components, as in the forward sweep (q read for
-    // the omega limit of the inner-loop schemes only)
-    const __amdgpu_buffer_rsrc_t vdq = jview(d.f[SHCFD_F_DQ], (long long)dq * d.NC * 8);
-    const __amdgpu_buffer_rsrc_t vq = jview(d.f[SHCFD_F_Q], (long long)dq * d.NC * 8);
-    const int c_lane = (int)((kk * d.NC + cidx(B, 0, rowok ? j : nj) + 1 - r) * 8);  // the cell of step t at + 8 (ni + 14 - t)
-    auto load = [&](int t, JStepIn& in) {
-        const int tc = t < nsteps ? t : nsteps - 1;
-        const int tn = t + 1 < nsteps ? t + 1 : nsteps - 1;
-        in.cp = jv_ld2(vcp, cp_lane, (ni + 14 - tc) * CP_STEP);
-        in.sp = jv_ld2(vsc, sc_lane, (ni + 14 - tn) * SC_STEP);
-        in.r = jv_ld(vdq, c_lane, (ni + 14 - tc) * 8);
-        in.q = jv_ld(vq, inner ? c_lane : JV_DROP, (ni + 14 - tc) * 8);  // omega's only
-    };
-    {
-        const double2 v0 = jv_ld2(vsc, sc_lane, (ni + 14) * SC_STEP);
-        if (carrier) {
-            scs[0][r][2 * sp_slot] = v0.x;
-            scs[0][r][2 * sp_slot + 1] = v0.y;
+    double res = 0.0, om = 1e300;
+    int i, j;
+    if (jslot_cell(S, B, t, r, i, j)) {
+        const long long c = cidx(B, i, j);
+        const char* rec = recs + (JPAD + S.base + t) * jrec_step<NY>();
+        const double al = FLD(d, SHCFD_F_ALPHA, 0, c);
+#pragma unroll
+        for (int w = 0; w < C; w++) {
+            const double2* z = reinterpret_cast<const double2*>(rec + jrec_off(NY, w) + JO_R) + 2 * r;
+            const double2 z0 = z[0], z1 = z[1];
+            const double x[4] = {al * z0.x, al * z0.y, al * z1.x, al * z1.y};
+#pragma unroll
+            for (int cc = 0; cc < 4; cc++) {
+                const int k = 4 * w + cc;
+                if (k >= dq) continue;
+                FLD(d, SHCFD_F_DQ, k, c) = x[cc];
+                if (inner) {
+                    if (k == NY + 2) res = x[cc] * x[cc];
+                    if (k < NY && x[cc] < 0.0) om = dmin(om, (-FLD(d, SHCFD_F_Q, k, c) / x[cc]) * d.p.dqmax);
+                } else if (B.active) {
+                    FLD(d, SHCFD_F_Q, k, c) = FLD(d, SHCFD_F_Q, k, c) + x[cc];
+                }
+            }
         }
     }
-    JStepIn buf[JPD + 1];
-    double hr[PH];
-#pragma unroll
-    for (int p = 0; p < PH; p++) hr[p] = jv_ld<JV_AGENT>(vin, h_lane, (ni - p) * dq * 8);  // columns ni..ni-PH+1
-#pragma unroll
-    for (int p = 0; p < JPD; p++) load(p, buf[p]);
-    lds_barrier();
-    double al = scs[0][r][JS_AL];
-    double a_in = 0.0, bo = 0.0, res = 0.0, omega = 1e300;
-    bool dead = false;
-    const int tend = ((nsteps + JPD) / (JPD + 1)) * (JPD + 1);
-    for (int t0 = 0; t0 < tend; t0 += JPD + 1) {
-#pragma unroll
-        for (int u = 0; u <= JPD; u++) {
-            const int t = t0 + u;
-            double hv = hr[u % PH];
-            hr[u % PH] = jv_ld<JV_AGENT>(vin, h_lane, (ni - t - PH) * dq * 8);
-            load(t + JPD, buf[(u + JPD) % (JPD + 1)]);
-            const JStepIn& in = buf[u];
-            const int i = ni - t + 15 - r;
-            const bool act = rowok && i >= 1 && i <= ni;
-            double b_in = shift_down4(bo);
-            if (__builtin_expect(__ballot(mine && is_sent16(hv)) != 0ULL, 0))
-                hv = poll16(hpoll + (long long)(ni - t) * dq, hv, mine, spin_limit, d.iflag, dead);
-            if (r == 15) b_in = kok ? hv : 0.0;
-            const double xc = in.r - al * (a_in + b_in);
-            const bool live = act && kok;
-            const double x = live ? xc : 0.0;
-            if (inner && live) {
-                if (k == NY + 2) res = res + x * x;
-                if (k < NY && x < 0.0) omega = dmin(omega, (-in.q / x) * dqmax);
-            }
-            jv_st(vdq, x, live ? c_lane : JV_DROP, (ni + 14 - t) * 8);
-            xs[u & 1][r][k] = x;
-            const double ps = quad_sum(k < NY ? x : 0.0);
-            const double pd = quad_sum(in.cp.y * x);
-            if ((L & 3) == 0) {
-                pq[u & 1][r][2 * w] = ps;
-                pq[u & 1][r][2 * w + 1] = pd;
-            }
-            if (carrier) {
-                scs[(u + 1) % 3][r][2 * sp_slot] = in.sp.x;
-                scs[(u + 1) % 3][r][2 * sp_slot + 1] = in.sp.y;
-            }
-            lds_barrier();
-            const double* sct = scs[u % 3][r];
-            const double* xr = xs[u & 1][r];
-            const double* pr = pq[u & 1][r];
-            double sx = pr[0], qd = pr[1];
-#pragma unroll
-            for (int q = 1; q < C; q++) {
-                sx = sx + pr[2 * q];
-                qd = qd + pr[2 * q + 1];
-            }
-            double ao, bn;
-            jvp_out<NY, false>(sx, qd, xr[NY], xr[NY + 1], xr[NY + 2], x, sct, kk, in.cp.x, ao, bn);
-            al = scs[(u + 1) % 3][r][JS_AL];
-            a_in = act ? ao : a_in;
-            bo = act ? bn : 0.0;
-            jv_st<JV_AGENT>(vout, bo, act ? h_store : JV_DROP, (ni + 15 - t) * dq * 8);
-        }
+    if (!inner) return;
+    for (int off = 32; off >= 1; off >>= 1) {
+        res = res + __shfl_xor(res, off);
+        om = dmin(om, __shfl_xor(om, off));
     }
-    if (inner) {
-        for (int off = 32; off >= 1; off >>= 1) {
-            res = res + __shfl_xor(res, off);
-            omega = dmin(omega, __shfl_xor(omega, off));
-        }
-        if (L == 0) { red[0][w] = res; red[1][w] = omega; }
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            double R = red[0][0], O = red[1][0];
-            for (int q = 1; q < C; q++) { R = R + red[0][q]; O = dmin(O, red[1][q]); }
-            part[2 * s] = R;
-            part[2 * s + 1] = O;
-        }
+    const int w = threadIdx.x >> 6;
+    if ((threadIdx.x & 63) == 0) { shr[w] = res; sho[w] = om; }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        part[2 * blockIdx.x] = (shr[0] + shr[1]) + (shr[2] + shr[3]);
+        part[2 * blockIdx.x + 1] = dmin(dmin(sho[0], sho[1]), dmin(sho[2], sho[3]));
     }
 }
 
@@ -750,11 +740,12 @@ k_sweep16j_bwd(DevCtx d, const Strip16* strips, int nstrips, double* hand, long 
                                                const double*, long long);                                     \
     template __global__ void k_sweep16_bwd<NY>(DevCtx, const Strip16*, int, double*, long long, double*,        \
                                                long long, const double*, long long);                          \
-    template __global__ void k_set_jd16<NY>(DevCtx, const Strip16*, double2*, double*);                         \
-    template __global__ void k_sweep16j_fwd<NY>(DevCtx, const Strip16*, int, double*, long long, long long,     \
-                                                const double2*, const double*);                               \
-    template __global__ void k_sweep16j_bwd<NY>(DevCtx, const Strip16*, int, double*, long long, double*,       \
-                                                long long, const double2*, const double*);
+    template __global__ void k_rhs_jd16<NY>(DevCtx, const Strip16*, int, int, int, char*, double*, long long);  \
+    template __global__ void k_sweep16j<NY, false>(DevCtx, const Strip16*, int, double*, long long, long long,  \
+                                                   char*);                                                    \
+    template __global__ void k_sweep16j<NY, true>(DevCtx, const Strip16*, int, double*, long long, long long,   \
+                                                  char*);                                                     \
+    template __global__ void k_post16j<NY>(DevCtx, const Strip16*, int, const char*, double*);
 SHCFD_FOR_EACH_NY(INST)
 #undef INST
 

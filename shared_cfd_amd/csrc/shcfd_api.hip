@@ -280,7 +280,7 @@ int shcfd_destroy(shcfd_ctx* ctx) {
     void* ptrs[] = {ctx->dblk, ctx->dtiles, ctx->dstrips, ctx->dprog, ctx->dbnd, ctx->dpart, ctx->scal,
                     ctx->iflag, ctx->dcut, ctx->dbc, ctx->dpool, ctx->dmech, ctx->dskew, ctx->dsbase,
                     ctx->djac16, ctx->dstrips16, ctx->dbnd16, ctx->dnasa9, ctx->dhist, ctx->ddefer,
-                    ctx->djcp16, ctx->djsc16};
+                    ctx->djrec16, ctx->djpart16};
     for (void* p : ptrs) if (p) hipFree(p);
     if (ctx->stream) hipStreamDestroy(ctx->stream);
     delete ctx;
@@ -837,29 +837,23 @@ static bool skew_enabled(shcfd_ctx* ctx) {
 // the 16-row sweeps apply the split Jacobians in closed form (no operator
 // copy) for the schemes whose A+-, B+- are the unpreconditioned ones
 static bool jvp16_scheme(const shcfd_ctx* ctx) {
-    // the Jacobian-free sweeps address the dq and q fields through one buffer
-    // view of all their components, whose size must stay below their drop
-    // offset (2^31 bytes)
-    const bool fits = (long long)(ctx->ny + 3) * ctx->NC * 8 < 0x7FF00000LL;
-    return ctx->use_jvp16 && fits && (ctx->p.scheme == SHCFD_SCHEME_LUSGS || ctx->p.scheme == SHCFD_SCHEME_NR);
+    return ctx->use_jvp16 && (ctx->p.scheme == SHCFD_SCHEME_LUSGS || ctx->p.scheme == SHCFD_SCHEME_NR);
 }
 
 static bool q16_layout(shcfd_ctx* ctx);
 
-// the cell data of the Jacobian-free 16-row sweeps; allocated (and cleared,
+// the cell records of the Jacobian-free 16-row sweeps; allocated (and cleared,
 // so slots of no cell hold zeros) on first use
 static bool jd16_ready(shcfd_ctx* ctx) {
-    if (ctx->djcp16) return true;
-    const int C = (ctx->dimq + 3) / 4;
-    const size_t ncp = (size_t)ctx->nsl16 * C * 64, nsc = (size_t)ctx->nsl16 * 16 * 16;
-    if (hipMalloc((void**)&ctx->djcp16, sizeof(double2) * ncp) != hipSuccess ||
-        hipMalloc((void**)&ctx->djsc16, sizeof(double) * nsc) != hipSuccess ||
-        hipMemset(ctx->djcp16, 0, sizeof(double2) * ncp) != hipSuccess ||
-        hipMemset(ctx->djsc16, 0, sizeof(double) * nsc) != hipSuccess) {
-        hipFree(ctx->djcp16);
-        hipFree(ctx->djsc16);
-        ctx->djcp16 = nullptr;
-        ctx->djsc16 = nullptr;
+    if (ctx->djrec16) return true;
+    const size_t bytes = ((size_t)ctx->nsl16 + 2 * JPAD) * jrec_off(ctx->ny, (ctx->dimq + 3) / 4);
+    const size_t pbytes = sizeof(double) * 2 * ctx->nstrips16 * ctx->nitem16;
+    if (hipMalloc((void**)&ctx->djpart16, pbytes) != hipSuccess ||
+        hipMalloc((void**)&ctx->djrec16, bytes) != hipSuccess || hipMemset(ctx->djrec16, 0, bytes) != hipSuccess) {
+        hipFree(ctx->djpart16);
+        hipFree(ctx->djrec16);
+        ctx->djpart16 = nullptr;
+        ctx->djrec16 = nullptr;
         (void)hipGetLastError();
         return false;
     }
@@ -910,7 +904,7 @@ static bool q16_layout(shcfd_ctx* ctx) {
             S.next = -1;
             S.base = nsl;  // in steps
             if (S.prev >= 0) st[S.prev].next = (int)st.size();
-            nsl += B.ni + 15;
+            nsl += (B.ni + 18 + 7) / 8 * 8;  // steps of the longest of the sweeps, whole rounds
             st.push_back(S);
         }
         (void)first;
@@ -936,6 +930,7 @@ static bool q16_layout(shcfd_ctx* ctx) {
         return false;
     }
     ctx->nstrips16 = ns;
+    ctx->nitem16 = (maxni + 18 + 15) / 16;
     ctx->nsl16 = nsl;
     ctx->bstride16 = bstride;
     return true;
@@ -948,17 +943,14 @@ static bool q16_layout(shcfd_ctx* ctx) {
 static int abpm_for_step(shcfd_ctx* ctx) {
     if (!fast_enabled(ctx)) {
         if (q16_enabled(ctx)) {
+            if (jvp16_scheme(ctx)) {
+                ctx->jd16_active = 1;  // the cell data is formed with the right-hand side
+                return SHCFD_OK;
+            }
             ProfScope ps(ctx, PROF_ABPM);
             int maxni = 0;
             for (const auto& B : ctx->hblk) maxni = std::max(maxni, B.ni);
             dim3 grid((unsigned)ctx->nstrips16, (unsigned)((maxni + 15 + 15) / 16));
-            if (jvp16_scheme(ctx)) {
-                DISPATCH_NY(ctx->ny, hipLaunchKernelGGL(k_set_jd16<NY>, grid, dim3(256), 0, ctx->stream, ctx->dev(),
-                                                        ctx->dstrips16, ctx->djcp16, ctx->djsc16));
-                LAUNCHCHK();
-                ctx->jd16_active = 1;
-                return SHCFD_OK;
-            }
             DISPATCH_NY(ctx->ny, hipLaunchKernelGGL(k_set_abpm16<NY>, grid, dim3(256), 0, ctx->stream, ctx->dev(),
                                                     ctx->dstrips16, ctx->djac16, ctx->nsl16));
             LAUNCHCHK();
@@ -1030,13 +1022,30 @@ bool fast_ready(Ctx* ctx) { return fast_enabled(static_cast<shcfd_ctx*>(ctx)); }
 }  // namespace shcfd
 }
 
+// the end of an inner iteration: (res, omega) from their n partials, and the
+// update, unless the next primitive pass applies it
+static int finish_inner(shcfd_ctx* ctx, int step_internal, const double* part, int n) {
+    { ProfScope ps(ctx, PROF_REDUCE);
+    hipLaunchKernelGGL(k_reduce_res_omega, dim3(1), dim3(256), 0, ctx->stream, ctx->dev(), part, n); }
+    if (step_internal == 1)
+        hipLaunchKernelGGL(k_copy_scal, dim3(1), dim3(1), 0, ctx->stream, ctx->dev(), (int)SCAL_RES1, (int)SCAL_RES);
+    if (ctx->defer_update) {
+        ctx->update_pending = 1;
+    } else {
+        ProfScope ps(ctx, PROF_UPDATE);
+        DISPATCH_NY(ctx->ny, TILE_LAUNCH(k_update<NY>));
+    }
+    LAUNCHCHK();
+    return SHCFD_OK;
+}
+
 static int implicit_async(shcfd_ctx* ctx, int step_internal) {
     const int ns = (int)ctx->hstrips.size();
     DevCtx d = ctx->dev();
     int* prog_f = ctx->dprog;
     int* prog_b = ctx->dprog + ns;
-    const bool jd16 = ctx->jd16_active && ctx->djcp16 && !fast_enabled(ctx);
-    const bool q16 = jd16 || (ctx->q16_active && ctx->djac16 && !fast_enabled(ctx));
+    const bool jd16 = ctx->jd16_active && ctx->djrec16 && !fast_enabled(ctx);
+    const bool q16 = ctx->q16_active && ctx->djac16 && !fast_enabled(ctx);
     ctx->q16_active = 0;
     ctx->jd16_active = 0;
     const int C16 = (ctx->dimq + 3) / 4, ns16 = ctx->nstrips16;
@@ -1047,6 +1056,34 @@ static int implicit_async(shcfd_ctx* ctx, int step_internal) {
         ctx->abpm_inline = 0;
         LAUNCHCHK();
         return rc;
+    }
+    if (jd16) {
+        const unsigned items = (unsigned)ns16 * (unsigned)ctx->nitem16;
+        double* hand_f = ctx->dbnd16;
+        double* hand_b = ctx->dbnd16 + ctx->bstride16 * (ns16 + 1);
+        { ProfScope ps(ctx, PROF_RHS);
+        DISPATCH_NY(ctx->ny, hipLaunchKernelGGL(k_rhs_jd16<NY>, dim3(items), dim3(256), 0, ctx->stream, d,
+                                                ctx->dstrips16, ns16, ctx->nitem16, ctx->dqdt_inline, ctx->djrec16,
+                                                ctx->dbnd16, ctx->bstride16)) }
+        ctx->dqdt_inline = 0;
+        ctx->abpm_inline = 0;
+        const dim3 blk((unsigned)(64 * (C16 + 2)));
+        { ProfScope ps(ctx, PROF_SWEEP_FWD);
+        DISPATCH_NY(ctx->ny, hipLaunchKernelGGL((k_sweep16j<NY, false>), dim3(ns16), blk, 0, ctx->stream, d,
+                                                ctx->dstrips16, ns16, hand_f, ctx->bstride16, ctx->spin_limit,
+                                                ctx->djrec16)) }
+        { ProfScope ps(ctx, PROF_SWEEP_BWD);
+        DISPATCH_NY(ctx->ny, hipLaunchKernelGGL((k_sweep16j<NY, true>), dim3(ns16), blk, 0, ctx->stream, d,
+                                                ctx->dstrips16, ns16, hand_b, ctx->bstride16, ctx->spin_limit,
+                                                ctx->djrec16)) }
+        { ProfScope ps(ctx, PROF_UPDATE);
+        DISPATCH_NY(ctx->ny, hipLaunchKernelGGL(k_post16j<NY>, dim3(items), dim3(256), 0, ctx->stream, d,
+                                                ctx->dstrips16, ctx->nitem16, ctx->djrec16, ctx->djpart16)) }
+        if (!inner_loop_scheme(ctx->p.scheme)) {
+            LAUNCHCHK();
+            return SHCFD_OK;
+        }
+        return finish_inner(ctx, step_internal, ctx->djpart16, (int)items);
     }
     { ProfScope ps(ctx, PROF_RHS);
     DISPATCH_NY(ctx->ny, TILE_LAUNCH(k_rhs<NY>, ctx->dprog, 2 * ns, ctx->dqdt_inline, ctx->abpm_inline)); }
@@ -1059,39 +1096,14 @@ static int implicit_async(shcfd_ctx* ctx, int step_internal) {
         { ProfScope ps(ctx, PROF_SWEEP_FWD);
         hipLaunchKernelGGL(k_fill16, dim3(256), dim3(256), 0, ctx->stream, d, ctx->dstrips16, ns16, ctx->dbnd16,
                            ctx->bstride16, ctx->dimq);
-        if (jd16)
-            DISPATCH_NY(ctx->ny, hipLaunchKernelGGL(k_sweep16j_fwd<NY>, dim3(ns16), blk, 0, ctx->stream, d,
-                                                    ctx->dstrips16, ns16, hand_f, ctx->bstride16, ctx->spin_limit,
-                                                    ctx->djcp16, ctx->djsc16))
-        else
-            DISPATCH_NY(ctx->ny, hipLaunchKernelGGL(k_sweep16_fwd<NY>, dim3(ns16), blk, 0, ctx->stream, d,
-                                                    ctx->dstrips16, ns16, hand_f, ctx->bstride16, ctx->spin_limit,
-                                                    ctx->djac16, ctx->nsl16)) }
+        DISPATCH_NY(ctx->ny, hipLaunchKernelGGL(k_sweep16_fwd<NY>, dim3(ns16), blk, 0, ctx->stream, d, ctx->dstrips16,
+                                                ns16, hand_f, ctx->bstride16, ctx->spin_limit, ctx->djac16,
+                                                ctx->nsl16)) }
         { ProfScope ps(ctx, PROF_SWEEP_BWD);
-        if (jd16)
-            DISPATCH_NY(ctx->ny, hipLaunchKernelGGL(k_sweep16j_bwd<NY>, dim3(ns16), blk, 0, ctx->stream, d,
-                                                    ctx->dstrips16, ns16, hand_b, ctx->bstride16, ctx->dpart,
-                                                    ctx->spin_limit, ctx->djcp16, ctx->djsc16))
-        else
-            DISPATCH_NY(ctx->ny, hipLaunchKernelGGL(k_sweep16_bwd<NY>, dim3(ns16), blk, 0, ctx->stream, d,
-                                                    ctx->dstrips16, ns16, hand_b, ctx->bstride16, ctx->dpart,
-                                                    ctx->spin_limit, ctx->djac16, ctx->nsl16)) }
-        if (jd16 && !inner_loop_scheme(ctx->p.scheme)) {
-            ProfScope ps(ctx, PROF_UPDATE);
-            DISPATCH_NY(ctx->ny, TILE_LAUNCH(k_add_dq<NY>));
-        }
-        if (inner_loop_scheme(ctx->p.scheme)) {
-            { ProfScope ps(ctx, PROF_REDUCE);
-            hipLaunchKernelGGL(k_reduce_res_omega, dim3(1), dim3(256), 0, ctx->stream, d, ctx->dpart, ns16); }
-            if (step_internal == 1)
-                hipLaunchKernelGGL(k_copy_scal, dim3(1), dim3(1), 0, ctx->stream, d, (int)SCAL_RES1, (int)SCAL_RES);
-            if (ctx->defer_update) {
-                ctx->update_pending = 1;
-            } else {
-                ProfScope ps(ctx, PROF_UPDATE);
-                DISPATCH_NY(ctx->ny, TILE_LAUNCH(k_update<NY>));
-            }
-        }
+        DISPATCH_NY(ctx->ny, hipLaunchKernelGGL(k_sweep16_bwd<NY>, dim3(ns16), blk, 0, ctx->stream, d, ctx->dstrips16,
+                                                ns16, hand_b, ctx->bstride16, ctx->dpart, ctx->spin_limit, ctx->djac16,
+                                                ctx->nsl16)) }
+        if (inner_loop_scheme(ctx->p.scheme)) return finish_inner(ctx, step_internal, ctx->dpart, ns16);
         LAUNCHCHK();
         return SHCFD_OK;
     }
@@ -1115,18 +1127,7 @@ static int implicit_async(shcfd_ctx* ctx, int step_internal) {
         DISPATCH_NY(ctx->ny, hipLaunchKernelGGL((k_sweep_bwd_plain<NY, false>), dim3(ns), dim3(64), 0, ctx->stream, d,
                                                 ctx->dstrips, ns, prog_b, ctx->dbnd, ctx->bnd_stride, ctx->dpart,
                                                 ctx->spin_limit, nullptr, 0LL, nullptr)) }
-    if (inner_loop_scheme(ctx->p.scheme)) {
-        { ProfScope ps(ctx, PROF_REDUCE);
-        hipLaunchKernelGGL(k_reduce_res_omega, dim3(1), dim3(256), 0, ctx->stream, d, ctx->dpart, ns); }
-        if (step_internal == 1)
-            hipLaunchKernelGGL(k_copy_scal, dim3(1), dim3(1), 0, ctx->stream, d, (int)SCAL_RES1, (int)SCAL_RES);
-        if (ctx->defer_update) {
-            ctx->update_pending = 1;
-        } else {
-            ProfScope ps(ctx, PROF_UPDATE);
-            DISPATCH_NY(ctx->ny, TILE_LAUNCH(k_update<NY>));
-        }
-    }
+    if (inner_loop_scheme(ctx->p.scheme)) return finish_inner(ctx, step_internal, ctx->dpart, ns);
     LAUNCHCHK();
     return SHCFD_OK;
 }

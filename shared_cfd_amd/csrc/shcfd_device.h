@@ -99,6 +99,16 @@ __device__ inline double shift_down4(double x) {
     return __hiloint2double(hi, lo);
 }
 
+// one row shift of a 64-bit value within the 16-lane rows (row_shr:4 towards
+// higher lanes, row_shl:4 towards lower); the lanes with no source keep `old`
+template <bool UP>
+__device__ inline double row_shift4(double old, double x) {
+    constexpr int ctrl = UP ? 0x114 : 0x104;
+    const int lo = __builtin_amdgcn_update_dpp(__double2loint(old), __double2loint(x), ctrl, 0xF, 0xF, false);
+    const int hi = __builtin_amdgcn_update_dpp(__double2hiint(old), __double2hiint(x), ctrl, 0xF, 0xF, false);
+    return __hiloint2double(hi, lo);
+}
+
 // quad broadcast with the source lane given at run time (constant after
 // unrolling, so the switch folds to one DPP pair)
 __device__ inline double quad_bcast_n(double x, int k) {

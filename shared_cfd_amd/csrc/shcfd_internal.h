@@ -192,9 +192,10 @@ struct Ctx {
     int defer_cap = 0;             // records: one per interior cell
     int q16_active = 0;            // the last set_ABpm of a step wrote the quad-row copy
     int use_jvp16 = 1;             // LU-SGS / NR at nY > 1: Jacobian-free 16-row sweeps
-    int jd16_active = 0;           // the last set_ABpm of a step wrote their cell data
-    double2* djcp16 = nullptr;     // their per-lane (c1, DHi) pairs: nsl16 x C x 64
-    double* djsc16 = nullptr;      // their cell scalars: nsl16 x 16 rows x 16
+    int jd16_active = 0;           // the next implicit update runs them
+    int nitem16 = 0;               // 16-step work items of the longest strip
+    char* djrec16 = nullptr;       // their cell records, nsl16 + 2 JPAD steps
+    double* djpart16 = nullptr;    // (res, omega) partials per work item
     int skew_active = 0;           // the last set_ABpm of a step wrote the skewed copy
     double* dskew = nullptr;
     long long skew_nsl = 0;        // slots: sum over strips of 64 (ni + 63)

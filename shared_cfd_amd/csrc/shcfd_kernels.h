@@ -554,18 +554,22 @@ template <int NY, bool SKEW>
 __global__ void k_sweep_bwd_plain(DevCtx, const Strip*, int, int*, double*, long long, double*, long long,
                                   const double*, long long, const long long*);
 template <int NY> __global__ void k_update(DevCtx, const Tile*);
-template <int NY> __global__ void k_add_dq(DevCtx, const Tile*);
 __global__ void k_reduce_res_omega(DevCtx, const double*, int);
 // quad-row sweeps for nY > 1 (k_sweep16.hip; operators from k_set_abpm16)
 template <int NY> __global__ void k_set_abpm16(DevCtx, const Strip16*, double*, long long);
 __global__ void k_fill16(DevCtx, const Strip16*, int, double*, long long, int);
-template <int NY> __global__ void k_set_jd16(DevCtx, const Strip16*, double2*, double*);
 template <int NY>
-__global__ void k_sweep16j_fwd(DevCtx, const Strip16*, int, double*, long long, long long, const double2*,
-                               const double*);
-template <int NY>
-__global__ void k_sweep16j_bwd(DevCtx, const Strip16*, int, double*, long long, double*, long long, const double2*,
-                               const double*);
+__global__ void k_rhs_jd16(DevCtx, const Strip16*, int, int, int, char*, double*, long long);
+template <int NY, bool BWD>
+__global__ void k_sweep16j(DevCtx, const Strip16*, int, double*, long long, long long, char*);
+template <int NY> __global__ void k_post16j(DevCtx, const Strip16*, int, const char*, double*);
+// bytes of a cell record of theirs, in waves of species alone and in the
+// others, and of wave w's offset in a step (w = the number of waves: the
+// step); steps of padding at both ends, which the sweeps' prefetch reads
+constexpr int JREC_S = 2304, JREC_M = 4096, JPAD = 8;
+__host__ __device__ constexpr int jrec_off(int ny, int w) {
+    return w < ny / 4 ? w * JREC_S : (ny / 4) * JREC_S + (w - ny / 4) * JREC_M;
+}
 template <int NY>
 __global__ void k_sweep16_fwd(DevCtx, const Strip16*, int, double*, long long, long long, const double*, long long);
 template <int NY>

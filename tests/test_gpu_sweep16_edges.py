@@ -1,0 +1,43 @@
+"""The closed-form sweeps of more than one species at the edges of their
+strips: block heights around multiples of the 16-row strip and its four-row
+groups, widths around the eight-step rounds, and species counts that leave
+the last compute wave with one to four components.
+
+Both sides evaluate the same update from the same state; the closed form sums
+in another order.  Each cell's increment is a chain of at most ni + nj
+products whose factors have norm below one (diagonal dominance), so the
+rounding differences add up to a small multiple of (ni + nj) eps of the
+increments; species with increments far below the others' carry the rounding
+of the larger ones, hence the scale over all components.
+"""
+import numpy as np
+import pytest
+
+from shared_cfd_amd import cases as C
+from shared_cfd_amd.native import OPT_SKEW_SWEEP, Solver
+
+pytestmark = pytest.mark.gpu
+
+
+def _increments(case, skew, reps):
+    s = Solver(case)
+    s.set_option(OPT_SKEW_SWEEP, skew)
+    s.prepare()
+    for k in range(reps):
+        s.step(k + 1, 0)
+    out = [s.download("Q", b)[2:-2, 2:-2] - case.q0[b][2:-2, 2:-2] for b in range(case.nblocks)]
+    s.close()
+    return out
+
+
+@pytest.mark.parametrize("scheme", [C.SCHEME_LUSGS, C.SCHEME_NR])
+@pytest.mark.parametrize("ny,ni,nj", [(2, 2, 2), (2, 14, 17), (3, 13, 4), (4, 15, 15), (5, 14, 5), (8, 30, 16),
+                                      (9, 31, 17), (9, 6, 48), (9, 22, 49), (10, 3, 65), (11, 130, 7), (13, 62, 33),
+                                      (16, 21, 33)])
+def test_strip_edges(scheme, ny, ni, nj):
+    case = C.random_case(seed=ni + nj, ni=(ni, 9), nj=(nj, 20), ny=ny, scheme=scheme)
+    case.params.res_rate_warning = case.params.res_rate_error = 1e300
+    for a, b in zip(_increments(case, 1, 2), _increments(case, 0, 2)):
+        scale = np.max(np.abs(b))
+        assert scale > 0.0
+        assert np.max(np.abs(a - b)) <= 1e-12 * scale
