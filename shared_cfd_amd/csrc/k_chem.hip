@@ -3,9 +3,20 @@
 // point-implicit LU update per cell) and a batched 0-D harness (Fex, Jex,
 // calc_T, CHEMEQ2, point-implicit on arrays of independent states).
 //
-// One lane owns one cell; the per-cell species vectors and the 10x10
-// Jacobian stay in registers (shcfd_chem.h).  The mechanism tables are read
-// through uniform (scalar) loads.
+// One lane owns one cell; the per-cell species vectors stay in registers
+// (shcfd_chem.h).  The mechanism tables are read through uniform (scalar)
+// loads.
+//
+// Bound by one wave's instruction issue: a lane needs up to 512 registers, so
+// a SIMD holds one wave and nothing covers its waits.  Those were the larger
+// part: species arrays indexed at run time sat in scratch and LDS memory, each
+// reaction's table entries were read where they were used, and the thermo sums
+// of the energy equation were kept, spilled, through the loop over the
+// reactions.  With the arrays in VGPRs, the next reaction's record read ahead
+// and the energy sums formed after the loop, at nine species (times in us):
+// point-implicit update on 1024 x 512 1488 -> 731 (46% of the wave cycles
+// waiting, then 36%), CHEMEQ2 on 223 x 99 154 -> 76, thermo on 1024 x 512
+// 121 -> 85, 16384 point-implicit states 1673 -> 461.
 #include "shcfd_chem.h"
 #include "shcfd_device.h"
 #include "shcfd_dvode.h"
@@ -145,14 +156,16 @@ __global__ void k_set_iflag(DevCtx d, int slot, int v) {
 
 // proceed_reaction with the point-implicit update (MODE 2), one wavefront per
 // workgroup: the (NS+1)^2 Newton matrix of each lane lives in LDS
-// (lane-interleaved) instead of registers, so the runtime species rows of
-// the Jacobian and the LU's pivot rows are indexed directly.  Workgroup k
-// handles row k % tile_rows of tile k / tile_rows.
+// (lane-interleaved), its last two columns in registers, so the runtime
+// species rows of the Jacobian and the LU's pivot rows are indexed directly.
+// Workgroup k handles row k % tile_rows of tile k / tile_rows.  With all
+// columns in LDS three of the CU's four SIMDs had a wave (957 us against 949
+// while scratch traffic bounded both).
 template <int NS>
 __global__ void __launch_bounds__(64) k_reaction_lds(DevCtx d, const Tile* tiles, int tile_rows,
                                                       const shcfd_mech* __restrict__ m) {
     constexpr int N = NS + 1;
-    __shared__ double jsh[N * N * 64];
+    __shared__ double jsh[chem::LdsMat<N>::SIZE];
     const Tile tl = tiles[blockIdx.x / tile_rows];
     const int i = tl.i0 + (int)threadIdx.x, j = tl.j0 + (int)(blockIdx.x % tile_rows);
     const DevBlock B = d.blk[tl.b];
@@ -181,9 +194,12 @@ __global__ void __launch_bounds__(64) k_reaction_lds(DevCtx d, const Tile* tiles
 }
 
 // batched 0-D harness: cell q's input row starts at in + q*ldi, output row at
-// out + q*ldo; status[q] receives an iteration/attempt count or -code.
+// out + q*ldo; status[q] receives an iteration/attempt count or -code.  One
+// wave per workgroup: 16384 rows are 256 waves, one for each CU (workgroups of
+// four waves, with the matrix in registers and scratch, 1673 us; 553 with one
+// and the matrix in LDS).
 template <int NS, int op>
-__global__ void __launch_bounds__(256) k_chem0d(const shcfd_mech* __restrict__ m, int n, const double* in, int ldi,
+__global__ void __launch_bounds__(64) k_chem0d(const shcfd_mech* __restrict__ m, int n, const double* in, int ldi,
                                                 double* out, int ldo, int* status, double dt) {
     constexpr int N = NS + 1;
     int q = blockIdx.x * blockDim.x + threadIdx.x;
@@ -241,7 +257,13 @@ __global__ void __launch_bounds__(256) k_chem0d(const shcfd_mech* __restrict__ m
         for (int k = 0; k < NS; k++) vrho[k] = x[k];
         int it = 0;
         double T1 = x[NS];
-        int e = chem::point_implicit<NS>(m, x[NS], vrho, dt, it, T1);
+        int e;
+        if constexpr (NS <= SHCFD_LDS_NEWTON_MAX_NS) {
+            __shared__ double jsh[chem::LdsMat<N>::SIZE];
+            e = chem::point_implicit_lds<NS>(m, x[NS], vrho, dt, it, T1, jsh + threadIdx.x);
+        } else {
+            e = chem::point_implicit<NS>(m, x[NS], vrho, dt, it, T1);
+        }
         st = e ? -e : it;
 #pragma unroll
         for (int k = 0; k < NS; k++) y[k] = vrho[k];

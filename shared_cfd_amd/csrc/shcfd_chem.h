@@ -5,10 +5,8 @@
 // store/therm_lib/chemkin/uvhp/uv/FJ.f90; each function names the lines it
 // covers.  NS (the species count) is a template parameter so per-species
 // vectors live in registers.  The mechanism's species indices are run-time
-// but uniform across a wavefront; they are applied with unrolled
-// compare-and-select over the NS slots (sel_get / sel_add), which keeps
-// every array statically indexed (no scratch memory) and each update in the
-// reference's order.
+// but uniform across a wavefront; vectors that they index are SVec, which keeps
+// them in registers, with each update in the reference's order.
 #pragma once
 #include "../../include/shcfd_types.h"
 
@@ -48,12 +46,12 @@ SHCFD_HD double pow2i(int k) {
 }
 
 SHCFD_HD double dexp(double x) {
-    if (x != x) return x + x;
-    if (x > 709.782712893384) return __builtin_huge_val();
-    if (x < -745.1332191019412) return 0.0;
-    double kd = __builtin_rint(x * INV_LN2);
+    // no branch: the lanes of a wave would take them one after another, and the
+    // vector registers would be saved around them
+    const double xc = x > 709.782712893384 ? 709.0 : x < -745.1332191019412 ? -745.0 : x != x ? 0.0 : x;
+    double kd = __builtin_rint(xc * INV_LN2);
     int k = (int)kd;
-    double r = __builtin_fma(-kd, LN2_HI, x);
+    double r = __builtin_fma(-kd, LN2_HI, xc);
     r = __builtin_fma(-kd, LN2_LO, r);
     double p = 1.0 / 6227020800.0;
     p = __builtin_fma(p, r, 1.0 / 479001600.0);
@@ -70,20 +68,16 @@ SHCFD_HD double dexp(double x) {
     p = __builtin_fma(p, r, 1.0);
     p = __builtin_fma(p, r, 1.0);
     int k1 = k / 2, k2 = k - k1;
-    return (p * pow2i(k1)) * pow2i(k2);
+    const double e = (p * pow2i(k1)) * pow2i(k2);
+    return x > 709.782712893384 ? __builtin_huge_val() : x < -745.1332191019412 ? 0.0 : x != x ? x + x : e;
 }
 
 SHCFD_HD double dlog(double x) {
-    if (x != x || x < 0.0) return __builtin_nan("");
-    if (x == 0.0) return -__builtin_huge_val();
-    if (x == __builtin_huge_val()) return x;
-    int kadj = 0;
-    if (x < 2.2250738585072014e-308) {
-        x = x * 18014398509481984.0;
-        kadj = -54;
-    }
+    const bool small = x < 2.2250738585072014e-308;
+    const int kadj = small ? -54 : 0;
+    const double xs = small ? x * 18014398509481984.0 : x;
     unsigned long long u;
-    __builtin_memcpy(&u, &x, 8);
+    __builtin_memcpy(&u, &xs, 8);
     int k = (int)((u >> 52) & 0x7ff) - 1023 + kadj;
     u = (u & 0x000fffffffffffffULL) | 0x3ff0000000000000ULL;
     double m;
@@ -108,7 +102,8 @@ SHCFD_HD double dlog(double x) {
     double f2 = f + f;
     double lm = __builtin_fma(f2, t, f2);
     double kd = (double)k;
-    return kd * LN2_HI + __builtin_fma(kd, LN2_LO, lm);
+    const double y = kd * LN2_HI + __builtin_fma(kd, LN2_LO, lm);
+    return x == 0.0 ? -__builtin_huge_val() : x == __builtin_huge_val() ? x : x >= 0.0 ? y : __builtin_nan("");
 }
 
 SHCFD_HD double dlog10(double x) { return dlog(x) * INV_LN10; }
@@ -116,27 +111,43 @@ SHCFD_HD double dsqrt(double x) { return __builtin_sqrt(x); }
 SHCFD_HD double fmax2(double a, double b) { return (a > b || b != b) ? a : b; }
 SHCFD_HD double fmin2(double a, double b) { return (a < b || b != b) ? a : b; }
 
-// ---- uniform run-time index into a register vector --------------------------
+// ---- a register vector with a uniform run-time index --------------------------
+// On the device a vector type: its elements stay in registers and the element
+// of a run-time index, the same in every active lane, is moved by VGPR
+// indexing (4 instructions).  A plain array indexed at run time, also through
+// a chain of compares, ends up in scratch or LDS memory.
 template <int N>
-SHCFD_HD double sel_get(const double (&a)[N], int idx) {
-    double x = a[0];
+struct SVec {
+#if defined(__HIP_DEVICE_COMPILE__)
+    typedef double V __attribute__((ext_vector_type(N <= 2 ? 2 : N <= 4 ? 4 : N <= 8 ? 8 : 16)));
+    V v;
+    static __device__ inline int uni(int k) { return __builtin_amdgcn_readfirstlane(k); }
+#else
+    double v[N];
+    static inline int uni(int k) { return k; }
+#endif
+    SHCFD_HD double get(int k) const { return v[k]; }          // k known at compile time
+    SHCFD_HD void set(int k, double x) { v[k] = x; }
+    SHCFD_HD double at(int k) const { return v[uni(k)]; }      // k uniform
+    SHCFD_HD void put(int k, double x) { v[uni(k)] = x; }
+    SHCFD_HD void add(int k, double x) {
+        k = uni(k);
+        v[k] = v[k] + x;
+    }
+    SHCFD_HD void sub(int k, double x) {
+        k = uni(k);
+        v[k] = v[k] - x;
+    }
+    SHCFD_HD void fill(double x) {
 #pragma unroll
-    for (int k = 1; k < N; k++)
-        if (k == idx) x = a[k];
-    return x;
-}
-template <int N>
-SHCFD_HD void sel_add(double (&a)[N], int idx, double v) {
+        for (int k = 0; k < N; k++) v[k] = x;
+    }
+    template <int M>
+    SHCFD_HD void from(const double (&a)[M]) {
 #pragma unroll
-    for (int k = 0; k < N; k++)
-        if (k == idx) a[k] = a[k] + v;
-}
-template <int N>
-SHCFD_HD void sel_sub(double (&a)[N], int idx, double v) {
-#pragma unroll
-    for (int k = 0; k < N; k++)
-        if (k == idx) a[k] = a[k] - v;
-}
+        for (int k = 0; k < N; k++) v[k] = a[k];
+    }
+};
 
 // ---- NASA-7 basis vectors (sub_chem.f90:20-150) ------------------------------
 struct Basis {
@@ -189,57 +200,81 @@ SHCFD_HD const double* coeff_at(const shcfd_mech* m, int k, double T) {
     return m->coeff[k][(T <= m->tthre[k][2]) ? 0 : 1];
 }
 
-// species sums of FJ.f90:185-197 / :516-540
+// species sums of FJ.f90:185-197 / :516-540, in two parts: what the reactions
+// need, and what the energy equation needs after them, so that a part's
+// registers are free while the other is in use
 template <int NS, bool DERIV>
-struct SpeciesThermo {
-    double vmu0rt[NS], vert[NS], vcvr[NS], vdmu0rt[DERIV ? NS : 1], vdcvrdT[DERIV ? NS : 1];
+struct SpeciesMu {
+    SVec<NS> vmu0rt, vdmu0rt;  // vdmu0rt: DERIV
 };
 template <int NS, bool DERIV>
-SHCFD_HD void species_thermo(const shcfd_mech* m, double T, double logT, SpeciesThermo<NS, DERIV>& S) {
+SHCFD_HD void species_mu(const shcfd_mech* m, double T, double logT, SpeciesMu<NS, DERIV>& S) {
     Basis B;
     set_coeff<DERIV>(T, logT, B);
 #pragma unroll
     for (int j = 0; j < NS; j++) {
         const double* c = coeff_at(m, j, T);
-        double t1 = 0.0, t2 = DERIV ? 0.0 : -1.0, t3 = -1.0, t4 = -1.0, t5 = 0.0;
-        if (DERIV) {
+        double t1 = 0.0, t2 = 0.0;
 #pragma unroll
-            for (int i = 0; i < 7; i++) {
-                double tmp = c[i];
-                t1 = t1 + tmp * B.cmurt[i];
-                t2 = t2 + tmp * B.cdmurt[i];
-                t3 = t3 + tmp * B.chrt[i];
-                t4 = t4 + tmp * B.ccpr[i];
-                t5 = t5 + tmp * B.cdcpr[i];
-            }
-            S.vmu0rt[j] = t1;
-            S.vdmu0rt[j] = t2;
-            S.vert[j] = t3;
-            S.vcvr[j] = t4;
-            S.vdcvrdT[j] = t5;
-        } else {
-#pragma unroll
-            for (int i = 0; i < 7; i++) {
-                double tmp = c[i];
-                t1 = t1 + tmp * B.cmurt[i];
-                t2 = t2 + tmp * B.chrt[i];
-                t3 = t3 + tmp * B.ccpr[i];
-            }
-            S.vmu0rt[j] = t1;
-            S.vert[j] = t2;
-            S.vcvr[j] = t3;
+        for (int i = 0; i < 7; i++) {
+            double tmp = c[i];
+            t1 = t1 + tmp * B.cmurt[i];
+            if (DERIV) t2 = t2 + tmp * B.cdmurt[i];
         }
+        S.vmu0rt.set(j, t1);
+        if (DERIV) S.vdmu0rt.set(j, t2);
     }
 }
+template <bool DERIV>
+SHCFD_HD void species_energy(const shcfd_mech* m, const Basis& B, int j, double T, double& vert, double& vcvr,
+                             double& vdcvrdT) {
+    const double* c = coeff_at(m, j, T);
+    double t3 = -1.0, t4 = -1.0, t5 = 0.0;
+#pragma unroll
+    for (int i = 0; i < 7; i++) {
+        double tmp = c[i];
+        t3 = t3 + tmp * B.chrt[i];
+        t4 = t4 + tmp * B.ccpr[i];
+        if (DERIV) t5 = t5 + tmp * B.cdcpr[i];
+    }
+    vert = t3;
+    vcvr = t4;
+    vdcvrdT = t5;
+}
+
+// Reaction i's part of the mechanism tables.  They are the same for a whole
+// wavefront, and a scalar load is waited for at its first use, so each loop
+// over the reactions reads the next one's record before it works on this one.
+struct Rxn {
+    int kind, reverse_off, exist_m, snu, num[2], ind[2][3];
+    double abe[3], cabe[3];
+    SHCFD_HD void load(const shcfd_mech* m, int i) {
+        kind = m->kind[i];
+        reverse_off = m->reverse_off[i];
+        exist_m = m->exist_m[i];
+        snu = m->snu[i];
+#pragma unroll
+        for (int s = 0; s < 2; s++) {
+            num[s] = m->num_nu[i][s];
+#pragma unroll
+            for (int k = 0; k < 3; k++) ind[s][k] = m->ind_nu[i][s][k];
+        }
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            abe[k] = m->abe[i][k];
+            cabe[k] = m->cabe[i][k];
+        }
+    }
+};
 
 // log rate constants of reaction i (FJ.f90:212-256 and :549-633)
 template <int NS, bool DERIV>
-SHCFD_HD void rate_constants(const shcfd_mech* m, int i, double T, double logT, double Tinv, double logPRT,
-                             double vlogM, const SpeciesThermo<NS, DERIV>& S, double* vlogk, double* dlnkdT,
+SHCFD_HD void rate_constants(const shcfd_mech* m, int i, const Rxn& R, double T, double logT, double Tinv, double logPRT,
+                             double vlogM, const SpeciesMu<NS, DERIV>& S, double* vlogk, double* dlnkdT,
                              double& dlnkdlnM) {
-    const double* abe = m->abe[i];
-    const double* cabe = m->cabe[i];
-    int kind = m->kind[i];
+    const double* abe = R.abe;
+    const double* cabe = R.cabe;
+    const int kind = R.kind;
     vlogk[0] = abe[0] + abe[1] * logT - abe[2] * Tinv;
     vlogk[1] = 0.0;
     if (DERIV) {
@@ -250,7 +285,7 @@ SHCFD_HD void rate_constants(const shcfd_mech* m, int i, double T, double logT, 
         vlogk[0] = vlogk[0] + vlogM;
         if (DERIV) dlnkdlnM = 1.0;
     }
-    if (m->reverse_off[i] != 0) return;
+    if (R.reverse_off != 0) return;
     if (kind == SHCFD_RXN_REV || kind == SHCFD_RXN_M_REV) {
         vlogk[1] = cabe[0] + cabe[1] * logT - cabe[2] * Tinv;
         if (DERIV) dlnkdT[1] = (cabe[1] + cabe[2] * Tinv) * Tinv;
@@ -307,39 +342,47 @@ SHCFD_HD void rate_constants(const shcfd_mech* m, int i, double T, double logT, 
     }
     // reverse rate through K_c (FJ.f90:246-256, :615-630)
     double numu0rt = 0.0, nudmu0rt = 0.0;
-    for (int k = 0; k < m->num_nu[i][0]; k++) {
-        int it = m->ind_nu[i][0][k];
-        numu0rt = numu0rt - sel_get(S.vmu0rt, it);
-        if (DERIV) nudmu0rt = nudmu0rt - sel_get(S.vdmu0rt, it);
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        if (k >= R.num[0]) break;
+        const int it = R.ind[0][k];
+        numu0rt = numu0rt - S.vmu0rt.at(it);
+        if (DERIV) nudmu0rt = nudmu0rt - S.vdmu0rt.at(it);
     }
-    for (int k = 0; k < m->num_nu[i][1]; k++) {
-        int it = m->ind_nu[i][1][k];
-        numu0rt = numu0rt + sel_get(S.vmu0rt, it);
-        if (DERIV) nudmu0rt = nudmu0rt + sel_get(S.vdmu0rt, it);
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        if (k >= R.num[1]) break;
+        const int it = R.ind[1][k];
+        numu0rt = numu0rt + S.vmu0rt.at(it);
+        if (DERIV) nudmu0rt = nudmu0rt + S.vdmu0rt.at(it);
     }
-    vlogk[1] = vlogk[0] - m->snu[i] * logPRT + numu0rt;
-    if (DERIV) dlnkdT[1] = dlnkdT[0] + m->snu[i] * Tinv + nudmu0rt;
+    vlogk[1] = vlogk[0] - R.snu * logPRT + numu0rt;
+    if (DERIV) dlnkdT[1] = dlnkdT[0] + R.snu * Tinv + nudmu0rt;
 }
 
 // third-body concentration (FJ.f90:199-210)
-template <int N>
-SHCFD_HD double third_body(const shcfd_mech* m, int i, const double (&n)[N], double sn, double logsn, double& vM) {
+template <int NS>
+SHCFD_HD double third_body(const shcfd_mech* m, int i, const SVec<NS>& n, double sn, double logsn, double& vM) {
     double tmp = sn;
-    for (int j = 0; j < m->num_m[i]; j++) tmp = tmp + m->men[i][j] * sel_get(n, m->ind_m[i][j]);
+    for (int j = 0; j < m->num_m[i]; j++) tmp = tmp + m->men[i][j] * n.at(m->ind_m[i][j]);
     vM = tmp;
     return (tmp == sn) ? logsn : dlog(tmp);
 }
 
 // forward minus reverse rate of reaction i (FJ.f90:272-284)
 template <int NS>
-SHCFD_HD void rates(const shcfd_mech* m, int i, const double (&n)[NS + 1], const double* vlogk, double& rf, double& rr) {
+SHCFD_HD void rates(const Rxn& R, const SVec<NS>& n, const double* vlogk, double& rf, double& rr) {
     double r = dexp(vlogk[0]);
-    for (int k = 0; k < m->num_nu[i][0]; k++) r = r * sel_get(n, m->ind_nu[i][0][k]);
+#pragma unroll
+    for (int k = 0; k < 3; k++)
+        if (k < R.num[0]) r = r * n.at(R.ind[0][k]);
     rf = r;
     rr = 0.0;
-    if (m->reverse_off[i] == 0) {
+    if (R.reverse_off == 0) {
         r = dexp(vlogk[1]);
-        for (int k = 0; k < m->num_nu[i][1]; k++) r = r * sel_get(n, m->ind_nu[i][1][k]);
+#pragma unroll
+        for (int k = 0; k < 3; k++)
+            if (k < R.num[1]) r = r * n.at(R.ind[1][k]);
         rr = r;
     }
 }
@@ -352,26 +395,41 @@ SHCFD_HD void fex(const shcfd_mech* m, const double (&n)[NS + 1], double (&dndt)
 #pragma unroll
     for (int j = 0; j < NS; j++) sn = sn + n[j];
     double logsn = dlog(sn);
-    SpeciesThermo<NS, false> S;
-    species_thermo<NS, false>(m, T, logT, S);
-#pragma unroll
-    for (int j = 0; j <= NS; j++) dndt[j] = 0.0;
+    SpeciesMu<NS, false> S;
+    species_mu<NS, false>(m, T, logT, S);
+    SVec<NS> nv, w;
+    nv.from(n);
+    w.fill(0.0);
     double vlogM = 0.0, vM = 0.0, unused = 0.0;
-    for (int i = 0; i < m->nr; i++) {
-        if (m->exist_m[i]) vlogM = third_body(m, i, n, sn, logsn, vM);
+    const int nr = m->nr;
+    Rxn next;
+    next.load(m, 0);
+    for (int i = 0; i < nr; i++) {
+        const Rxn R = next;
+        next.load(m, i + 1 < nr ? i + 1 : i);
+        if (R.exist_m) vlogM = third_body<NS>(m, i, nv, sn, logsn, vM);
         double vlogk[2];
-        rate_constants<NS, false>(m, i, T, logT, Tinv, logPRT, vlogM, S, vlogk, nullptr, unused);
+        rate_constants<NS, false>(m, i, R, T, logT, Tinv, logPRT, vlogM, S, vlogk, nullptr, unused);
         double rf, rr;
-        rates<NS>(m, i, n, vlogk, rf, rr);
-        double Dr = (m->reverse_off[i] == 0) ? rf - rr : rf;
-        for (int k = 0; k < m->num_nu[i][0]; k++) sel_sub(dndt, m->ind_nu[i][0][k], Dr);
-        for (int k = 0; k < m->num_nu[i][1]; k++) sel_add(dndt, m->ind_nu[i][1][k], Dr);
+        rates<NS>(R, nv, vlogk, rf, rr);
+        double Dr = (R.reverse_off == 0) ? rf - rr : rf;
+#pragma unroll
+        for (int k = 0; k < 3; k++)
+            if (k < R.num[0]) w.sub(R.ind[0][k], Dr);
+#pragma unroll
+        for (int k = 0; k < 3; k++)
+            if (k < R.num[1]) w.add(R.ind[1][k], Dr);
     }
+    Basis B;
+    set_coeff<false>(T, logT, B);
     double de = 0.0, cv = 0.0;
 #pragma unroll
     for (int j = 0; j < NS; j++) {
-        de = de + S.vert[j] * dndt[j];
-        cv = cv + S.vcvr[j] * n[j];
+        double vert, vcvr, unused_d;
+        species_energy<false>(m, B, j, T, vert, vcvr, unused_d);
+        dndt[j] = w.get(j);
+        de = de + vert * dndt[j];
+        cv = cv + vcvr * n[j];
     }
     dndt[NS] = -(de * T / cv);
 }
@@ -384,32 +442,50 @@ SHCFD_HD void fex_var(const shcfd_mech* m, const double (&n)[NS + 1], double (&d
 #pragma unroll
     for (int j = 0; j < NS; j++) sn = sn + n[j];
     double logsn = dlog(sn);
-    SpeciesThermo<NS, false> S;
-    species_thermo<NS, false>(m, T, logT, S);
-#pragma unroll
-    for (int j = 0; j <= NS; j++) {
-        dp[j] = 0.0;
-        dm[j] = 0.0;
-    }
+    SpeciesMu<NS, false> S;
+    species_mu<NS, false>(m, T, logT, S);
+    SVec<NS> nv, wp, wm;
+    nv.from(n);
+    wp.fill(0.0);
+    wm.fill(0.0);
     double vlogM = 0.0, vM = 0.0, unused = 0.0;
-    for (int i = 0; i < m->nr; i++) {
-        if (m->exist_m[i]) vlogM = third_body(m, i, n, sn, logsn, vM);
+    const int nr = m->nr;
+    Rxn next;
+    next.load(m, 0);
+    for (int i = 0; i < nr; i++) {
+        const Rxn R = next;
+        next.load(m, i + 1 < nr ? i + 1 : i);
+        if (R.exist_m) vlogM = third_body<NS>(m, i, nv, sn, logsn, vM);
         double vlogk[2];
-        rate_constants<NS, false>(m, i, T, logT, Tinv, logPRT, vlogM, S, vlogk, nullptr, unused);
+        rate_constants<NS, false>(m, i, R, T, logT, Tinv, logPRT, vlogM, S, vlogk, nullptr, unused);
         double rf, rr;
-        rates<NS>(m, i, n, vlogk, rf, rr);
-        for (int k = 0; k < m->num_nu[i][0]; k++) sel_sub(dm, m->ind_nu[i][0][k], rf);
-        for (int k = 0; k < m->num_nu[i][1]; k++) sel_add(dp, m->ind_nu[i][1][k], rf);
-        if (m->reverse_off[i] == 0) {
-            for (int k = 0; k < m->num_nu[i][0]; k++) sel_add(dp, m->ind_nu[i][0][k], rr);
-            for (int k = 0; k < m->num_nu[i][1]; k++) sel_sub(dm, m->ind_nu[i][1][k], rr);
+        rates<NS>(R, nv, vlogk, rf, rr);
+#pragma unroll
+        for (int k = 0; k < 3; k++)
+            if (k < R.num[0]) wm.sub(R.ind[0][k], rf);
+#pragma unroll
+        for (int k = 0; k < 3; k++)
+            if (k < R.num[1]) wp.add(R.ind[1][k], rf);
+        if (R.reverse_off == 0) {
+#pragma unroll
+            for (int k = 0; k < 3; k++)
+                if (k < R.num[0]) wp.add(R.ind[0][k], rr);
+#pragma unroll
+            for (int k = 0; k < 3; k++)
+                if (k < R.num[1]) wm.sub(R.ind[1][k], rr);
         }
     }
+    Basis B;
+    set_coeff<false>(T, logT, B);
     double de = 0.0, cv = 0.0;
 #pragma unroll
     for (int j = 0; j < NS; j++) {
-        de = de + S.vert[j] * (dp[j] + dm[j]);
-        cv = cv + S.vcvr[j] * n[j];
+        double vert, vcvr, unused_d;
+        species_energy<false>(m, B, j, T, vert, vcvr, unused_d);
+        dp[j] = wp.get(j);
+        dm[j] = wm.get(j);
+        de = de + vert * (dp[j] + dm[j]);
+        cv = cv + vcvr * n[j];
     }
     double dT = -(de * T / cv);
     dp[NS] = fmax2(dT, 0.0);
@@ -425,38 +501,51 @@ struct RegMat {
     SHCFD_HD double get(int a, int b) const { return J[a][b]; }
     SHCFD_HD void set(int a, int b, double v) { J[a][b] = v; }
     template <int NR>
-    SHCFD_HD void sub_row(int it, const double (&v)[N]) {
+    SHCFD_HD void sub_row(int it, const SVec<NR>& v, double vT) {
 #pragma unroll
         for (int a = 0; a < NR; a++)
             if (a == it) {
 #pragma unroll
-                for (int b = 0; b < N; b++) J[a][b] = J[a][b] - v[b];
+                for (int b = 0; b < N; b++) J[a][b] = J[a][b] - (b < NR ? v.get(b < NR ? b : 0) : vT);
             }
     }
     template <int NR>
-    SHCFD_HD void add_row(int it, const double (&v)[N]) {
+    SHCFD_HD void add_row(int it, const SVec<NR>& v, double vT) {
 #pragma unroll
         for (int a = 0; a < NR; a++)
             if (a == it) {
 #pragma unroll
-                for (int b = 0; b < N; b++) J[a][b] = J[a][b] + v[b];
+                for (int b = 0; b < N; b++) J[a][b] = J[a][b] + (b < NR ? v.get(b < NR ? b : 0) : vT);
             }
     }
 };
+// columns 0 .. NL-1 in LDS, the last two in registers, so that at nine species
+// four workgroups of one wave fit a CU's 160 KB: one for each of its SIMDs
 template <int N>
 struct LdsMat {
-    double* p;  // this lane's element (0,0); element (a,b) at p[(a N + b) 64]
-    __device__ double get(int a, int b) const { return p[(a * N + b) * 64]; }
-    __device__ void set(int a, int b, double v) { p[(a * N + b) * 64] = v; }
-    template <int NR>
-    __device__ void sub_row(int it, const double (&v)[N]) {
-#pragma unroll
-        for (int b = 0; b < N; b++) p[(it * N + b) * 64] = p[(it * N + b) * 64] - v[b];
+    static constexpr int NL = N - 2;
+    static constexpr int SIZE = NL > 0 ? 64 * N * NL : 1;  // doubles per wave
+    double* p;  // this lane's element (0,0); element (a,b) at p[(a NL + b) 64]
+    SVec<N> c[2];
+    SHCFD_HD double& at(int a, int b) const { return p[(a * NL + b) * 64]; }
+    SHCFD_HD double get(int a, int b) const { return b < NL ? at(a, b) : c[b - NL].get(a); }
+    SHCFD_HD void set(int a, int b, double v) {
+        if (b < NL) at(a, b) = v;
+        else c[b - NL].set(a, v);
     }
     template <int NR>
-    __device__ void add_row(int it, const double (&v)[N]) {
+    SHCFD_HD void sub_row(int it, const SVec<NR>& v, double vT) {
 #pragma unroll
-        for (int b = 0; b < N; b++) p[(it * N + b) * 64] = p[(it * N + b) * 64] + v[b];
+        for (int b = 0; b < NL; b++) at(it, b) = at(it, b) - v.get(b);
+        c[0].sub(it, v.get(NR - 1));
+        c[1].sub(it, vT);
+    }
+    template <int NR>
+    SHCFD_HD void add_row(int it, const SVec<NR>& v, double vT) {
+#pragma unroll
+        for (int b = 0; b < NL; b++) at(it, b) = at(it, b) + v.get(b);
+        c[0].add(it, v.get(NR - 1));
+        c[1].add(it, vT);
     }
 };
 
@@ -470,66 +559,89 @@ SHCFD_HD void jex_impl(const shcfd_mech* m, const double (&n)[NS + 1], Mat& J, d
     for (int j = 0; j < NS; j++) sn = sn + n[j];
     sn = fmax2(sn, 1e-300);
     double logsn = dlog(sn);
-    SpeciesThermo<NS, true> S;
-    species_thermo<NS, true>(m, T, logT, S);
+    SpeciesMu<NS, true> S;
+    species_mu<NS, true>(m, T, logT, S);
+    SVec<NS> nv, w;
+    nv.from(n);
+    w.fill(0.0);
 #pragma unroll
-    for (int a = 0; a < N; a++) {
-        dndt[a] = 0.0;
+    for (int a = 0; a < N; a++)
 #pragma unroll
         for (int b = 0; b < N; b++) J.set(a, b, 0.0);
-    }
     double vlogM = 0.0, vM = 0.0, dlnkdlnM = 0.0;
-    for (int i = 0; i < m->nr; i++) {
-        if (m->exist_m[i]) vlogM = third_body(m, i, n, sn, logsn, vM);
+    const int nr = m->nr;
+    Rxn next;
+    next.load(m, 0);
+    for (int i = 0; i < nr; i++) {
+        const Rxn R = next;
+        next.load(m, i + 1 < nr ? i + 1 : i);
+        if (R.exist_m) vlogM = third_body<NS>(m, i, nv, sn, logsn, vM);
         double vlogk[2], dlnkdT[2];
-        rate_constants<NS, true>(m, i, T, logT, Tinv, logPRT, vlogM, S, vlogk, dlnkdT, dlnkdlnM);
-        double drdn[N];
-#pragma unroll
-        for (int k = 0; k < NS; k++) drdn[k] = 0.0;
+        rate_constants<NS, true>(m, i, R, T, logT, Tinv, logPRT, vlogM, S, vlogk, dlnkdT, dlnkdlnM);
+        SVec<NS> drdn;
+        drdn.fill(0.0);
         double r = dexp(vlogk[0]);
-        for (int k = 0; k < m->num_nu[i][0]; k++) r = r * sel_get(n, m->ind_nu[i][0][k]);
+#pragma unroll
+        for (int k = 0; k < 3; k++)
+            if (k < R.num[0]) r = r * nv.at(R.ind[0][k]);
         double Dr = r;
-        drdn[NS] = dlnkdT[0] * r;
-        for (int k = 0; k < m->num_nu[i][0]; k++) {
-            int it = m->ind_nu[i][0][k];
-            sel_add(drdn, it, r / sel_get(n, it));
+        double drdT = dlnkdT[0] * r;
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            if (k >= R.num[0]) break;
+            const int it = R.ind[0][k];
+            drdn.add(it, r / nv.at(it));
         }
-        if (m->reverse_off[i] == 0) {
+        if (R.reverse_off == 0) {
             r = dexp(vlogk[1]);
-            for (int k = 0; k < m->num_nu[i][1]; k++) r = r * sel_get(n, m->ind_nu[i][1][k]);
+#pragma unroll
+            for (int k = 0; k < 3; k++)
+                if (k < R.num[1]) r = r * nv.at(R.ind[1][k]);
             Dr = Dr - r;
-            drdn[NS] = drdn[NS] - r * dlnkdT[1];
-            for (int k = 0; k < m->num_nu[i][1]; k++) {
-                int it = m->ind_nu[i][1][k];
-                sel_sub(drdn, it, r / sel_get(n, it));
+            drdT = drdT - r * dlnkdT[1];
+#pragma unroll
+            for (int k = 0; k < 3; k++) {
+                if (k >= R.num[1]) break;
+                const int it = R.ind[1][k];
+                drdn.sub(it, r / nv.at(it));
             }
         }
-        if (m->exist_m[i]) {
+        if (R.exist_m) {
             double t1 = Dr * dlnkdlnM / vM;
 #pragma unroll
-            for (int k = 0; k < NS; k++) drdn[k] = drdn[k] + t1;
-            for (int k = 0; k < m->num_m[i]; k++) sel_add(drdn, m->ind_m[i][k], t1 * m->men[i][k]);
+            for (int k = 0; k < NS; k++) drdn.set(k, drdn.get(k) + t1);
+            for (int k = 0; k < m->num_m[i]; k++) drdn.add(m->ind_m[i][k], t1 * m->men[i][k]);
         }
-        for (int k = 0; k < m->num_nu[i][0]; k++) {
-            int it = m->ind_nu[i][0][k];
-            sel_sub(dndt, it, Dr);
-            J.template sub_row<NS>(it, drdn);
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            if (k >= R.num[0]) break;
+            const int it = R.ind[0][k];
+            w.sub(it, Dr);
+            J.template sub_row<NS>(it, drdn, drdT);
         }
-        for (int k = 0; k < m->num_nu[i][1]; k++) {
-            int it = m->ind_nu[i][1][k];
-            sel_add(dndt, it, Dr);
-            J.template add_row<NS>(it, drdn);
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            if (k >= R.num[1]) break;
+            const int it = R.ind[1][k];
+            w.add(it, Dr);
+            J.template add_row<NS>(it, drdn, drdT);
         }
     }
     // FJ.f90:680-697
+    Basis B;
+    set_coeff<true>(T, logT, B);
+    double vert[NS], vcvr[NS];
     double de = 0.0, cv = 0.0, dcv = 0.0, t1 = 0.0, t2 = 0.0;
 #pragma unroll
     for (int j = 0; j < NS; j++) {
-        t1 = t1 + S.vert[j] * J.get(j, NS);
-        de = de + S.vert[j] * dndt[j];
-        dcv = dcv + S.vcvr[j] * dndt[j];
-        cv = cv + S.vcvr[j] * n[j];
-        t2 = t2 + S.vdcvrdT[j] * n[j];
+        double vdcvrdT;
+        species_energy<true>(m, B, j, T, vert[j], vcvr[j], vdcvrdT);
+        dndt[j] = w.get(j);
+        t1 = t1 + vert[j] * J.get(j, NS);
+        de = de + vert[j] * dndt[j];
+        dcv = dcv + vcvr[j] * dndt[j];
+        cv = cv + vcvr[j] * n[j];
+        t2 = t2 + vdcvrdT * n[j];
     }
     double dTdt = -(de * T / cv);
     dndt[NS] = dTdt;
@@ -538,8 +650,8 @@ SHCFD_HD void jex_impl(const shcfd_mech* m, const double (&n)[NS + 1], Mat& J, d
     for (int j = 0; j < NS; j++) {
         double s = 0.0;
 #pragma unroll
-        for (int k = 0; k < NS; k++) s = s + S.vert[k] * J.get(k, j);
-        J.set(NS, j, -((T * s + dTdt * S.vcvr[j]) / cv));
+        for (int k = 0; k < NS; k++) s = s + vert[k] * J.get(k, j);
+        J.set(NS, j, -((T * s + dTdt * vcvr[j]) / cv));
     }
 }
 
@@ -652,9 +764,9 @@ SHCFD_HD int calc_t(const shcfd_mech* m, const double* vrho, double rho, double 
     // Wilke mixture viscosity (:1600-1633)
     double logT = dlog(T), invT = 1.0 / T;
     double cmu[4] = {logT, invT, invT * invT, 1.0};
-    double muN[NS];
-#pragma unroll
-    for (int i = 0; i < NS; i++) muN[i] = 0.0;
+    SVec<NS> muN, nv;
+    muN.fill(0.0);
+    nv.from(n);
     for (int i = 0; i < m->nt; i++) {
         int s = -1;  // check_section_number_trans, :151-173
         if (m->trange[i][0][0] > T) s = 0;
@@ -665,32 +777,30 @@ SHCFD_HD int calc_t(const shcfd_mech* m, const double* vrho, double rho, double 
             }
         if (s == -1) s = m->nsec_trans[i] - 1;
         double v = 0.0;
-        if (sel_get(n, m->tr2th[i]) > 0.0) {
+        if (nv.at(m->tr2th[i]) > 0.0) {
             double t = 0.0;
 #pragma unroll
             for (int j = 0; j < 4; j++) t = t + cmu[j] * m->trans[i][s][j];
             v = dexp(t);
         }
-#pragma unroll
-        for (int q = 0; q < NS; q++)
-            if (q == i) muN[q] = v;
+        muN.put(i, v);
     }
     double mu = 0.0;
     for (int i = 0; i < m->nt; i++) {
-        double mui = sel_get(muN, i);
+        double mui = muN.at(i);
         if (mui > 0.0) {
             int it = m->tr2th[i];
             double denom = 0.0;
             for (int j = 0; j < m->nt; j++) {
-                double muj = sel_get(muN, j);
+                double muj = muN.at(j);
                 if (muj > 0.0) {
                     int jt = m->tr2th[j];
                     double x = 1.0 + dsqrt(mui / muj) * dsqrt(dsqrt(m->mw[jt] / m->mw[it]));
                     double phi = 0.25 * (x * x) * dsqrt(2.0 * m->mw[jt] / (m->mw[it] + m->mw[jt]));
-                    denom = denom + sel_get(n, jt) * phi;
+                    denom = denom + nv.at(jt) * phi;
                 }
             }
-            mu = mu + sel_get(n, it) * mui / denom;
+            mu = mu + nv.at(it) * mui / denom;
         }
     }
     out.mu = mu * 1e-7;
@@ -1008,12 +1118,27 @@ __device__ int lu_solve_lds(LdsMat<N>& A, double (&b)[N]) {
         for (int i = k + 1; i < N; i++) col[i] = t * col[i];
 #pragma unroll
         for (int i = k; i < N; i++) A.set(i, k, col[i]);
-        for (int j = k + 1; j < N; j++) {
-            const double tj = A.get(l, j);
-            if (l != k) A.set(l, j, A.get(k, j));
-            A.set(k, j, tj);
+        for (int j = k + 1; j < LdsMat<N>::NL; j++) {
+            const double tj = A.at(l, j);
+            if (l != k) A.at(l, j) = A.at(k, j);
+            A.at(k, j) = tj;
 #pragma unroll
-            for (int i = k + 1; i < N; i++) A.set(i, j, A.get(i, j) + tj * col[i]);
+            for (int i = k + 1; i < N; i++) A.at(i, j) = A.at(i, j) + tj * col[i];
+        }
+#pragma unroll
+        for (int q = 0; q < 2; q++) {
+            if (LdsMat<N>::NL + q <= k) continue;
+            const double a0 = A.c[q].get(k);
+            double tj = a0;
+#pragma unroll
+            for (int i = k + 1; i < N; i++) {
+                const double ai = A.c[q].get(i);
+                tj = i == l ? ai : tj;
+                A.c[q].set(i, i == l ? a0 : ai);
+            }
+            A.c[q].set(k, tj);
+#pragma unroll
+            for (int i = k + 1; i < N; i++) A.c[q].set(i, A.c[q].get(i) + tj * col[i]);
         }
     }
     piv[N - 1] = N - 1;
@@ -1022,13 +1147,15 @@ __device__ int lu_solve_lds(LdsMat<N>& A, double (&b)[N]) {
 #pragma unroll
     for (int k = 0; k < N - 1; k++) {
         const int l = piv[k];
-        double t = b[k];
+        // selects of values: an element chosen by address puts b in scratch
+        const double b0 = b[k];
+        double t = b0;
 #pragma unroll
-        for (int i = k + 1; i < N; i++)
-            if (i == l) t = b[i];
-#pragma unroll
-        for (int i = k + 1; i < N; i++)
-            if (i == l) b[i] = b[k];
+        for (int i = k + 1; i < N; i++) {
+            const double bi = b[i];
+            t = i == l ? bi : t;
+            b[i] = i == l ? b0 : bi;
+        }
         b[k] = t;
 #pragma unroll
         for (int i = k + 1; i < N; i++) b[i] = b[i] + t * A.get(i, k);
@@ -1050,7 +1177,8 @@ template <int NS>
 __device__ int point_implicit_lds(const shcfd_mech* m, double T, double (&vrho)[NS], double dt, int& iters,
                                   double& T_out, double* Jl) {
     constexpr int N = NS + 1;
-    LdsMat<N> J{Jl};
+    LdsMat<N> J;
+    J.p = Jl;
     double y0[N], y[N];
 #pragma unroll
     for (int j = 0; j < NS; j++) {
@@ -1074,10 +1202,13 @@ __device__ int point_implicit_lds(const shcfd_mech* m, double T, double (&vrho)[
         it = it + 1;
         double f[N];
         jex_impl<NS>(m, y, J, f);  // F(y) beside J, as in point_implicit
-        for (int a = 0; a < N; a++) {
-            for (int b = 0; b < N; b++) J.set(a, b, -(dt * J.get(a, b)));
-            J.set(a, a, J.get(a, a) + 1.0);
-        }
+#pragma unroll
+        for (int a = 0; a < N; a++)
+#pragma unroll
+            for (int b = 0; b < N; b++) {
+                const double e = -(dt * J.get(a, b));
+                J.set(a, b, a == b ? e + 1.0 : e);
+            }
 #pragma unroll
         for (int a = 0; a < N; a++) f[a] = (y0[a] - y[a]) + dt * f[a];
         if (lu_solve_lds<N>(J, f) != 0) {

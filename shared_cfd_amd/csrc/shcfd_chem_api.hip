@@ -37,7 +37,7 @@ int row_out(int op, int ns) {
 template <int NS>
 void launch0d(int op, const shcfd_mech* dm, int n, const double* din, int ldi, double* dout, int ldo, int* dst,
               double dt) {
-    dim3 g((unsigned)((n + 255) / 256)), b(256);
+    dim3 g((unsigned)((n + 63) / 64)), b(64);
     switch (op) {
     case SHCFD_CHEM_FEX: hipLaunchKernelGGL((k_chem0d<NS, CHEM_OP_FEX>), g, b, 0, 0, dm, n, din, ldi, dout, ldo, dst, dt); break;
     case SHCFD_CHEM_FEXVAR: hipLaunchKernelGGL((k_chem0d<NS, CHEM_OP_FEXVAR>), g, b, 0, 0, dm, n, din, ldi, dout, ldo, dst, dt); break;

@@ -732,12 +732,14 @@ struct ColMat {
     SHCFD_HD double get(int a, int b) const { return p[a + N * b]; }
     SHCFD_HD void set(int a, int b, double v) { p[a + N * b] = v; }
     template <int NR>
-    SHCFD_HD void sub_row(int it, const double (&v)[N]) {
-        for (int b = 0; b < N; b++) p[it + N * b] = p[it + N * b] - v[b];
+    SHCFD_HD void sub_row(int it, const SVec<NR>& v, double vT) {
+#pragma unroll
+        for (int b = 0; b < N; b++) p[it + N * b] = p[it + N * b] - (b < NR ? v.get(b < NR ? b : 0) : vT);
     }
     template <int NR>
-    SHCFD_HD void add_row(int it, const double (&v)[N]) {
-        for (int b = 0; b < N; b++) p[it + N * b] = p[it + N * b] + v[b];
+    SHCFD_HD void add_row(int it, const SVec<NR>& v, double vT) {
+#pragma unroll
+        for (int b = 0; b < N; b++) p[it + N * b] = p[it + N * b] + (b < NR ? v.get(b < NR ? b : 0) : vT);
     }
 };
 

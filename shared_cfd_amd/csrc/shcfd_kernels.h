@@ -29,9 +29,10 @@
 #endif
 #define SHCFD_FOR_EACH_NS(X) SHCFD_FOR_EACH_NY(X)
 #define SHCFD_FOR_EACH_FLOW_NS(X) SHCFD_FOR_EACH_NY(X)
-// the point-implicit flow kernel keeps each lane's (NS+1)^2 Newton matrix in
-// LDS up to this species count (64 lanes x 121 doubles = 62 KB); above it the
-// register kernel runs
+// the point-implicit kernels keep each lane's (NS+1)^2 Newton matrix, but for
+// two columns, in LDS up to this species count (64 lanes x 99 doubles = 51 KB,
+// three waves per CU; 11 species would leave two); above it the register
+// kernel runs
 #define SHCFD_LDS_NEWTON_MAX_NS 10
 
 namespace shcfd {

@@ -1,0 +1,45 @@
+"""The chemistry kernels over species counts around the lines of their rules:
+the vector widths 8 and 16 of the run-time indexed species vectors, and the
+Newton matrix in LDS up to ten species, in registers above; each with row
+counts around one wavefront.
+
+The kernels evaluate the oracle's expressions in the oracle's order with the
+same exp and log, so the bound is that of tests/test_gpu_chem.py (1e-13, for
+results that pass through no other convergence test than the oracle's own).
+"""
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+from oracle.chem_inp import read_cheminp
+from shared_cfd_amd import chem
+
+from chem_cases import NO27, mixture_states, no27_plus_inert, random_states
+
+pytestmark = pytest.mark.gpu
+
+
+def _rel(a, b):
+    a, b = np.asarray(a), np.asarray(b)
+    return float(np.max(np.abs(a - b) / (np.abs(b) + 1e-300 + 1e-14 * np.max(np.abs(b)))))
+
+
+@pytest.mark.parametrize("inert,rows", [(0, 1), (0, 65), (1, 63), (2, 65), (3, 64), (4, 65), (8, 65)])
+def test_rates_jacobian_and_point_implicit(tmp_path, inert, rows):
+    p = NO27 if inert == 0 else no27_plus_inert(str(tmp_path), inert)[0]
+    lm, om = chem.parse(p), read_cheminp(p, chem.MW_INP)
+    ns = 8 + inert
+    assert lm.ns == om.ns == ns
+    y = random_states(om, rows, seed=inert + rows)
+    f, _ = chem.chem_eval(lm, chem.FEX, y)
+    J, _ = chem.chem_eval(lm, chem.JEX, y)
+    for s in range(0, rows, 9):
+        assert _rel(f[s], O.chem_fex(om, y[s])) <= 1e-13
+        assert _rel(J[s].reshape(ns + 1, ns + 1, order="F"), O.chem_jex(om, y[s])) <= 1e-13
+    states = mixture_states(om, rows, seed=inert)
+    out, st = chem.chem_eval(lm, chem.POINT_IMPLICIT, np.array([np.append(v, T) for v, _, _, T in states]), dt=1e-7)
+    for s, (v, _, _, T) in enumerate(states):
+        e, v1, it, T1 = O.chem_point_implicit(om, T, v, 1e-7)
+        assert st[s] == (-e if e else it)
+        if e == 0:
+            assert _rel(out[s, :ns], v1) <= 1e-13 and _rel(out[s, ns:], [T1]) <= 1e-13
