@@ -311,50 +311,52 @@ __device__ inline MusclD muscl_derivs(double wm, double w0, double w1, double w2
     return m;
 }
 
+// One thread per cell and variable (blockIdx.z): a thread's eight faces are a
+// long chain of dependent limiter derivatives and a line of cells too few
+// waves to cover it; with the variables in one thread's loop 80 us on 96 x 24
+// and 27 us on 512 x 128, now 13 and 10.5 us.
 __global__ void __launch_bounds__(128) k_adj_muscl(DevCtx d, AdjView a, int b) {
     const DevBlock B = d.blk[b];
     const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x) - 1;
-    const int j = (int)blockIdx.y - 1;
+    const int j = (int)blockIdx.y - 1, k = (int)blockIdx.z;
     if (i > B.ni + 2 || j > B.nj + 2) return;
     const long long c = cidx(B, i, j), P = B.pitch;
     const bool row = j >= 1 && j <= B.nj, col = i >= 1 && i <= B.ni;
-    for (int k = 0; k < D1::dw; k++) {
-        const double* W = d.f[SHCFD_F_W] + (long long)k * d.NC;
-        double s = 0.0;
-        if (row) {
-            // faces f = i-2 .. i+1 of row j (f in [0, ni])
-            for (int f = i - 2; f <= i + 1; f++) {
-                if (f < 0 || f > B.ni) continue;
-                const long long cf = cidx(B, f, j);
-                const MusclD m = muscl_derivs(W[cf - 1], W[cf], W[cf + 1], W[cf + 2], d);
-                const double bl = a.face[AdjView::WLI][k * d.NC + cf], br = a.face[AdjView::WRI][k * d.NC + cf];
-                const int o = i - f;  // position of this cell relative to f
-                if (o >= -1 && o <= 1) s += bl * m.l[o + 1];
-                if (o >= 0 && o <= 2) s += br * m.r[o];
-            }
+    const double* W = d.f[SHCFD_F_W] + (long long)k * d.NC;
+    double s = 0.0;
+    if (row) {
+        // faces f = i-2 .. i+1 of row j (f in [0, ni])
+        for (int f = i - 2; f <= i + 1; f++) {
+            if (f < 0 || f > B.ni) continue;
+            const long long cf = cidx(B, f, j);
+            const MusclD m = muscl_derivs(W[cf - 1], W[cf], W[cf + 1], W[cf + 2], d);
+            const double bl = a.face[AdjView::WLI][k * d.NC + cf], br = a.face[AdjView::WRI][k * d.NC + cf];
+            const int o = i - f;  // position of this cell relative to f
+            if (o >= -1 && o <= 1) s += bl * m.l[o + 1];
+            if (o >= 0 && o <= 2) s += br * m.r[o];
         }
-        if (col) {
-            for (int f = j - 2; f <= j + 1; f++) {
-                if (f < 0 || f > B.nj) continue;
-                const long long cf = cidx(B, i, f);
-                const MusclD m = muscl_derivs(W[cf - P], W[cf], W[cf + P], W[cf + 2 * P], d);
-                const double bl = a.face[AdjView::WLJ][k * d.NC + cf], br = a.face[AdjView::WRJ][k * d.NC + cf];
-                const int o = j - f;
-                if (o >= -1 && o <= 1) s += bl * m.l[o + 1];
-                if (o >= 0 && o <= 2) s += br * m.r[o];
-            }
-        }
-        if (d.p.viscous && i >= 0 && i <= B.ni + 1 && j >= 0 && j <= B.nj + 1 && vw_slot(k) >= 0)
-            s += viscous_gather(d, B, a.vw_i, a.vw_j, NVW, vw_slot(k), i, j);
-        a.wbar[k * d.NC + c] = s;
     }
+    if (col) {
+        for (int f = j - 2; f <= j + 1; f++) {
+            if (f < 0 || f > B.nj) continue;
+            const long long cf = cidx(B, i, f);
+            const MusclD m = muscl_derivs(W[cf - P], W[cf], W[cf + P], W[cf + 2 * P], d);
+            const double bl = a.face[AdjView::WLJ][k * d.NC + cf], br = a.face[AdjView::WRJ][k * d.NC + cf];
+            const int o = j - f;
+            if (o >= -1 && o <= 1) s += bl * m.l[o + 1];
+            if (o >= 0 && o <= 2) s += br * m.r[o];
+        }
+    }
+    if (d.p.viscous && i >= 0 && i <= B.ni + 1 && j >= 0 && j <= B.nj + 1 && vw_slot(k) >= 0)
+        s += viscous_gather(d, B, a.vw_i, a.vw_j, NVW, vw_slot(k), i, j);
+    a.wbar[k * d.NC + c] = s;
 }
 
 // corner ghosts (set_corners, cond/no-nV/condition.tail.f90:331-356: the
 // mean of the corner cell and its two side ghosts), reversed before the
-// side rows; one thread per block
+// side rows; one thread per block and variable
 __global__ void k_adj_bc_corner(DevCtx d, AdjView a) {
-    const int b = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+    const int t = (int)(blockIdx.x * blockDim.x + threadIdx.x), b = t / D1::dw, k = t % D1::dw;
     if (b >= d.nb) return;
     const DevBlock B = d.blk[b];
     for (int q = 0; q < 4; q++) {
@@ -362,13 +364,11 @@ __global__ void k_adj_bc_corner(DevCtx d, AdjView a) {
         const int i = pi < 0 ? 1 : B.ni, j = pj < 0 ? 1 : B.nj;
         const long long cc = cidx(B, i + pi, j + pj), c0 = cidx(B, i, j), cj = cidx(B, i, j + pj),
                         ci = cidx(B, i + pi, j);
-        for (int k = 0; k < D1::dw; k++) {
-            const double x = a.wbar[k * d.NC + cc] * (1.0 / 3.0);
-            a.wbar[k * d.NC + cc] = 0.0;
-            a.wbar[k * d.NC + c0] += x;
-            a.wbar[k * d.NC + cj] += x;
-            a.wbar[k * d.NC + ci] += x;
-        }
+        const double x = a.wbar[k * d.NC + cc] * (1.0 / 3.0);
+        a.wbar[k * d.NC + cc] = 0.0;
+        a.wbar[k * d.NC + c0] += x;
+        a.wbar[k * d.NC + cj] += x;
+        a.wbar[k * d.NC + ci] += x;
     }
 }
 
@@ -410,13 +410,12 @@ __global__ void k_adj_ghost_centres(DevCtx d, AdjView a, int b, int pass) {
 }
 
 // ---------------------------------------------------------------------------
-// boundary rows: ghost bars -> source cells (one launch per row, one thread
-// per position along the side, one workgroup so the fixed-state sums reduce
-// in a fixed order)
+// boundary rows: ghost bars -> source cells (one thread per position along the
+// side, one workgroup so the fixed-state sums reduce in a fixed order)
 // ---------------------------------------------------------------------------
-// one side row, by all threads of the workgroup (red: 256 doubles of LDS)
+// one side row, by all threads of the workgroup (red: LDS)
 __device__ inline void adj_bc_row(const DevCtx& d, AdjView& a, const int* row, const double* pool, double* poolbar,
-                                  double* red) {
+                                  double (&red)[D1::dw][ADJ_BC_THREADS]) {
     const int b = row[0] - 1, side = row[1], kind = row[4], off = row[5];
     const DevBlock B = d.blk[b];
     const int n = (side <= SHCFD_SIDE_IMAX) ? B.nj : B.ni;
@@ -433,10 +432,14 @@ __device__ inline void adj_bc_row(const DevCtx& d, AdjView& a, const int* row, c
         default: ii = tpos; jj = B.nj; ig1 = tpos; jg1 = B.nj + 1; ig2 = tpos; jg2 = B.nj + 2; break;
         }
         const long long ci = cidx(B, ii, jj), c1 = cidx(B, ig1, jg1), c2 = cidx(B, ig2, jg2);
-        double gb[D1::dw];
+        double gb[D1::dw], wi[D1::dw];  // all loads before the first store: one round trip
 #pragma unroll
         for (int k = 0; k < D1::dw; k++) {
             gb[k] = a.wbar[k * d.NC + c1] + a.wbar[k * d.NC + c2];
+            wi[k] = a.wbar[k * d.NC + ci];
+        }
+#pragma unroll
+        for (int k = 0; k < D1::dw; k++) {
             a.wbar[k * d.NC + c1] = 0.0;
             a.wbar[k * d.NC + c2] = 0.0;
         }
@@ -486,19 +489,24 @@ __device__ inline void adj_bc_row(const DevCtx& d, AdjView& a, const int* row, c
             nbar[d.NC + cf] += -2.0 * (bn * v + un * vb);
         }
 #pragma unroll
-        for (int k = 0; k < D1::dw; k++) a.wbar[k * d.NC + ci] += gb[k];
+        for (int k = 0; k < D1::dw; k++) a.wbar[k * d.NC + ci] = wi[k] + gb[k];
     }
     if (kind != SHCFD_BC_FIXED && kind != SHCFD_BC_INFLOW_TUV) return;
     const int npv = kind == SHCFD_BC_FIXED ? D1::dw : 3;  // pool entries with bars
-    for (int k = 0; k < npv; k++) {
-        red[threadIdx.x] = pacc[k];
-        __syncthreads();
-        for (int w = blockDim.x / 2; w > 0; w >>= 1) {
-            if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-            __syncthreads();
-        }
-        if (threadIdx.x == 0) poolbar[off + k] += red[0];
-        __syncthreads();
+#pragma unroll
+    for (int k = 0; k < D1::dw; k++)
+        if (k < npv) red[k][threadIdx.x] = pacc[k];
+    __syncthreads();
+    // wave w sums entries w, w + 8, ...: a lane its columns of the row, then
+    // the lanes in a tree
+    const int L = (int)threadIdx.x & 63;
+    for (int k = (int)threadIdx.x >> 6; k < npv; k += ADJ_BC_THREADS / 64) {
+        double x = 0.0;
+#pragma unroll
+        for (int m = 0; m < ADJ_BC_THREADS; m += 64) x += red[k][m + L];
+#pragma unroll
+        for (int w = 32; w > 0; w >>= 1) x += __shfl_xor(x, w);
+        if (L == 0) poolbar[off + k] += x;
     }
 }
 
@@ -510,9 +518,12 @@ __device__ inline void adj_cut_row(const DevCtx& d, AdjView& a, const int* t) {
             int bd, di, dj, bs, si, sj;
             if (!cut_map(t, inc, copy, bd, di, dj, bs, si, sj)) break;
             const long long g = cidx(d.blk[bd], di, dj), src = cidx(d.blk[bs], si, sj);
+            double x[D1::dw];  // all loads before the first store, as in adj_bc_row
+#pragma unroll
+            for (int k = 0; k < D1::dw; k++) x[k] = a.wbar[k * d.NC + src] + a.wbar[k * d.NC + g];
 #pragma unroll
             for (int k = 0; k < D1::dw; k++) {
-                a.wbar[k * d.NC + src] += a.wbar[k * d.NC + g];
+                a.wbar[k * d.NC + src] = x[k];
                 a.wbar[k * d.NC + g] = 0.0;
             }
         }
@@ -522,9 +533,15 @@ __device__ inline void adj_cut_row(const DevCtx& d, AdjView& a, const int* t) {
 // the forward fill: the side rows, last row first, then the cut rows, last
 // first.  Rows that meet at a block corner add into the same interior cell,
 // so each row starts after a barrier.  The pool bars are cleared first.
-__global__ void __launch_bounds__(256) k_adj_bc_rows(DevCtx d, AdjView a, const int* bc, int nbc, const double* pool,
+//
+// Bound by memory latency, row after row: a row is one round trip per 512
+// positions, where a position's loads all precede its stores, and one barrier
+// for the pool sums of all variables.  With 256 threads, the interior bars
+// loaded after the ghosts' and a tree of barriers per variable 46 us on
+// 512 x 128 and 28 us on 96 x 24, now 22 and 11.
+__global__ void __launch_bounds__(ADJ_BC_THREADS) k_adj_bc_rows(DevCtx d, AdjView a, const int* bc, int nbc, const double* pool,
                                                      double* poolbar, int npool, const int* cut, int ncut) {
-    __shared__ double red[256];
+    __shared__ double red[D1::dw][ADJ_BC_THREADS];
     for (int k = (int)threadIdx.x; k < npool; k += (int)blockDim.x) poolbar[k] = 0.0;
     __syncthreads();
     for (int r = nbc - 1; r >= 0; r--) {

@@ -5,6 +5,8 @@
 
 namespace shcfd {
 
+constexpr int ADJ_BC_THREADS = 512;  // workgroup of the reverse boundary rows
+
 // Arrays indexed like the cell fields (component k of cell c at k*NC + c);
 // face arrays are stored at the index of the face's left/lower cell, node
 // arrays at the index of the node.

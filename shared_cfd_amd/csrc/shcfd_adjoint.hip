@@ -215,14 +215,14 @@ void vjp_async(shcfd_ctx* ctx, bool metrics = true) {
     }
     for (int b = 0; b < ctx->nb; b++) {
         const DevBlock& B = ctx->hblk[b];
-        hipLaunchKernelGGL(k_adj_muscl, dim3((unsigned)((B.ni + 4 + 127) / 128), (unsigned)(B.nj + 4)), dim3(128), 0, st,
-                           d, a, b);
+        hipLaunchKernelGGL(k_adj_muscl, dim3((unsigned)((B.ni + 4 + 127) / 128), (unsigned)(B.nj + 4), Dims<1>::dw),
+                           dim3(128), 0, st, d, a, b);
     }
     // reverse of the forward fill order: corners (read by the viscous
     // fluxes only), then side rows and cut rows in one workgroup (which
     // clears the pool bars first)
-    if (vis) hipLaunchKernelGGL(k_adj_bc_corner, dim3((unsigned)((ctx->nb + 63) / 64)), dim3(64), 0, st, d, a);
-    hipLaunchKernelGGL(k_adj_bc_rows, dim3(1), dim3(256), 0, st, d, a, ctx->dbc, ctx->nbc, ctx->dpool,
+    if (vis) hipLaunchKernelGGL(k_adj_bc_corner, dim3((unsigned)((ctx->nb * Dims<1>::dw + 63) / 64)), dim3(64), 0, st, d, a);
+    hipLaunchKernelGGL(k_adj_bc_rows, dim3(1), dim3(ADJ_BC_THREADS), 0, st, d, a, ctx->dbc, ctx->nbc, ctx->dpool,
                        ctx->adj->poolbar, ctx->npool > 0 ? ctx->npool : 1, ctx->dcut, ctx->ncut);
     for (int b = 0; b < ctx->nb; b++) {
         const DevBlock& B = ctx->hblk[b];
