@@ -114,10 +114,17 @@ __global__ void __launch_bounds__(256) k_primitive_ideal(DevCtx d, const Tile* t
 template <int NY>
 __device__ inline void copy_wv(const DevCtx& d, long long dst, long long src) {
     using D = Dims<NY>;
+    // all loads before the first store: a load behind a store that may alias
+    // it waits for the loads before that store, one round trip per component
+    double wv[D::dw], vh[NY];
 #pragma unroll
-    for (int k = 0; k < D::dw; k++) FLD(d, SHCFD_F_W, k, dst) = FLD(d, SHCFD_F_W, k, src);
+    for (int k = 0; k < D::dw; k++) wv[k] = FLD(d, SHCFD_F_W, k, src);
 #pragma unroll
-    for (int k = 0; k < NY; k++) FLD(d, SHCFD_F_VHI, k, dst) = FLD(d, SHCFD_F_VHI, k, src);
+    for (int k = 0; k < NY; k++) vh[k] = FLD(d, SHCFD_F_VHI, k, src);
+#pragma unroll
+    for (int k = 0; k < D::dw; k++) FLD(d, SHCFD_F_W, k, dst) = wv[k];
+#pragma unroll
+    for (int k = 0; k < NY; k++) FLD(d, SHCFD_F_VHI, k, dst) = vh[k];
 }
 
 // section_exchange: cond/no-nV/condition.tail.f90:2-70.  One thread per
@@ -197,9 +204,12 @@ __global__ void k_bc_side(DevCtx d, const int* bc, int nbc, const double* pool, 
         const double pin = FLD(d, SHCFD_F_W, IW_P, ci);
         wv[IW_RHO] = (pin * pv[D::dw + NY]) / pv[D::dw + NY + 1];
         if (kind == SHCFD_BC_INJECT_WALL) {
-            const int kn = (side <= SHCFD_SIDE_IMAX) ? IW_U : IW_V, kt = (side <= SHCFD_SIDE_IMAX) ? IW_V : IW_U;
-            wv[kt] = -FLD(d, SHCFD_F_W, kt, ci);
-            wv[kn] = (pv[D::dw + NY + 2] * 2.0) - FLD(d, SHCFD_F_W, kn, ci);
+            // no run-time index into wv, here and below: it would put wv in scratch
+            const double u = FLD(d, SHCFD_F_W, IW_U, ci), v = FLD(d, SHCFD_F_W, IW_V, ci);
+            const double vn = pv[D::dw + NY + 2] * 2.0;
+            const bool iside = side <= SHCFD_SIDE_IMAX;
+            wv[IW_U] = iside ? vn - u : -u;
+            wv[IW_V] = iside ? -v : vn - v;
         }
         wv[IW_P] = pin;
         wv[D::ih] = pv[D::ih] + 0.5 * ((wv[IW_U] * wv[IW_U]) + (wv[IW_V] * wv[IW_V]));
@@ -211,8 +221,9 @@ __global__ void k_bc_side(DevCtx d, const int* bc, int nbc, const double* pool, 
 #pragma unroll
         for (int k = 0; k < NY; k++) vh[k] = FLD(d, SHCFD_F_VHI, k, ci);
         if (kind == SHCFD_BC_REFLECT) {
-            int kv = (side <= SHCFD_SIDE_IMAX) ? IW_U : IW_V;
-            wv[kv] = -wv[kv];
+            const bool iside = side <= SHCFD_SIDE_IMAX;
+            wv[IW_U] = iside ? -wv[IW_U] : wv[IW_U];
+            wv[IW_V] = iside ? wv[IW_V] : -wv[IW_V];
         } else if (kind == SHCFD_BC_NOSLIP) {
             wv[IW_U] = -wv[IW_U];
             wv[IW_V] = -wv[IW_V];
@@ -250,13 +261,17 @@ __device__ inline void bc_corner_cell(const DevCtx& d, int gid) {
     int pi = (gid & 1) ? 1 : -1, pj = (gid & 2) ? 1 : -1;
     int i = (pi < 0) ? 1 : B.ni, j = (pj < 0) ? 1 : B.nj;
     long long cc = cidx(B, i + pi, j + pj), c0 = cidx(B, i, j), cj = cidx(B, i, j + pj), ci = cidx(B, i + pi, j);
+    double wv[D::dw], vh[NY];  // all loads before the first store, as in copy_wv
 #pragma unroll
     for (int k = 0; k < D::dw; k++)
-        FLD(d, SHCFD_F_W, k, cc) = (1.0 / 3.0) * ((FLD(d, SHCFD_F_W, k, c0) + FLD(d, SHCFD_F_W, k, cj)) + FLD(d, SHCFD_F_W, k, ci));
+        wv[k] = (1.0 / 3.0) * ((FLD(d, SHCFD_F_W, k, c0) + FLD(d, SHCFD_F_W, k, cj)) + FLD(d, SHCFD_F_W, k, ci));
 #pragma unroll
     for (int k = 0; k < NY; k++)
-        FLD(d, SHCFD_F_VHI, k, cc) =
-            (1.0 / 3.0) * ((FLD(d, SHCFD_F_VHI, k, c0) + FLD(d, SHCFD_F_VHI, k, cj)) + FLD(d, SHCFD_F_VHI, k, ci));
+        vh[k] = (1.0 / 3.0) * ((FLD(d, SHCFD_F_VHI, k, c0) + FLD(d, SHCFD_F_VHI, k, cj)) + FLD(d, SHCFD_F_VHI, k, ci));
+#pragma unroll
+    for (int k = 0; k < D::dw; k++) FLD(d, SHCFD_F_W, k, cc) = wv[k];
+#pragma unroll
+    for (int k = 0; k < NY; k++) FLD(d, SHCFD_F_VHI, k, cc) = vh[k];
 }
 template <int NY>
 __global__ void k_bc_corner(DevCtx d) {
