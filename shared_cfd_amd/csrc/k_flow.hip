@@ -577,14 +577,14 @@ __global__ void __launch_bounds__(256) k_set_abpm_skew(DevCtx d, const Strip* st
 
 // set_ABpm writing the quad-row copy of the 16-row sweeps: thread = row r of
 // step t of a strip (16 steps x 16 rows per workgroup); grid = (strips,
-// ceil((max ni + 15)/16))
+// ceil((max ni + JSPAN)/16))
 template <int NY>
 __global__ void __launch_bounds__(256) k_set_abpm16(DevCtx d, const Strip16* strips, double* jac, long long nsl) {
     const Strip16 S = strips[blockIdx.x];
     const int t = (int)blockIdx.y * 16 + (int)(threadIdx.x >> 4), r = (int)(threadIdx.x & 15);
     const DevBlock B = d.blk[S.b];
-    if (t >= B.ni + 15) return;
-    const int i = t - r + 1, j = S.j0 + r;
+    if (t >= B.ni + JSPAN) return;
+    const int i = t - r - JGD * (r >> 2) + 1, j = S.j0 + r;
     if (i < 1 || i > B.ni || j > B.nj) return;
     set_abpm_cell<NY, 3>(d, B, i, j, jac, nsl, 64LL * (S.base + t) + 4 * r);
 }

@@ -4,32 +4,15 @@
 // preconLU-SGS/2d/time_precon_viscous.f90; dual time with its S scaling keeps
 // the row-per-lane sweeps of k_implicit.hip).
 //
-// Layout.  A workgroup owns 16 rows of a block and has C = ceil(dq/4) waves;
-// lane 4r + c of wave w holds component k = 4w + c of row j0 + r, so the
-// 16 x dq unknowns of a strip occupy one lane each.  At step t row r works on
-// column i = t - r + 1 (forward) or i = ni - t + 15 - r (backward):
-//   * the i-neighbour's contribution stays in the lane (same row, previous
-//     column);
-//   * the j-neighbour's contribution comes from row r -/+ 1 of the same wave
-//     by a 4-lane DPP shift, and for the edge row from the neighbouring
-//     strip through a hand-off row: the producer stores each column's value
-//     into a slot that k_fill16 set to a NaN sentinel, the consumer keeps a
-//     ring of PH loads ahead and polls a slot only while it still holds the
-//     sentinel (no flags, so no wave ever waits for its own stores);
-//   * the dq components of x needed by a lane's matrix rows are exchanged
-//     through LDS (double-buffered, one barrier per step).
-// Every lane evaluates the reference's per-cell formula with the same
-// operation order as the row-per-lane sweeps, on the same inputs, in a
-// topological order of the same dependency graph, so the results are
-// identical.  A lane reads its two matrix rows (2 dq doubles) and the cell's
-// alpha, dsci, dscj of each step from the quad-row copy written by
-// k_set_abpm16 as dq + 2 pairs of doubles, pair p of global step g = base + t
-// at ((((set NT + g) C + w) (dq+2) + p) 64 + lane) 2: every 16-byte load of
-// a wave reads 1 KB of consecutive bytes, and one step of a strip is one
-// contiguous block (few pages per step).  Loads run PD steps ahead of their use in
-// straight-line code (the last steps re-read a valid step), so the
-// compiler's memory waits count exactly the loads issued after the one a
-// step consumes.
+// A workgroup owns 16 rows of a block and has C = ceil(dq/4) compute waves: the
+// 16 x dq unknowns of a strip occupy one lane each.  The i-neighbour's
+// contribution stays in the lane, the j-neighbour's comes from the row above or
+// below by a 4-lane DPP shift or, at the edges of the four-row groups, through
+// an LDS ring, and from the neighbouring strip through a hand-off row: the
+// producer stores each column's value into a slot that holds a NaN sentinel, the
+// consumer polls the slots (no flags, so no wave waits for its own stores).
+// Two families: with the products A x in closed form (LU-SGS, NR), and over
+// stored matrices (the preconditioned schemes).
 #include "shcfd_device.h"
 #include "shcfd_kernels.h"
 
@@ -37,45 +20,22 @@ namespace shcfd {
 
 namespace {
 
-constexpr int PD = 3;  // prefetch distance of the operator rows, in steps
-constexpr int PH = 4;  // hand-off loads in flight (PD + 1: one unrolled round)
 constexpr int HO = 24; // hand-off column offset: entry (col + HO) dq + k, col >= -HO
 constexpr unsigned long long SENT16 = 0x7FF4DEADBEEFCAFEULL;  // never produced by arithmetic
 
 __device__ inline bool is_sent16(double x) { return (unsigned long long)__double_as_longlong(x) == SENT16; }
 
-__device__ inline void set_error16(const DevCtx& d, int code) { atomicCAS(d.iflag + IFLAG_ERR, 0, code); }
-
 // workgroup barrier after this wave's LDS writes have completed; global
 // loads in flight are not waited for (the prefetched operator rows)
 __device__ inline void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-// rare path of the hand-off: poll the slot until the lanes `mine` see a
-// value; past the bound raise SHCFD_E_SPIN and go on with zero.  Then wait
-// for the wave's outstanding loads so the common path inherits no partial
-// wait state.
-__device__ inline double poll16(const double* slot, double x, bool mine, long long spin_limit,
-                                                   int* iflag, bool& dead) {
-    long long it = 0;
-    while (!dead && __ballot(mine && is_sent16(x)) != 0ULL) {
-        if (it++ >= spin_limit) {
-            atomicCAS(iflag + IFLAG_ERR, 0, SHCFD_E_SPIN);
-            dead = true;  // no further waits in this sweep: it runs to its end with zeros
-            break;
-        }
-        __builtin_amdgcn_s_sleep(2);
-        x = load_agent(slot);
-    }
-    __builtin_amdgcn_s_waitcnt(0x0F70);
-    return (mine && !dead) ? x : 0.0;
-}
-
-// per-lane inputs of one step: the lane's rows of the two matrices, the
-// cell values of its row and the lane's components of Δq* (and q)
+// per-lane inputs of one step of the sweeps over stored matrices: the lane's
+// rows of the two matrices, the cell values of its row and the lane's
+// component of the right-hand side
 template <int DQ>
 struct StepIn {
     double a[DQ], b[DQ];
-    double al, fi, fj, r, q;
+    double al, fi, fj, r;
 };
 
 // the pair-interleaved operator rows and scalars of one step: `base` is the
@@ -96,224 +56,6 @@ __device__ inline void load_ops(const double* __restrict__ base, StepIn<DQ>& in)
 }
 
 }  // namespace
-
-// hand-off rows of both sweeps: the sentinel for the columns 1..ni of the
-// strip's block, zero elsewhere and in the final row (read by the strips
-// that have no neighbour)
-#if SHCFD_INST_GROUP == 0
-__global__ void __launch_bounds__(256) k_fill16(DevCtx d, const Strip16* strips, int nstrips, double* hand,
-                                                long long hstride, int dq) {
-    const long long n = 2LL * (nstrips + 1) * hstride;
-    const double sv = __longlong_as_double((long long)SENT16);
-    for (long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x; e < n; e += (long long)gridDim.x * blockDim.x) {
-        const int row = (int)((e / hstride) % (nstrips + 1));
-        const long long col = (e % hstride) / dq - HO;
-        const bool live = row < nstrips && col >= 1 && col <= d.blk[strips[row].b].ni;
-        hand[e] = live ? sv : 0.0;
-    }
-}
-#endif
-
-// ---------------------------------------------------------------------------
-// forward sweep: x = alpha (R + A+(i-1) x(i-1) dsci + B+(j-1) x(j-1) dscj)
-// ---------------------------------------------------------------------------
-// one wave per 4 components: up to 4 waves for dq <= 16, 5 above
-template <int NY>
-__global__ void __launch_bounds__(NY + 3 <= 16 ? 256 : 320) __attribute__((amdgpu_waves_per_eu(1, 1)))
-k_sweep16_fwd(DevCtx d, const Strip16* strips, int nstrips, double* hand, long long hstride, long long spin_limit,
-              const double* __restrict__ jac, long long nsl) {
-    constexpr int dq = NY + 3, C = (dq + 3) / 4, DQP = 4 * C;
-    __shared__ double xs[2][16][DQP];
-    const int s = blockIdx.x;
-    const int w = (int)(threadIdx.x >> 6), L = (int)(threadIdx.x & 63), r = L >> 2, k = 4 * w + (L & 3);
-    const Strip16 S = strips[s];
-    const DevBlock B = d.blk[S.b];
-    const int ni = B.ni, nj = B.nj, j = S.j0 + r;
-    const bool rowok = j <= nj, kok = k < dq;
-    const bool has_next = S.next >= 0;
-    const bool mine = r == 0 && kok;  // lanes that take the neighbour strip's value
-    const int nsteps = ni + 15;
-    constexpr int dq2 = dq + 2;
-    // lane's pair 0 of step 0 (set 0); one step = C dq2 64 pairs
-    const double* jl = jac + (((S.base * C + w) * dq2) * 64 + L) * 2;
-    const int kk = kok ? k : 0;
-    const double* hsrc = hand + (long long)(S.prev >= 0 ? S.prev : nstrips) * hstride + (long long)HO * dq + kk;
-    double* hdst = hand + (long long)s * hstride + (long long)HO * dq + kk;
-    double* dqf = d.f[SHCFD_F_DQ] + (long long)kk * d.NC;
-    auto load = [&](int t, StepIn<dq>& in) {
-        t = t < nsteps ? t : nsteps - 1;  // past the end: re-read the last step
-        load_ops<dq>(jl + 128LL * C * dq2 * t, in);
-        const int i = t - r + 1;
-        const int ic = i < 1 ? 1 : (i > ni ? ni : i);
-        in.r = dqf[cidx(B, ic, rowok ? j : nj)];
-    };
-    StepIn<dq> buf[PD + 1];
-    double hr[PH];
-#pragma unroll
-    for (int p = 0; p < PH; p++) hr[p] = load_agent(hsrc + (long long)(p + 1) * dq);  // columns 1..PH
-#pragma unroll
-    for (int p = 0; p < PD; p++) load(p, buf[p]);
-    double a_in = 0.0, bo = 0.0;
-    bool dead = false;
-    const int tend = ((nsteps + PD) / (PD + 1)) * (PD + 1);  // whole rounds; the extra steps are idle
-    for (int t0 = 0; t0 < tend; t0 += PD + 1) {
-#pragma unroll
-        for (int u = 0; u <= PD; u++) {
-            const int t = t0 + u;
-            {
-                // neighbour value of column t + 1; refill the slot with column t + 1 + PH
-                double hv = hr[u];
-                hr[u] = load_agent(hsrc + (long long)(t + 1 + PH) * dq);
-                load(t + PD, buf[(u + PD) % (PD + 1)]);
-                const StepIn<dq>& in = buf[u];
-                const int i = t - r + 1;
-                const bool act = rowok && i >= 1 && i <= ni;
-                double b_in = shift_up4(bo);
-                if (__builtin_expect(__ballot(mine && is_sent16(hv)) != 0ULL, 0))
-                    hv = poll16(hsrc + (long long)(t + 1) * dq, hv, mine, spin_limit, d.iflag, dead);
-                if (r == 0) b_in = kok ? hv : 0.0;
-                double x = 0.0;
-                if (act && kok) {
-                    x = in.al * (in.r + (a_in + b_in));
-                    dqf[cidx(B, i, j)] = x;
-                }
-                xs[t & 1][r][k] = x;
-                lds_barrier();
-                double xa[dq];
-#pragma unroll
-                for (int l = 0; l < dq; l++) xa[l] = xs[t & 1][r][l];
-                if (act) {
-                    double sa = 0.0, sb = 0.0;
-#pragma unroll
-                    for (int l = 0; l < dq; l++) sa = sa + in.a[l] * xa[l];
-#pragma unroll
-                    for (int l = 0; l < dq; l++) sb = sb + in.b[l] * xa[l];
-                    a_in = in.fi * sa;
-                    bo = in.fj * sb;
-                } else {
-                    bo = 0.0;
-                }
-                if (has_next && r == 15 && act && kok) store_agent(hdst + (long long)i * dq, bo);
-            }
-        }
-    }
-}
-
-// ---------------------------------------------------------------------------
-// backward sweep: x = x* - alpha (A-(i+1) x(i+1) dsci + B-(j+1) x(j+1) dscj),
-// then q += x (LU-SGS, preconLU-SGS) or the (res, omega) partials of the
-// inner-loop schemes.  Workgroup g handles strip nstrips-1-g, so the strip
-// it waits on (the one above) has a lower workgroup id.
-// ---------------------------------------------------------------------------
-template <int NY>
-__global__ void __launch_bounds__(NY + 3 <= 16 ? 256 : 320) __attribute__((amdgpu_waves_per_eu(1, 1)))
-k_sweep16_bwd(DevCtx d, const Strip16* strips, int nstrips, double* hand, long long hstride, double* part,
-              long long spin_limit, const double* __restrict__ jac, long long nsl) {
-    constexpr int dq = NY + 3, C = (dq + 3) / 4, DQP = 4 * C;
-    __shared__ double xs[2][16][DQP];
-    __shared__ double red[2][4];
-    const int s = nstrips - 1 - (int)blockIdx.x;
-    const int w = (int)(threadIdx.x >> 6), L = (int)(threadIdx.x & 63), r = L >> 2, k = 4 * w + (L & 3);
-    const Strip16 S = strips[s];
-    const DevBlock B = d.blk[S.b];
-    const int ni = B.ni, nj = B.nj, j = S.j0 + r;
-    const bool rowok = j <= nj, kok = k < dq;
-    const bool has_prev = S.prev >= 0;
-    const bool mine = r == 15 && kok;
-    const bool inner = inner_loop_scheme(d.p.scheme);
-    const double dqmax = d.p.dqmax;
-    const int nsteps = ni + 15;
-    constexpr int dq2 = dq + 2;
-    // lane's pair 0 of step 0 of set 1 (nsl = total steps of all strips)
-    const double* jl = jac + ((((nsl + S.base) * C + w) * dq2) * 64 + L) * 2;
-    const int kk = kok ? k : 0;
-    const double* hsrc = hand + (long long)(S.next >= 0 ? S.next : nstrips) * hstride + (long long)HO * dq + kk;
-    double* hdst = hand + (long long)s * hstride + (long long)HO * dq + kk;
-    double* dqf = d.f[SHCFD_F_DQ] + (long long)kk * d.NC;
-    double* qf = d.f[SHCFD_F_Q] + (long long)kk * d.NC;
-    auto load = [&](int t, StepIn<dq>& in) {
-        t = t < nsteps ? t : nsteps - 1;  // past the end: re-read the last step
-        // cell (i, j0+r) sits at forward step i + r - 1 = ni + 14 - t
-        load_ops<dq>(jl + 128LL * C * dq2 * (ni + 14 - t), in);
-        const int i = ni - t + 15 - r;
-        const int ic = i < 1 ? 1 : (i > ni ? ni : i);
-        const long long c = cidx(B, ic, rowok ? j : nj);
-        in.r = dqf[c];
-        in.q = qf[c];
-    };
-    StepIn<dq> buf[PD + 1];
-    double hr[PH];
-#pragma unroll
-    for (int p = 0; p < PH; p++) hr[p] = load_agent(hsrc + (long long)(ni - p) * dq);  // columns ni..ni-PH+1
-#pragma unroll
-    for (int p = 0; p < PD; p++) load(p, buf[p]);
-    double a_in = 0.0, bo = 0.0, res = 0.0, omega = 1e300;
-    bool dead = false;
-    const int tend = ((nsteps + PD) / (PD + 1)) * (PD + 1);  // whole rounds; the extra steps are idle
-    for (int t0 = 0; t0 < tend; t0 += PD + 1) {
-#pragma unroll
-        for (int u = 0; u <= PD; u++) {
-            const int t = t0 + u;
-            {
-                // neighbour value of column ni - t (row 15); refill with column ni - t - PH
-                double hv = hr[u];
-                hr[u] = load_agent(hsrc + (long long)(ni - t - PH) * dq);
-                load(t + PD, buf[(u + PD) % (PD + 1)]);
-                const StepIn<dq>& in = buf[u];
-                const int i = ni - t + 15 - r;
-                const bool act = rowok && i >= 1 && i <= ni;
-                double b_in = shift_down4(bo);
-                if (__builtin_expect(__ballot(mine && is_sent16(hv)) != 0ULL, 0))
-                    hv = poll16(hsrc + (long long)(ni - t) * dq, hv, mine, spin_limit, d.iflag, dead);
-                if (r == 15) b_in = kok ? hv : 0.0;
-                double x = 0.0;
-                if (act && kok) {
-                    const long long c = cidx(B, i, j);
-                    x = in.r - in.al * (a_in + b_in);
-                    if (inner) {
-                        if (k == NY + 2) res = res + x * x;
-                        if (k < NY && x < 0.0) omega = dmin(omega, (-in.q / x) * dqmax);
-                    } else if (B.active) {
-                        qf[c] = in.q + x;
-                    }
-                    dqf[c] = x;
-                }
-                xs[t & 1][r][k] = x;
-                lds_barrier();
-                double xa[dq];
-#pragma unroll
-                for (int l = 0; l < dq; l++) xa[l] = xs[t & 1][r][l];
-                if (act) {
-                    double sa = 0.0, sb = 0.0;
-#pragma unroll
-                    for (int l = 0; l < dq; l++) sa = sa + in.a[l] * xa[l];
-#pragma unroll
-                    for (int l = 0; l < dq; l++) sb = sb + in.b[l] * xa[l];
-                    a_in = in.fi * sa;
-                    bo = in.fj * sb;
-                } else {
-                    bo = 0.0;
-                }
-                if (has_prev && r == 0 && act && kok) store_agent(hdst + (long long)i * dq, bo);
-            }
-        }
-    }
-    if (inner) {
-        // fixed-order reduction over the strip: lanes, then waves
-        for (int off = 32; off >= 1; off >>= 1) {
-            res = res + __shfl_xor(res, off);
-            omega = dmin(omega, __shfl_xor(omega, off));
-        }
-        if (L == 0) { red[0][w] = res; red[1][w] = omega; }
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            double R = red[0][0], O = red[1][0];
-            for (int q = 1; q < C; q++) { R = R + red[0][q]; O = dmin(O, red[1][q]); }
-            part[2 * s] = R;
-            part[2 * s + 1] = O;
-        }
-    }
-}
 
 // ---------------------------------------------------------------------------
 // Jacobian-free quad-row sweeps: LU-SGS and NR at nY > 1.
@@ -367,8 +109,6 @@ k_sweep16_bwd(DevCtx d, const Strip16* strips, int nstrips, double* hand, long l
 
 namespace {
 constexpr int JU = 8;          // steps per unrolled round; prefetch runs JU - 1 steps ahead
-constexpr int JGD = 1;         // extra steps between the four-row groups
-constexpr int JSPAN = 15 + 3 * JGD;  // steps row 15 runs behind row 0
 constexpr int JRS = 8;         // ring slots
 constexpr int JRIN = 4;        // ring lanes of the neighbour strip's components
 
@@ -424,6 +164,20 @@ struct JLds {
     double f[2][16][3][(C + 1) / 2 * 2];  // the waves' partial sums of each row's dot products
 };
 
+// hand-off rows of both sweeps: the sentinel for the columns 1..ni of the
+// strip's block, zero elsewhere; over the whole grid
+__device__ inline void refill_hand(const DevCtx& d, const Strip16* strips, int nstrips, double* hand, long long hstride,
+                                   int dq) {
+    const long long n = 2LL * (nstrips + 1) * hstride;
+    const double sv = __longlong_as_double((long long)SENT16);
+    for (long long e = (long long)blockIdx.x * 256 + threadIdx.x; e < n; e += (long long)gridDim.x * 256) {
+        const int row = (int)((e / hstride) % (nstrips + 1));
+        const long long col = (e % hstride) / dq - HO;
+        const bool live = row < nstrips && col >= 1 && col <= d.blk[strips[row].b].ni;
+        hand[e] = live ? sv : 0.0;
+    }
+}
+
 // cell of (strip, step t, row r)
 __device__ inline bool jslot_cell(const Strip16& S, const DevBlock& B, int t, int r, int& i, int& j) {
     i = t - r - JGD * (r >> 2) + 1;
@@ -441,16 +195,7 @@ __global__ void __launch_bounds__(256) k_rhs_jd16(DevCtx d, const Strip16* strip
                                                   int dqdt_inline, char* recs, double* hand, long long hstride) {
     using D = Dims<NY>;
     constexpr int dq = D::dq, C = (dq + 3) / 4, W0 = NY / 4;
-    {
-        const long long n = 2LL * (nstrips + 1) * hstride;
-        const double sv = __longlong_as_double((long long)SENT16);
-        for (long long e = (long long)blockIdx.x * 256 + threadIdx.x; e < n; e += (long long)gridDim.x * 256) {
-            const int row = (int)((e / hstride) % (nstrips + 1));
-            const long long col = (e % hstride) / dq - HO;
-            const bool live = row < nstrips && col >= 1 && col <= d.blk[strips[row].b].ni;
-            hand[e] = live ? sv : 0.0;
-        }
-    }
+    refill_hand(d, strips, nstrips, hand, hstride, D::dq);
     const int s = (int)blockIdx.x / nsteps16;
     const Strip16 S = strips[s];
     const int t = 16 * ((int)blockIdx.x % nsteps16) + (int)(threadIdx.x & 15), r = (int)(threadIdx.x >> 4);
@@ -587,6 +332,68 @@ __device__ inline void jsweep_compute(JLds<NY>& lds, char* rec, int nt, int w, i
 #undef JLOAD
 }
 
+// the wave that takes the neighbour strip's columns: step e takes column
+// col0 + e (forward) or col0 - e (backward), in the ring before the barrier of
+// step e - 1.  Two loads cover 2 NQ steps; the next pair is issued, from the
+// step then wanted, before the last is looked at.  Takes nt + 1 barriers.
+template <int NY, bool BWD>
+__device__ inline void jcourier_in(double (&ring)[JRS][(NY + 6) / 4 * 64], const DevCtx& d, const Strip16& S,
+                                   const double* hand, long long hstride, long long spin_limit, int nt, int L) {
+    constexpr int dq = NY + 3;
+    constexpr int NQ = 64 / dq;
+    const int from = BWD ? S.next : S.prev;
+    if (from < 0) {
+        for (int t = 0; t < nt + 1; t++) jbarrier();
+        return;
+    }
+    const __amdgpu_buffer_rsrc_t rin = jview(hand + (long long)from * hstride, hstride * 8);
+    const int col0 = BWD ? nt - JSPAN : 1;
+    const int q0 = L / dq, k = L % dq;
+    const bool used = q0 < NQ;
+    auto poll = [&](int e, double& x0, double& x1) {
+        asm volatile("" ::: "memory");  // a poll is a new load
+        const int c0 = col0 + (BWD ? -(e + q0) : e + q0), c1 = c0 + (BWD ? -NQ : NQ);
+        x0 = jv_ld(rin, ((HO + c0) * dq + k) * 8);
+        x1 = jv_ld(rin, ((HO + c1) * dq + k) * 8);
+    };
+    int have = 0, f1 = 0;  // steps below `have` are in the ring
+    double x0, x1;
+    poll(0, x0, x1);
+    long long it = 0;
+    bool dead = false;
+    // looks at the loads in flight; steps up to `last` may enter the ring
+    auto look = [&](int last) {
+        const double v0 = x0, v1 = x1;
+        const int f = f1;
+        f1 = have;
+        poll(have, x0, x1);
+        const unsigned long long m0 = __ballot(dead || !used || !is_sent16(v0));
+        const unsigned long long m1 = __ballot(dead || !used || !is_sent16(v1));
+        int ready = m0 == ~0ULL ? NQ : __builtin_ctzll(~m0) / dq;
+        if (ready == NQ) ready += m1 == ~0ULL ? NQ : __builtin_ctzll(~m1) / dq;
+        const int upto = min(f + ready - 1, last);
+        const int e0 = f + q0, e1 = e0 + NQ;
+        const int lane = 64 * (k >> 2) + JRIN + (k & 3);
+        if (used && e0 >= have && e0 <= upto) ring[e0 & (JRS - 1)][lane] = is_sent16(v0) ? 0.0 : v0;
+        if (used && e1 >= have && e1 <= upto) ring[e1 & (JRS - 1)][lane] = is_sent16(v1) ? 0.0 : v1;
+        if (upto >= have) {
+            have = upto + 1;
+            it = 0;
+        } else if (!dead && it++ >= spin_limit + 1) {
+            atomicCAS(d.iflag + IFLAG_ERR, 0, SHCFD_E_SPIN);
+            dead = true;  // no further waits in this sweep: it runs to its end with zeros
+        }
+    };
+    while (have < 1) look(0);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    jbarrier();
+    for (int t = 0; t < nt; t++) {
+        while (have < t + 2) look(t + JRS - 1);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        jbarrier();
+    }
+}
+
 // forward and backward sweeps: one workgroup of C compute waves and two
 // hand-off waves per strip.  Backward, workgroup g handles strip nstrips-1-g,
 // so the strip it waits on (the one above) has a lower workgroup id.
@@ -608,62 +415,7 @@ k_sweep16j(DevCtx d, const Strip16* strips, int nstrips, double* hand, long long
         if (wave < NY / 4) jsweep_compute<NY, BWD, true>(lds, rec, nt, wave, L);
         else jsweep_compute<NY, BWD, false>(lds, rec, nt, wave, L);
     } else if (wave == C) {
-        // the neighbour strip's columns: step e takes column col0 + e (forward)
-        // or col0 - e (backward), in the ring before the barrier of step e - 1.
-        // Two loads cover 2 NQ steps; the next pair is issued, from the step
-        // then wanted, before the last is looked at
-        constexpr int NQ = 64 / dq;
-        const int from = BWD ? S.next : S.prev;
-        if (from < 0) {
-            for (int t = 0; t < nt + 2; t++) jbarrier();
-            return;
-        }
-        const __amdgpu_buffer_rsrc_t rin = jview(hand + (long long)from * hstride, hstride * 8);
-        const int col0 = BWD ? nt - JSPAN : 1;
-        const int q0 = L / dq, k = L % dq;
-        const bool used = q0 < NQ;
-        auto poll = [&](int e, double& x0, double& x1) {
-            asm volatile("" ::: "memory");  // a poll is a new load
-            const int c0 = col0 + (BWD ? -(e + q0) : e + q0), c1 = c0 + (BWD ? -NQ : NQ);
-            x0 = jv_ld(rin, ((HO + c0) * dq + k) * 8);
-            x1 = jv_ld(rin, ((HO + c1) * dq + k) * 8);
-        };
-        int have = 0, f1 = 0;  // steps below `have` are in the ring
-        double x0, x1;
-        poll(0, x0, x1);
-        long long it = 0;
-        bool dead = false;
-        // looks at the loads in flight; steps up to `last` may enter the ring
-        auto look = [&](int last) {
-            const double v0 = x0, v1 = x1;
-            const int f = f1;
-            f1 = have;
-            poll(have, x0, x1);
-            const unsigned long long m0 = __ballot(dead || !used || !is_sent16(v0));
-            const unsigned long long m1 = __ballot(dead || !used || !is_sent16(v1));
-            int ready = m0 == ~0ULL ? NQ : __builtin_ctzll(~m0) / dq;
-            if (ready == NQ) ready += m1 == ~0ULL ? NQ : __builtin_ctzll(~m1) / dq;
-            const int upto = min(f + ready - 1, last);
-            const int e0 = f + q0, e1 = e0 + NQ;
-            const int lane = 64 * (k >> 2) + JRIN + (k & 3);
-            if (used && e0 >= have && e0 <= upto) lds.ring[e0 & (JRS - 1)][lane] = is_sent16(v0) ? 0.0 : v0;
-            if (used && e1 >= have && e1 <= upto) lds.ring[e1 & (JRS - 1)][lane] = is_sent16(v1) ? 0.0 : v1;
-            if (upto >= have) {
-                have = upto + 1;
-                it = 0;
-            } else if (!dead && it++ >= spin_limit + 1) {
-                atomicCAS(d.iflag + IFLAG_ERR, 0, SHCFD_E_SPIN);
-                dead = true;  // no further waits in this sweep: it runs to its end with zeros
-            }
-        };
-        while (have < 1) look(0);
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        jbarrier();
-        for (int t = 0; t < nt; t++) {
-            while (have < t + 2) look(t + JRS - 1);
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-            jbarrier();
-        }
+        jcourier_in<NY, BWD>(lds.ring, d, S, hand, hstride, spin_limit, nt, L);
         jbarrier();
     } else {
         // the strip's own columns: the terms of step t are in the ring after
@@ -684,9 +436,150 @@ k_sweep16j(DevCtx d, const Strip16* strips, int nstrips, double* hand, long long
     }
 }
 
-// after the sweeps: dq = alpha z into the natural field; LU-SGS: q += dq over
-// the active blocks; NR: (res, omega) partials per workgroup
+// ---------------------------------------------------------------------------
+// Sweeps over the stored matrices (precon, preconLU-SGS; LU-SGS and NR with the
+// closed form switched off), in the same layout and schedule, with the same
+// hand-off in its own wave.  Every lane evaluates the reference's per-cell
+// formula with the operation order of the row-per-lane sweeps, on the same
+// inputs, in a topological order of the same dependency graph, so the results
+// are identical:
+//     x = alpha (R + (A+(i-1) x(i-1) dsci + B+(j-1) x(j-1) dscj))   forward
+//     x = x* - alpha (A-(i+1) x(i+1) dsci + B-(j+1) x(j+1) dscj)    backward
+// A lane reads its two matrix rows (2 dq doubles) and the cell's alpha, dsci,
+// dscj of each step from the quad-row copy written by k_set_abpm16 as dq + 2
+// pairs of doubles, pair p of global step g = base + t at
+// ((((set NT + g) C + w) (dq+2) + p) 64 + lane) 2: every 16-byte load of a wave
+// reads 1 KB of consecutive bytes.  The right-hand side and the results, R* in
+// place, are stored by (strip, step, wave, lane).  Slots of no cell hold zeros.
+//
+// Bound by the matrix rows: 43 KB per step at nY = 9 through one CU's 64 bytes
+// per cycle (280 ns of the 400 ns of a step), beside 48 dependent FP64
+// operations; then by the hand-off.  Measured at nY = 9 on 223 x 99: 249 us
+// forward and 245 us backward (before, dq and q read and written in place and
+// the hand-off polled by the computing waves, 327 and 447 us); prefetching
+// four steps instead of three 260 us, since the rows then pass through
+// accumulation registers.
+// ---------------------------------------------------------------------------
 template <int NY>
+__global__ void __launch_bounds__(256) k_rhs16m(DevCtx d, const Strip16* strips, int nstrips, int nsteps16,
+                                                int dqdt_inline, double* Rs, double* hand, long long hstride) {
+    using D = Dims<NY>;
+    constexpr int dq = D::dq, C = (dq + 3) / 4;
+    refill_hand(d, strips, nstrips, hand, hstride, dq);
+    const int s = (int)blockIdx.x / nsteps16;
+    const Strip16 S = strips[s];
+    const int t = 16 * ((int)blockIdx.x % nsteps16) + (int)(threadIdx.x & 15), r = (int)(threadIdx.x >> 4);
+    const DevBlock B = d.blk[S.b];
+    if (t >= (B.ni + JSPAN + JU - 1) / JU * JU) return;
+    int i, j;
+    double x[dq];
+    if (jslot_cell(S, B, t, r, i, j)) {
+        const long long c = cidx(B, i, j);
+        double bal[dq];
+        flux_balance<NY>(d, B, c, bal);
+        rhs_of_cell<NY>(
+            d, c, bal, dqdt_inline != 0, [&](int k) { return FLD(d, SHCFD_F_PRE1, k, c); },
+            [&](int k) { return FLD(d, SHCFD_F_PRE2, k, c); }, [&]() { return FLD(d, SHCFD_F_PRESCA, 1, c); }, x);
+    } else {
+#pragma unroll
+        for (int k = 0; k < dq; k++) x[k] = 0.0;
+    }
+#pragma unroll
+    for (int w = 0; w < C; w++) {
+        double rv[4];
+#pragma unroll
+        for (int cc = 0; cc < 4; cc++) rv[cc] = 4 * w + cc < dq ? x[4 * w + cc < dq ? 4 * w + cc : 0] : 0.0;
+        double2* o = reinterpret_cast<double2*>(Rs + ((S.base + t) * C + w) * 64) + 2 * r;
+        o[0] = make_double2(rv[0], rv[1]);
+        o[1] = make_double2(rv[2], rv[3]);
+    }
+}
+
+template <int NY>
+struct MLds {
+    static constexpr int C = (NY + 6) / 4;
+    double ring[JRS][C * 64];
+    double x[2][16][4 * C];    // the unknowns of each row's cell
+};
+
+// prefetch distance, in steps: up to four waves have a SIMD's 512 registers
+// each, more share them
+template <int NY>
+constexpr int pdm() { return NY <= 9 ? 3 : NY <= 13 ? 2 : 1; }
+
+template <int NY, bool BWD>
+__global__ void __launch_bounds__(64 * ((NY + 6) / 4 + 1))
+k_sweep16m(DevCtx d, const Strip16* strips, int nstrips, double* hand, long long hstride, long long spin_limit,
+           const double* __restrict__ jac, long long nsl, double* Rs) {
+    constexpr int dq = NY + 3, C = (dq + 3) / 4, dq2 = dq + 2, PD = pdm<NY>(), NB = PD + 1;
+    static_assert(JU == 8, "rounds");
+    __shared__ __attribute__((aligned(16))) MLds<NY> lds;
+    const int s = BWD ? nstrips - 1 - (int)blockIdx.x : (int)blockIdx.x;
+    const int L = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const Strip16 S = strips[s];
+    const int ni = d.blk[S.b].ni, nt = (ni + JSPAN + JU - 1) / JU * JU;
+    for (int e = (int)threadIdx.x; e < JRS * C * 64; e += 64 * (C + 1)) lds.ring[e / (C * 64)][e % (C * 64)] = 0.0;
+    lds_barrier();
+    if (w == C) {
+        jcourier_in<NY, BWD>(lds.ring, d, S, hand, hstride, spin_limit, nt, L);
+        return;
+    }
+    const int r = L >> 2, c = L & 3, k = 4 * w + c, gr = L >> 4;
+    const int src = 64 * w + (BWD ? (gr == 3 ? JRIN + c : 16 * (gr + 1) + c)
+                                  : (gr == 0 ? JRIN + c : 16 * (gr - 1) + 12 + c));
+    const int dst = 64 * w + ((L & ~3) == JRIN ? L + 4 : L);
+    const double* jl = jac + ((((BWD ? nsl : 0) + S.base) * C + w) * dq2 * 64 + L) * 2;
+    double* Rl = Rs + (S.base * C + w) * 64 + L;
+    auto at = [&](int t) { return (long long)(BWD ? nt - 1 - t : t); };  // stored step of sweep step t
+    auto load = [&](int t, StepIn<dq>& in) {
+        const long long g = at(min(t, nt - 1));  // past the end: the last step again
+        load_ops<dq>(jl + 128LL * C * dq2 * g, in);
+        in.r = Rl[g * (C * 64)];
+    };
+    // the strip's own hand-off: row 15 (forward) or 0 (backward), column col at step t
+    const bool out = (BWD ? S.prev : S.next) >= 0 && r == (BWD ? 0 : 15) && k < dq;
+    const __amdgpu_buffer_rsrc_t rout = jview(hand + (long long)s * hstride, hstride * 8);
+    StepIn<dq> buf[NB];
+#pragma unroll
+    for (int p = 0; p < PD; p++) load(p, buf[p]);
+    wait_vmem();
+    jbarrier();  // ring cleared, the neighbour's column of step 0 there
+    double nb = lds.ring[0][src], a_in = 0.0, bo = 0.0;
+    for (int t0 = 0; t0 < nt; t0 += NB) {
+#pragma unroll
+        for (int u = 0; u < NB; u++) {
+            const int t = t0 + u;
+            if (t >= nt) break;
+            load(t + PD, buf[(u + PD) % NB]);
+            const StepIn<dq>& in = buf[u];
+            const double b_in = row_shift4<!BWD>(nb, bo);
+            const double x = BWD ? in.r - in.al * (a_in + b_in) : in.al * (in.r + (a_in + b_in));
+            Rl[at(t) * (C * 64)] = x;
+            lds.x[t & 1][r][k] = x;
+            lds_barrier();
+            double xa[dq];
+#pragma unroll
+            for (int l = 0; l < dq; l++) xa[l] = lds.x[t & 1][r][l];
+            nb = lds.ring[(t + 1) & (JRS - 1)][src];
+            double sa = 0.0, sb = 0.0;
+#pragma unroll
+            for (int l = 0; l < dq; l++) {
+                sa = sa + in.a[l] * xa[l];
+                sb = sb + in.b[l] * xa[l];
+            }
+            a_in = in.fi * sa;
+            bo = in.fj * sb;
+            lds.ring[(t + 1 + JGD) & (JRS - 1)][dst] = bo;
+            const int col = BWD ? nt - t : t + 1 - JSPAN;
+            jv_st(rout, bo, out ? ((HO + col) * dq + k) * 8 : JV_DROP);
+        }
+    }
+}
+
+// after the sweeps: dq (alpha z of the closed form; x of the matrix sweeps, MAT)
+// into the natural field; LU-SGS and preconLU-SGS: q += dq over the active
+// blocks; NR and precon: (res, omega) partials per workgroup
+template <int NY, bool MAT>
 __global__ void __launch_bounds__(256) k_post16j(DevCtx d, const Strip16* strips, int nsteps16, const char* recs,
                                                  double* part) {
     constexpr int dq = NY + 3, C = (dq + 3) / 4;
@@ -700,11 +593,11 @@ __global__ void __launch_bounds__(256) k_post16j(DevCtx d, const Strip16* strips
     int i, j;
     if (jslot_cell(S, B, t, r, i, j)) {
         const long long c = cidx(B, i, j);
-        const char* rec = recs + (JPAD + S.base + t) * jrec_step<NY>();
-        const double al = FLD(d, SHCFD_F_ALPHA, 0, c);
+        const char* rec = recs + (MAT ? (S.base + t) * (C * 512) : (JPAD + S.base + t) * jrec_step<NY>());
+        const double al = MAT ? 1.0 : FLD(d, SHCFD_F_ALPHA, 0, c);
 #pragma unroll
         for (int w = 0; w < C; w++) {
-            const double2* z = reinterpret_cast<const double2*>(rec + jrec_off(NY, w) + JO_R) + 2 * r;
+            const double2* z = reinterpret_cast<const double2*>(rec + (MAT ? w * 512 : jrec_off(NY, w) + JO_R)) + 2 * r;
             const double2 z0 = z[0], z1 = z[1];
             const double x[4] = {al * z0.x, al * z0.y, al * z1.x, al * z1.y};
 #pragma unroll
@@ -736,16 +629,18 @@ __global__ void __launch_bounds__(256) k_post16j(DevCtx d, const Strip16* strips
 }
 
 #define INST(NY)                                                                                              \
-    template __global__ void k_sweep16_fwd<NY>(DevCtx, const Strip16*, int, double*, long long, long long,      \
-                                               const double*, long long);                                     \
-    template __global__ void k_sweep16_bwd<NY>(DevCtx, const Strip16*, int, double*, long long, double*,        \
-                                               long long, const double*, long long);                          \
+    template __global__ void k_rhs16m<NY>(DevCtx, const Strip16*, int, int, int, double*, double*, long long);   \
+    template __global__ void k_sweep16m<NY, false>(DevCtx, const Strip16*, int, double*, long long, long long,  \
+                                                   const double*, long long, double*);                        \
+    template __global__ void k_sweep16m<NY, true>(DevCtx, const Strip16*, int, double*, long long, long long,   \
+                                                  const double*, long long, double*);                         \
     template __global__ void k_rhs_jd16<NY>(DevCtx, const Strip16*, int, int, int, char*, double*, long long);  \
     template __global__ void k_sweep16j<NY, false>(DevCtx, const Strip16*, int, double*, long long, long long,  \
                                                    char*);                                                    \
     template __global__ void k_sweep16j<NY, true>(DevCtx, const Strip16*, int, double*, long long, long long,   \
                                                   char*);                                                     \
-    template __global__ void k_post16j<NY>(DevCtx, const Strip16*, int, const char*, double*);
+    template __global__ void k_post16j<NY, false>(DevCtx, const Strip16*, int, const char*, double*);           \
+    template __global__ void k_post16j<NY, true>(DevCtx, const Strip16*, int, const char*, double*);
 SHCFD_FOR_EACH_NY(INST)
 #undef INST
 

@@ -280,7 +280,7 @@ int shcfd_destroy(shcfd_ctx* ctx) {
     void* ptrs[] = {ctx->dblk, ctx->dtiles, ctx->dstrips, ctx->dprog, ctx->dbnd, ctx->dpart, ctx->scal,
                     ctx->iflag, ctx->dcut, ctx->dbc, ctx->dpool, ctx->dmech, ctx->dskew, ctx->dsbase,
                     ctx->djac16, ctx->dstrips16, ctx->dbnd16, ctx->dnasa9, ctx->dhist, ctx->ddefer,
-                    ctx->djrec16, ctx->djpart16};
+                    ctx->djrec16, ctx->djx16, ctx->djpart16};
     for (void* p : ptrs) if (p) hipFree(p);
     if (ctx->stream) hipStreamDestroy(ctx->stream);
     delete ctx;
@@ -842,17 +842,23 @@ static bool jvp16_scheme(const shcfd_ctx* ctx) {
 
 static bool q16_layout(shcfd_ctx* ctx);
 
+// the (res, omega) partials of the 16-row sweeps' update, one pair per work item
+static bool part16_ready(shcfd_ctx* ctx) {
+    if (ctx->djpart16) return true;
+    if (hipMalloc((void**)&ctx->djpart16, sizeof(double) * 2 * ctx->nstrips16 * ctx->nitem16) == hipSuccess) return true;
+    ctx->djpart16 = nullptr;
+    (void)hipGetLastError();
+    return false;
+}
+
 // the cell records of the Jacobian-free 16-row sweeps; allocated (and cleared,
 // so slots of no cell hold zeros) on first use
 static bool jd16_ready(shcfd_ctx* ctx) {
     if (ctx->djrec16) return true;
     const size_t bytes = ((size_t)ctx->nsl16 + 2 * JPAD) * jrec_off(ctx->ny, (ctx->dimq + 3) / 4);
-    const size_t pbytes = sizeof(double) * 2 * ctx->nstrips16 * ctx->nitem16;
-    if (hipMalloc((void**)&ctx->djpart16, pbytes) != hipSuccess ||
-        hipMalloc((void**)&ctx->djrec16, bytes) != hipSuccess || hipMemset(ctx->djrec16, 0, bytes) != hipSuccess) {
-        hipFree(ctx->djpart16);
+    if (!part16_ready(ctx)) return false;
+    if (hipMalloc((void**)&ctx->djrec16, bytes) != hipSuccess || hipMemset(ctx->djrec16, 0, bytes) != hipSuccess) {
         hipFree(ctx->djrec16);
-        ctx->djpart16 = nullptr;
         ctx->djrec16 = nullptr;
         (void)hipGetLastError();
         return false;
@@ -874,10 +880,13 @@ static bool q16_enabled(shcfd_ctx* ctx) {
         ctx->use_jvp16 = 0;  // no room: the operator copy below
     }
     if (ctx->djac16) return true;
-    const int dq = ctx->dimq, C = (dq + 3) / 4;
-    if (hipMalloc((void**)&ctx->djac16, sizeof(double) * 2 * 2 * 64 * C * (dq + 2) * (size_t)ctx->nsl16) != hipSuccess ||
-        hipMemset(ctx->djac16, 0, sizeof(double) * 2 * 2 * 64 * C * (dq + 2) * (size_t)ctx->nsl16) != hipSuccess) {
+    const size_t dq = (size_t)ctx->dimq, C = (dq + 3) / 4, lanes = 64 * C * (size_t)ctx->nsl16;
+    const size_t jbytes = sizeof(double) * 2 * 2 * (dq + 2) * lanes;
+    if (!part16_ready(ctx) || hipMalloc((void**)&ctx->djx16, sizeof(double) * lanes) != hipSuccess ||
+        hipMalloc((void**)&ctx->djac16, jbytes) != hipSuccess || hipMemset(ctx->djac16, 0, jbytes) != hipSuccess) {
+        hipFree(ctx->djx16);
         hipFree(ctx->djac16);
+        ctx->djx16 = nullptr;
         ctx->djac16 = nullptr;
         ctx->use_skew = 0;
         (void)hipGetLastError();
@@ -895,7 +904,6 @@ static bool q16_layout(shcfd_ctx* ctx) {
     for (int b = 0; b < ctx->nb; b++) {
         const DevBlock& B = ctx->hblk[b];
         maxni = std::max(maxni, B.ni);
-        const int first = (int)st.size();
         for (int j0 = 1; j0 <= B.nj; j0 += 16) {
             Strip16 S{};
             S.b = b;
@@ -907,10 +915,8 @@ static bool q16_layout(shcfd_ctx* ctx) {
             nsl += (B.ni + 18 + 7) / 8 * 8;  // steps of the longest of the sweeps, whole rounds
             st.push_back(S);
         }
-        (void)first;
     }
     const int ns = (int)st.size();
-    if (2 * ns > 2 * ctx->npart) return false;  // (res, omega) partials per strip
     // hand-off row: columns -24 .. maxni + 40 (the consumers' loads run ahead)
     const long long bstride = (long long)(maxni + 64) * dq;
     auto al = [](void** p, size_t bytes) {
@@ -950,7 +956,7 @@ static int abpm_for_step(shcfd_ctx* ctx) {
             ProfScope ps(ctx, PROF_ABPM);
             int maxni = 0;
             for (const auto& B : ctx->hblk) maxni = std::max(maxni, B.ni);
-            dim3 grid((unsigned)ctx->nstrips16, (unsigned)((maxni + 15 + 15) / 16));
+            dim3 grid((unsigned)ctx->nstrips16, (unsigned)((maxni + JSPAN + 15) / 16));
             DISPATCH_NY(ctx->ny, hipLaunchKernelGGL(k_set_abpm16<NY>, grid, dim3(256), 0, ctx->stream, ctx->dev(),
                                                     ctx->dstrips16, ctx->djac16, ctx->nsl16));
             LAUNCHCHK();
@@ -1077,7 +1083,7 @@ static int implicit_async(shcfd_ctx* ctx, int step_internal) {
                                                 ctx->dstrips16, ns16, hand_b, ctx->bstride16, ctx->spin_limit,
                                                 ctx->djrec16)) }
         { ProfScope ps(ctx, PROF_UPDATE);
-        DISPATCH_NY(ctx->ny, hipLaunchKernelGGL(k_post16j<NY>, dim3(items), dim3(256), 0, ctx->stream, d,
+        DISPATCH_NY(ctx->ny, hipLaunchKernelGGL((k_post16j<NY, false>), dim3(items), dim3(256), 0, ctx->stream, d,
                                                 ctx->dstrips16, ctx->nitem16, ctx->djrec16, ctx->djpart16)) }
         if (!inner_loop_scheme(ctx->p.scheme)) {
             LAUNCHCHK();
@@ -1085,28 +1091,37 @@ static int implicit_async(shcfd_ctx* ctx, int step_internal) {
         }
         return finish_inner(ctx, step_internal, ctx->djpart16, (int)items);
     }
+    if (q16) {
+        const unsigned items = (unsigned)ns16 * (unsigned)ctx->nitem16;
+        double* hand_f = ctx->dbnd16;
+        double* hand_b = ctx->dbnd16 + ctx->bstride16 * (ns16 + 1);
+        { ProfScope ps(ctx, PROF_RHS);
+        DISPATCH_NY(ctx->ny, hipLaunchKernelGGL(k_rhs16m<NY>, dim3(items), dim3(256), 0, ctx->stream, d, ctx->dstrips16,
+                                                ns16, ctx->nitem16, ctx->dqdt_inline, ctx->djx16, ctx->dbnd16,
+                                                ctx->bstride16)) }
+        ctx->dqdt_inline = 0;
+        ctx->abpm_inline = 0;
+        const dim3 blk((unsigned)(64 * (C16 + 1)));
+        { ProfScope ps(ctx, PROF_SWEEP_FWD);
+        DISPATCH_NY(ctx->ny, hipLaunchKernelGGL((k_sweep16m<NY, false>), dim3(ns16), blk, 0, ctx->stream, d,
+                                                ctx->dstrips16, ns16, hand_f, ctx->bstride16, ctx->spin_limit,
+                                                ctx->djac16, ctx->nsl16, ctx->djx16)) }
+        { ProfScope ps(ctx, PROF_SWEEP_BWD);
+        DISPATCH_NY(ctx->ny, hipLaunchKernelGGL((k_sweep16m<NY, true>), dim3(ns16), blk, 0, ctx->stream, d,
+                                                ctx->dstrips16, ns16, hand_b, ctx->bstride16, ctx->spin_limit,
+                                                ctx->djac16, ctx->nsl16, ctx->djx16)) }
+        { ProfScope ps(ctx, PROF_UPDATE);
+        DISPATCH_NY(ctx->ny, hipLaunchKernelGGL((k_post16j<NY, true>), dim3(items), dim3(256), 0, ctx->stream, d,
+                                                ctx->dstrips16, ctx->nitem16, (const char*)ctx->djx16,
+                                                ctx->djpart16)) }
+        if (inner_loop_scheme(ctx->p.scheme)) return finish_inner(ctx, step_internal, ctx->djpart16, (int)items);
+        LAUNCHCHK();
+        return SHCFD_OK;
+    }
     { ProfScope ps(ctx, PROF_RHS);
     DISPATCH_NY(ctx->ny, TILE_LAUNCH(k_rhs<NY>, ctx->dprog, 2 * ns, ctx->dqdt_inline, ctx->abpm_inline)); }
     ctx->dqdt_inline = 0;
     ctx->abpm_inline = 0;
-    if (q16) {
-        const dim3 blk((unsigned)(64 * C16));
-        double* hand_f = ctx->dbnd16;
-        double* hand_b = ctx->dbnd16 + ctx->bstride16 * (ns16 + 1);
-        { ProfScope ps(ctx, PROF_SWEEP_FWD);
-        hipLaunchKernelGGL(k_fill16, dim3(256), dim3(256), 0, ctx->stream, d, ctx->dstrips16, ns16, ctx->dbnd16,
-                           ctx->bstride16, ctx->dimq);
-        DISPATCH_NY(ctx->ny, hipLaunchKernelGGL(k_sweep16_fwd<NY>, dim3(ns16), blk, 0, ctx->stream, d, ctx->dstrips16,
-                                                ns16, hand_f, ctx->bstride16, ctx->spin_limit, ctx->djac16,
-                                                ctx->nsl16)) }
-        { ProfScope ps(ctx, PROF_SWEEP_BWD);
-        DISPATCH_NY(ctx->ny, hipLaunchKernelGGL(k_sweep16_bwd<NY>, dim3(ns16), blk, 0, ctx->stream, d, ctx->dstrips16,
-                                                ns16, hand_b, ctx->bstride16, ctx->dpart, ctx->spin_limit, ctx->djac16,
-                                                ctx->nsl16)) }
-        if (inner_loop_scheme(ctx->p.scheme)) return finish_inner(ctx, step_internal, ctx->dpart, ns16);
-        LAUNCHCHK();
-        return SHCFD_OK;
-    }
     const bool sk = ctx->skew_active && ctx->dskew;
     ctx->skew_active = 0;
     { ProfScope ps(ctx, PROF_SWEEP_FWD);

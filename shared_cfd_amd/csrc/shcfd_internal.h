@@ -195,6 +195,7 @@ struct Ctx {
     int jd16_active = 0;           // the next implicit update runs them
     int nitem16 = 0;               // 16-step work items of the longest strip
     char* djrec16 = nullptr;       // their cell records, nsl16 + 2 JPAD steps
+    double* djx16 = nullptr;       // right-hand side and results of the matrix sweeps by (strip, step, wave, lane)
     double* djpart16 = nullptr;    // (res, omega) partials per work item
     int skew_active = 0;           // the last set_ABpm of a step wrote the skewed copy
     double* dskew = nullptr;

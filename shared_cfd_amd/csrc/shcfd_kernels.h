@@ -558,24 +558,24 @@ template <int NY> __global__ void k_update(DevCtx, const Tile*);
 __global__ void k_reduce_res_omega(DevCtx, const double*, int);
 // quad-row sweeps for nY > 1 (k_sweep16.hip; operators from k_set_abpm16)
 template <int NY> __global__ void k_set_abpm16(DevCtx, const Strip16*, double*, long long);
-__global__ void k_fill16(DevCtx, const Strip16*, int, double*, long long, int);
+template <int NY> __global__ void k_rhs16m(DevCtx, const Strip16*, int, int, int, double*, double*, long long);
+template <int NY, bool BWD>
+__global__ void k_sweep16m(DevCtx, const Strip16*, int, double*, long long, long long, const double*, long long, double*);
 template <int NY>
 __global__ void k_rhs_jd16(DevCtx, const Strip16*, int, int, int, char*, double*, long long);
 template <int NY, bool BWD>
 __global__ void k_sweep16j(DevCtx, const Strip16*, int, double*, long long, long long, char*);
-template <int NY> __global__ void k_post16j(DevCtx, const Strip16*, int, const char*, double*);
-// bytes of a cell record of theirs, in waves of species alone and in the
+template <int NY, bool MAT> __global__ void k_post16j(DevCtx, const Strip16*, int, const char*, double*);
+// extra steps between the four-row groups of a strip, and the steps that row 15
+// runs behind row 0: row r works on column t - r - JGD (r >> 2) + 1 at step t
+constexpr int JGD = 1, JSPAN = 15 + 3 * JGD;
+// bytes of a cell record of the closed form's sweeps, in waves of species alone and in the
 // others, and of wave w's offset in a step (w = the number of waves: the
 // step); steps of padding at both ends, which the sweeps' prefetch reads
 constexpr int JREC_S = 2304, JREC_M = 4096, JPAD = 8;
 __host__ __device__ constexpr int jrec_off(int ny, int w) {
     return w < ny / 4 ? w * JREC_S : (ny / 4) * JREC_S + (w - ny / 4) * JREC_M;
 }
-template <int NY>
-__global__ void k_sweep16_fwd(DevCtx, const Strip16*, int, double*, long long, long long, const double*, long long);
-template <int NY>
-__global__ void k_sweep16_bwd(DevCtx, const Strip16*, int, double*, long long, double*, long long, const double*,
-                              long long);
 __global__ void k_copy_scal(DevCtx, int, int);
 // chemistry (k_chem.hip)
 enum { CHEM_OP_FEX = 0, CHEM_OP_FEXVAR = 1, CHEM_OP_JEX = 2, CHEM_OP_CALCT = 3, CHEM_OP_CHEMEQ2 = 4,

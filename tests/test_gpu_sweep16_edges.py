@@ -1,10 +1,10 @@
-"""The closed-form sweeps of more than one species at the edges of their
-strips: block heights around multiples of the 16-row strip and its four-row
+"""The sweeps of more than one species at the edges of their strips: block heights around multiples of the 16-row strip and its four-row
 groups, widths around the eight-step rounds, and species counts that leave
 the last compute wave with one to four components.
 
-Both sides evaluate the same update from the same state; the closed form sums
-in another order.  Each cell's increment is a chain of at most ni + nj
+Both sides evaluate the same update from the same state.  The sweeps over stored
+matrices keep the order of every sum, so their result is the same; the closed
+form sums in another order.  Each cell's increment is a chain of at most ni + nj
 products whose factors have norm below one (diagonal dominance), so the
 rounding differences add up to a small multiple of (ni + nj) eps of the
 increments; species with increments far below the others' carry the rounding
@@ -14,14 +14,19 @@ import numpy as np
 import pytest
 
 from shared_cfd_amd import cases as C
-from shared_cfd_amd.native import OPT_SKEW_SWEEP, Solver
+from shared_cfd_amd.native import OPT_JVP_SWEEP, OPT_SKEW_SWEEP, Solver
 
 pytestmark = pytest.mark.gpu
 
 
-def _increments(case, skew, reps):
+SIZES = [(2, 2, 2), (2, 14, 17), (3, 13, 4), (4, 15, 15), (5, 14, 5), (8, 30, 16), (9, 31, 17), (9, 6, 48),
+         (9, 22, 49), (10, 3, 65), (11, 130, 7), (13, 62, 33), (16, 21, 33)]
+
+
+def _increments(case, skew, reps, jvp=1):
     s = Solver(case)
     s.set_option(OPT_SKEW_SWEEP, skew)
+    s.set_option(OPT_JVP_SWEEP, jvp)
     s.prepare()
     for k in range(reps):
         s.step(k + 1, 0)
@@ -31,9 +36,7 @@ def _increments(case, skew, reps):
 
 
 @pytest.mark.parametrize("scheme", [C.SCHEME_LUSGS, C.SCHEME_NR])
-@pytest.mark.parametrize("ny,ni,nj", [(2, 2, 2), (2, 14, 17), (3, 13, 4), (4, 15, 15), (5, 14, 5), (8, 30, 16),
-                                      (9, 31, 17), (9, 6, 48), (9, 22, 49), (10, 3, 65), (11, 130, 7), (13, 62, 33),
-                                      (16, 21, 33)])
+@pytest.mark.parametrize("ny,ni,nj", SIZES)
 def test_strip_edges(scheme, ny, ni, nj):
     case = C.random_case(seed=ni + nj, ni=(ni, 9), nj=(nj, 20), ny=ny, scheme=scheme)
     case.params.res_rate_warning = case.params.res_rate_error = 1e300
@@ -41,3 +44,15 @@ def test_strip_edges(scheme, ny, ni, nj):
         scale = np.max(np.abs(b))
         assert scale > 0.0
         assert np.max(np.abs(a - b)) <= 1e-12 * scale
+
+
+@pytest.mark.parametrize("scheme", [C.SCHEME_LUSGS, C.SCHEME_PRECON_LUSGS, C.SCHEME_PRECON])
+@pytest.mark.parametrize("ny,ni,nj", SIZES)
+def test_strip_edges_stored_matrices(scheme, ny, ni, nj):
+    local = scheme != C.SCHEME_LUSGS
+    case = C.random_case(seed=ni + nj, ni=(ni, 9), nj=(nj, 20), ny=ny, scheme=scheme, time_step=1 if local else 0,
+                         mach=0.3)
+    case.params.res_rate_warning = case.params.res_rate_error = 1e300
+    for a, b in zip(_increments(case, 1, 2, jvp=0), _increments(case, 0, 2)):
+        assert np.max(np.abs(b)) > 0.0
+        assert np.array_equal(a, b)
