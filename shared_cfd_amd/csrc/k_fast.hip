@@ -322,8 +322,8 @@ __device__ inline int col_off(int col) { return (col + HOFF) * 32; }
 // DPP moves per step.
 //
 // Measured, forward / backward us per launch: 258,048-cell forward step 167 /
-// 152 -> 130 / 118; 512x128 C-mesh 84 / 87 -> 65 / 66; 400x4 tube 46 / 47 ->
-// 32 / 32 (one strip: 112 -> 75 ns per step).  A hop between strips costs 18
+// 152 -> 135 / 122; 512x128 C-mesh 84 / 87 -> 65 / 66; 400x4 tube 47 / 47 ->
+// 29 / 33 (one strip: 112 -> 75 ns per step).  A hop between strips costs 18
 // steps of skew, up to 5 of chunk granularity and 1.3 us from the producer's
 // store to the consumer's look.
 constexpr int CS = 4;                                   // steps per LDS chunk

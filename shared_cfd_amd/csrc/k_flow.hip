@@ -261,17 +261,15 @@ __device__ inline void bc_corner_cell(const DevCtx& d, int gid) {
     int pi = (gid & 1) ? 1 : -1, pj = (gid & 2) ? 1 : -1;
     int i = (pi < 0) ? 1 : B.ni, j = (pj < 0) ? 1 : B.nj;
     long long cc = cidx(B, i + pi, j + pj), c0 = cidx(B, i, j), cj = cidx(B, i, j + pj), ci = cidx(B, i + pi, j);
-    double wv[D::dw], vh[NY];  // all loads before the first store, as in copy_wv
+    // component by component: k_set_hv_tg runs this beside its faces, and holding
+    // all components here costs it registers (167 -> 188 us on 48 plate blocks)
 #pragma unroll
     for (int k = 0; k < D::dw; k++)
-        wv[k] = (1.0 / 3.0) * ((FLD(d, SHCFD_F_W, k, c0) + FLD(d, SHCFD_F_W, k, cj)) + FLD(d, SHCFD_F_W, k, ci));
+        FLD(d, SHCFD_F_W, k, cc) = (1.0 / 3.0) * ((FLD(d, SHCFD_F_W, k, c0) + FLD(d, SHCFD_F_W, k, cj)) + FLD(d, SHCFD_F_W, k, ci));
 #pragma unroll
     for (int k = 0; k < NY; k++)
-        vh[k] = (1.0 / 3.0) * ((FLD(d, SHCFD_F_VHI, k, c0) + FLD(d, SHCFD_F_VHI, k, cj)) + FLD(d, SHCFD_F_VHI, k, ci));
-#pragma unroll
-    for (int k = 0; k < D::dw; k++) FLD(d, SHCFD_F_W, k, cc) = wv[k];
-#pragma unroll
-    for (int k = 0; k < NY; k++) FLD(d, SHCFD_F_VHI, k, cc) = vh[k];
+        FLD(d, SHCFD_F_VHI, k, cc) =
+            (1.0 / 3.0) * ((FLD(d, SHCFD_F_VHI, k, c0) + FLD(d, SHCFD_F_VHI, k, cj)) + FLD(d, SHCFD_F_VHI, k, ci));
 }
 template <int NY>
 __global__ void k_bc_corner(DevCtx d) {
