@@ -40,7 +40,7 @@ __global__ void __launch_bounds__(256) k_thermo_chem(DevCtx d, const Tile* tiles
 #pragma unroll
     for (int k = 0; k < NS; k++) vrho[k] = FLD(d, SHCFD_F_Q, k, c);
     chem::ThermoOut<NS> o;
-    if (chem::calc_t<NS>(m, vrho, rho, ei, T, o) < 0) atomicCAS(d.iflag + IFLAG_ERR, 0, SHCFD_E_TNEWTON);
+    if (chem::calc_t<NS, NS>(m, vrho, rho, ei, T, o) < 0) atomicCAS(d.iflag + IFLAG_ERR, 0, SHCFD_E_TNEWTON);
     double rg = chem::R_UNI / o.mwave;
     double p = rho * rg * T;
     FLD(d, SHCFD_F_W, D::ir, c) = rg;

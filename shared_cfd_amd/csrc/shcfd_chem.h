@@ -701,7 +701,11 @@ template <int NS>
 struct ThermoOut {
     double kappa, mwave, mu, dhi[NS], vhi[NS];
 };
-template <int NS>
+// NT bounds the transport entries (m->nt): a table may list a species twice, so
+// it may hold more entries than species.  The flow, whose tables are refused
+// with more, takes NT = NS (16 entries at six species: 166 -> 182 VGPRs, two
+// waves per SIMD instead of three).
+template <int NS, int NT = SHCFD_CHEM_MAX_NS>
 SHCFD_HD int calc_t(const shcfd_mech* m, const double* vrho, double rho, double E, double& T_io, ThermoOut<NS>& out) {
     double n[NS];
     double tmp = rho * 1e-11;
@@ -764,7 +768,8 @@ SHCFD_HD int calc_t(const shcfd_mech* m, const double* vrho, double rho, double 
     // Wilke mixture viscosity (:1600-1633)
     double logT = dlog(T), invT = 1.0 / T;
     double cmu[4] = {logT, invT, invT * invT, 1.0};
-    SVec<NS> muN, nv;
+    SVec<NT> muN;  // by transport entry
+    SVec<NS> nv;
     muN.fill(0.0);
     nv.from(n);
     for (int i = 0; i < m->nt; i++) {

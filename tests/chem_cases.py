@@ -108,3 +108,20 @@ def no27_plus_inert(outdir, k):
     with open(p, "w") as f:
         f.write("\n".join(out))
     return p, ["N2", "O2", "H2", "OH", "O", "H", "HO2", "H2O"] + names
+
+
+def repeated_trans(outdir, extra):
+    """no27_trans.inp with its first `extra` entries listed a second time: a
+    table with more transport entries than species once extra > 1 (no27: seven
+    entries for eight species)."""
+    lines = open(NO27.replace("chem", "trans")).read().split("\n")
+    entries, k = [], 1
+    while lines[k][:3].upper() != "END" and lines[k].strip():
+        n = 1 + int(lines[k][35]) + int(lines[k][37])
+        entries.append(lines[k:k + n])
+        k += n
+    os.makedirs(outdir, exist_ok=True)
+    p = os.path.join(outdir, "trans.inp")
+    with open(p, "w") as f:
+        f.write("\n".join([lines[0]] + [ln for e in entries + entries[:extra] for ln in e] + ["END"]))
+    return p

@@ -1,8 +1,10 @@
 """Host-side chemistry of the library (no GPU): boundary states and the
 parser of the 9-species test mechanism, against the CPU oracle; the
-production rates Jex forms beside the Jacobian, against Fex."""
+production rates Jex forms beside the Jacobian, against Fex; tables with more
+transport entries than species."""
 import ctypes
 import os
+import subprocess
 
 import numpy as np
 import pytest
@@ -11,7 +13,7 @@ from oracle import oracle as O
 from oracle.chem_inp import read_cheminp
 from shared_cfd_amd import chem
 
-from chem_cases import no27_plus_h2o2
+from chem_cases import NO27, no27_plus_h2o2, repeated_trans
 
 
 @pytest.fixture(scope="module")
@@ -74,3 +76,23 @@ def test_jex_production_rates_are_fex_bit_for_bit(mechs, which):
                           g.ctypes.data_as(dp)) == 0
     assert np.all(np.isfinite(f)) and np.max(np.abs(f[:, :ns])) > 0
     assert np.array_equal(f, g)
+
+
+@pytest.mark.parametrize("extra", [0, 1, 2, 5])
+def test_more_transport_entries_than_species(tmp_path, extra):
+    """A trans.inp that lists species twice gives up to 16 entries for any
+    species count: every index stays in its array, and the viscosity is the
+    oracle's, bit for bit."""
+    t = repeated_trans(str(tmp_path), extra)
+    lm, om = chem.parse(NO27, t), read_cheminp(NO27, chem.MW_INP, t)
+    assert (lm.ns, lm.nt) == (om.ns, om.nt) == (8, 7 + extra)
+    table = tmp_path / "mech.bin"
+    table.write_bytes(bytes(lm))
+    rel = np.random.default_rng(extra).random(8) + 0.01
+    exe = os.path.join(os.path.dirname(os.path.abspath(__file__)), "host", "chem_bounds")
+    r = subprocess.run([exe, str(table), "1500.0", *[repr(float(v)) for v in rel]], capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr
+    vrho, rho, E = O.chem_rho_rel2abs(om, 1.01325e5, 1500.0, rel)
+    mu = O.chem_calc_t(om, vrho, rho, E, 1500.0)[1][2]
+    assert float(r.stdout) == mu
+    assert chem.boundary_state(lm, 1.01325e5, 1500.0, rel)[0][8 + 7] == mu

@@ -12,9 +12,11 @@ import pytest
 
 from oracle import oracle as O
 from oracle.chem_inp import read_cheminp
+from shared_cfd_amd import cases as C
 from shared_cfd_amd import chem
+from shared_cfd_amd.native import Solver
 
-from chem_cases import NO27, mixture_states, no27_plus_inert, random_states
+from chem_cases import NO27, mixture_states, no27_plus_inert, random_states, repeated_trans
 
 pytestmark = pytest.mark.gpu
 
@@ -43,3 +45,24 @@ def test_rates_jacobian_and_point_implicit(tmp_path, inert, rows):
         assert st[s] == (-e if e else it)
         if e == 0:
             assert _rel(out[s, :ns], v1) <= 1e-13 and _rel(out[s, ns:], [T1]) <= 1e-13
+
+
+@pytest.mark.parametrize("extra", [1, 2, 9])
+def test_more_transport_entries_than_species(tmp_path, extra):
+    """Tables that list species twice: calc_T takes up to 16 transport entries
+    for any species count; the flow refuses more entries than species."""
+    t = repeated_trans(str(tmp_path), extra)
+    lm, om = chem.parse(NO27, t), read_cheminp(NO27, chem.MW_INP, t)
+    assert (lm.ns, lm.nt) == (8, min(7 + extra, 14))
+    states = mixture_states(om, 65, seed=extra)
+    out, _ = chem.chem_eval(lm, chem.CALCT, np.array([np.concatenate([v, [rho, E, T * 1.02]])
+                                                      for v, rho, E, T in states]))
+    for s, (v, rho, E, T) in enumerate(states):
+        T1, o, _ = O.chem_calc_t(om, v, rho, E, T * 1.02)
+        assert _rel(out[s, :4], [T1, o[0], o[1], o[2]]) <= 1e-13
+    case = C.mixing_layer(lm, ni=8, nj=6, fuel=np.eye(8)[2], ox=np.eye(8)[1])
+    if lm.nt > lm.ns:
+        with pytest.raises(RuntimeError, match="shcfd_set_mechanism"):
+            Solver(case)
+    else:
+        Solver(case).close()
