@@ -9,6 +9,7 @@
 #include <new>
 
 #include "../../include/shcfd.h"
+#include "shcfd_chem.h"
 #include "shcfd_kernels.h"
 #include "shcfd_fast.h"
 
@@ -580,8 +581,7 @@ int shcfd_set_thermo_prop(shcfd_ctx* ctx, int step) {
 }
 
 int shcfd_set_mechanism(shcfd_ctx* ctx, const shcfd_mech* mech) {
-    if (!ctx || !mech || mech->ns != ctx->ny || mech->nr < 1 || mech->nr > SHCFD_CHEM_MAX_NR ||
-        mech->nt < 0 || mech->nt > mech->ns)
+    if (!ctx || !mech || mech->ns != ctx->ny || mech->nt < 0 || mech->nt > mech->ns || !chem::mech_ok(mech))
         return SHCFD_E_ARG;
     if (!ctx->dmech) HIPCHK(hipMalloc((void**)&ctx->dmech, sizeof(shcfd_mech)));
     HIPCHK(hipMemcpy(ctx->dmech, mech, sizeof(shcfd_mech), hipMemcpyHostToDevice));

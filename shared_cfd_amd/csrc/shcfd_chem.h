@@ -695,6 +695,33 @@ SHCFD_HD void rho_rel2abs(const shcfd_mech* m, double p, double T, double* vrho,
     rho = r;
 }
 
+// A table's indices are used as they are: SVec elements, LDS rows and the
+// table's own arrays are addressed by them.  The parser writes none outside its
+// arrays; a table handed in is looked over before its first use.
+inline bool transport_ok(const shcfd_mech* m) {
+    if (m->nt > SHCFD_CHEM_MAX_NS) return false;
+    for (int i = 0; i < m->nt; i++)
+        if (m->tr2th[i] < 0 || m->tr2th[i] >= m->ns) return false;
+    return true;
+}
+inline bool mech_ok(const shcfd_mech* m) {
+    if (m->ns < 1 || m->ns > SHCFD_CHEM_MAX_NS || m->nr < 1 || m->nr > SHCFD_CHEM_MAX_NR || !transport_ok(m))
+        return false;
+    auto species = [m](int k) { return k >= 0 && k < m->ns; };
+    for (int i = 0; i < m->nr; i++) {
+        for (int s = 0; s < 2; s++) {
+            if (m->num_nu[i][s] > 3) return false;
+            for (int k = 0; k < m->num_nu[i][s]; k++)
+                if (!species(m->ind_nu[i][s][k])) return false;
+        }
+        if (!m->exist_m[i]) continue;
+        if (m->num_m[i] > SHCFD_CHEM_MAX_NS) return false;
+        for (int k = 0; k < m->num_m[i]; k++)
+            if (!species(m->ind_m[i][k])) return false;
+    }
+    return true;
+}
+
 // calc_T: sub_chem.f90:1507-1645 with ns_tocalc = ns.  T is the Newton start
 // on entry.  Returns the iteration count, or -1 past max_T_loop = 1000.
 template <int NS>

@@ -62,10 +62,6 @@ void launch0d_ns(int ns, int op, const shcfd_mech* dm, int n, const double* din,
     }
 }
 
-bool mech_ok(const shcfd_mech* m) {
-    return m->ns >= 1 && m->ns <= SHCFD_MAX_NY && m->nr >= 1 && m->nr <= SHCFD_CHEM_MAX_NR;
-}
-
 template <int NS>
 int boundary_state(const shcfd_mech* m, double p, double T, const double* vrho_rel, double* w, double* vhi,
                    double* dhi) {
@@ -133,7 +129,7 @@ extern "C" {
 
 int shcfd_chem_eval_noalloc(const shcfd_mech* m, int op, int n, const double* in, double* out, int* status,
                             double dt) {
-    if (!m || n < 0 || !in || !out || !mech_ok(m)) return SHCFD_E_ARG;
+    if (!m || n < 0 || !in || !out || !chem::mech_ok(m)) return SHCFD_E_ARG;
     const int ldi = row_in(op, m->ns), ldo = row_out(op, m->ns);
     if (ldi < 0) return SHCFD_E_ARG;
     if (n == 0) return SHCFD_OK;
@@ -165,7 +161,7 @@ int shcfd_chem_eval_noalloc(const shcfd_mech* m, int op, int n, const double* in
 
 int shcfd_chem_boundary_state(const shcfd_mech* m, double p, double T, const double* vrho_rel, double* w,
                               double* vhi, double* dhi) {
-    if (!m || !vrho_rel || !w || !vhi || !(p > 0.0) || !(T > 0.0)) return SHCFD_E_ARG;
+    if (!m || !vrho_rel || !w || !vhi || !(p > 0.0) || !(T > 0.0) || !chem::transport_ok(m)) return SHCFD_E_ARG;
     switch (m->ns) {
 #define SHCFD_NS_CASE(N) case N: return boundary_state<N>(m, p, T, vrho_rel, w, vhi, dhi);
     SHCFD_NS_CASE(1) SHCFD_NS_CASE(2) SHCFD_NS_CASE(3) SHCFD_NS_CASE(4) SHCFD_NS_CASE(5) SHCFD_NS_CASE(6)
@@ -213,7 +209,7 @@ int shcfd_load_nasa9(shcfd_ctx* ctx, const char* chem_inp, const char* thermo_in
 }
 
 int shcfd_chem_eval(const shcfd_mech* m, int op, int n, const double* in, double* out, int* status, double dt) {
-    if (!m || n < 0 || !in || !out || !mech_ok(m)) return SHCFD_E_ARG;
+    if (!m || n < 0 || !in || !out || !chem::mech_ok(m)) return SHCFD_E_ARG;
     int ldi = row_in(op, m->ns), ldo = row_out(op, m->ns);
     if (ldi < 0) return SHCFD_E_ARG;
     if (n == 0) return SHCFD_OK;

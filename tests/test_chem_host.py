@@ -1,7 +1,7 @@
 """Host-side chemistry of the library (no GPU): boundary states and the
 parser of the 9-species test mechanism, against the CPU oracle; the
 production rates Jex forms beside the Jacobian, against Fex; tables with more
-transport entries than species."""
+transport entries than species, and with indices of no species."""
 import ctypes
 import os
 import subprocess
@@ -96,3 +96,35 @@ def test_more_transport_entries_than_species(tmp_path, extra):
     mu = O.chem_calc_t(om, vrho, rho, E, 1500.0)[1][2]
     assert float(r.stdout) == mu
     assert chem.boundary_state(lm, 1.01325e5, 1500.0, rel)[0][8 + 7] == mu
+
+
+TRANSPORT = [("tr2th[0]", 9), ("tr2th[1]", -1), ("nt", 17)]
+REACTIONS = [("num_nu[0][0]", 4), ("ind_nu[1][1][0]", 9), ("ind_nu[0][0][0]", -1), ("num_m[4]", 17), ("ind_m[4][0]", 9)]
+
+
+@pytest.mark.parametrize("entry,value", TRANSPORT + REACTIONS)
+def test_tables_with_indices_of_no_species_are_refused(mechs, entry, value):
+    """shcfd_chem_eval looks at the table before it looks for a GPU; the
+    boundary states use its transport entries alone."""
+    m = chem.Mech.from_buffer_copy(bytes(mechs["syn"][0]))
+    assert m.nt > 1 and m.exist_m[4] == 1 and m.num_m[4] > 0
+    name, *idx = entry.replace("]", "").split("[")
+    if idx:
+        a = getattr(m, name)
+        for i in idx[:-1]:
+            a = a[int(i)]
+        a[int(idx[-1])] = value
+    else:
+        setattr(m, name, value)
+    x, out, st = np.zeros(10), np.zeros(10), np.zeros(1, np.int32)
+    dp, ip = ctypes.POINTER(ctypes.c_double), ctypes.POINTER(ctypes.c_int)
+    L = chem._lib()
+    for call in (L.shcfd_chem_eval, L.shcfd_chem_eval_noalloc):
+        rc = call(ctypes.byref(m), chem.FEX, 1, x.ctypes.data_as(dp), out.ctypes.data_as(dp), st.ctypes.data_as(ip),
+                  ctypes.c_double(0.0))
+        assert rc == 1  # SHCFD_E_ARG
+    if (entry, value) in TRANSPORT:
+        with pytest.raises(ValueError):
+            chem.boundary_state(m, 1.01325e5, 1000.0, np.ones(9))
+    else:
+        chem.boundary_state(m, 1.01325e5, 1000.0, np.ones(9))

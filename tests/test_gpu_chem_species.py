@@ -66,3 +66,20 @@ def test_more_transport_entries_than_species(tmp_path, extra):
             Solver(case)
     else:
         Solver(case).close()
+
+
+@pytest.mark.parametrize("entry", ["ind_nu", "ind_m", "num_nu", "num_m"])
+def test_flow_refuses_tables_with_indices_of_no_species(entry):
+    m = chem.parse(NO27)
+    case = C.mixing_layer(m, ni=8, nj=6, fuel=np.eye(8)[2], ox=np.eye(8)[1])
+    r = next(i for i in range(m.nr) if m.exist_m[i] and m.num_m[i])
+    if entry == "ind_nu":
+        m.ind_nu[r][0][0] = 8
+    elif entry == "ind_m":
+        m.ind_m[r][0] = -1
+    elif entry == "num_nu":
+        m.num_nu[r][1] = 4
+    else:
+        m.num_m[r] = 17
+    with pytest.raises(RuntimeError, match="shcfd_set_mechanism"):
+        Solver(case)
