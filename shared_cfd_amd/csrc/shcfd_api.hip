@@ -627,12 +627,13 @@ int shcfd_proceed_reaction(shcfd_ctx* ctx) {
         if (rc) return rc;
     }
     ProfScope ps(ctx, PROF_REACTION);
-    if (ctx->p.reaction == SHCFD_REACTION_POINT_IMPLICIT && ctx->ny <= SHCFD_LDS_NEWTON_MAX_NS)
-        DISPATCH_FLOW_NS(ctx->ny, hipLaunchKernelGGL(k_reaction_lds<NS>, dim3((unsigned)(ntiles(ctx) * ctx->tile_rows)),
-                                                     dim3(64), 0, ctx->stream, ctx->dev(), ctx->dtiles,
-                                                     ctx->tile_rows, ctx->dmech))
-    else if (ctx->p.reaction == SHCFD_REACTION_POINT_IMPLICIT)
-        DISPATCH_FLOW_NS(ctx->ny, TILE_LAUNCH((k_reaction<NS, SHCFD_REACTION_POINT_IMPLICIT>), ctx->dmech, nullptr, 0))
+    if (ctx->p.reaction == SHCFD_REACTION_POINT_IMPLICIT)
+        DISPATCH_FLOW_NS(ctx->ny,
+                         if constexpr (NS <= SHCFD_LDS_NEWTON_MAX_NS)
+                             hipLaunchKernelGGL(k_reaction_lds<NS>, dim3((unsigned)(ntiles(ctx) * ctx->tile_rows)),
+                                                dim3(64), 0, ctx->stream, ctx->dev(), ctx->dtiles, ctx->tile_rows,
+                                                ctx->dmech);
+                         else TILE_LAUNCH((k_reaction<NS, SHCFD_REACTION_POINT_IMPLICIT>), ctx->dmech, nullptr, 0))
     else {
         // CHEMEQ2, then DVODE for the cells it hands over (sub_chem.f90:1751-1770):
         // the list is emptied, filled by the CHEMEQ2 pass and drained by a

@@ -118,6 +118,7 @@ SHCFD_HD double fmin2(double a, double b) { return (a < b || b != b) ? a : b; }
 // a chain of compares, ends up in scratch or LDS memory.
 template <int N>
 struct SVec {
+    static_assert(N >= 1 && N <= 16, "the widest vector type");
 #if defined(__HIP_DEVICE_COMPILE__)
     typedef double V __attribute__((ext_vector_type(N <= 2 ? 2 : N <= 4 ? 4 : N <= 8 ? 8 : 16)));
     V v;

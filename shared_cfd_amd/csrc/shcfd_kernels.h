@@ -34,6 +34,11 @@
 // three waves per CU; 11 species would leave two); above it the register
 // kernel runs
 #define SHCFD_LDS_NEWTON_MAX_NS 10
+#if SHCFD_INST_GROUP <= 2  // the counts up to SHCFD_LDS_NEWTON_MAX_NS
+#define SHCFD_FOR_EACH_LDS_NS(X) SHCFD_FOR_EACH_NY(X)
+#else
+#define SHCFD_FOR_EACH_LDS_NS(X)
+#endif
 
 namespace shcfd {
 
