@@ -502,10 +502,13 @@ struct MLds {
     double x[2][16][4 * C];    // the unknowns of each row's cell
 };
 
-// prefetch distance, in steps: up to four waves have a SIMD's 512 registers
-// each, more share them
+// prefetch distance, in steps, as far as the registers go without scratch: up
+// to four waves have a SIMD's 512 registers each, more waves half of them.
+// Eight steps of preconditioned LU-SGS on 223 x 99, in ms, one / two / three
+// steps ahead: nY = 9 5.8 / 5.5 / 5.4, nY = 12 13.3 / 13.3 / 26.6, nY = 13 15.1 /
+// 20.9 / 32.3 (from two on the rows spill), nY = 16 22.6 / 37.6 / 49.2
 template <int NY>
-constexpr int pdm() { return NY <= 9 ? 3 : NY <= 13 ? 2 : 1; }
+constexpr int pdm() { return NY <= 9 ? 3 : NY <= 12 ? 2 : 1; }
 
 template <int NY, bool BWD>
 __global__ void __launch_bounds__(64 * ((NY + 6) / 4 + 1))
