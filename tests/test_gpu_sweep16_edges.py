@@ -17,7 +17,10 @@ import numpy as np
 import pytest
 
 from shared_cfd_amd import cases as C
+from shared_cfd_amd import chem
 from shared_cfd_amd.native import OPT_JVP_SWEEP, OPT_SKEW_SWEEP, Solver
+
+from chem_cases import NO27, no27_plus_inert
 
 pytestmark = pytest.mark.gpu
 
@@ -64,3 +67,19 @@ def test_strip_edges_stored_matrices(scheme, ny, ni, nj):
     for a, b in zip(_increments(case, 1, 2, jvp=0), _increments(case, 0, 2)):
         assert np.max(np.abs(b)) > 0.0
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("inert", [0, 1, 4, 8])
+def test_closed_form_with_a_mechanism(tmp_path, inert):
+    """One step of a disturbed mixing layer: every species' DHi, the first's too,
+    from the thermodynamics, which both sides evaluate on the same state."""
+    ns = 8 + inert
+    lm = chem.parse(no27_plus_inert(str(tmp_path), inert)[0] if inert else NO27)
+    rng = np.random.default_rng(ns)
+    fuel, ox = rng.uniform(0.01, 0.1, ns), rng.uniform(0.01, 0.1, ns)
+    case = C.mixing_layer(lm, ni=31, nj=33, reaction=0, fuel=fuel / fuel.sum(), ox=ox / ox.sum())
+    case.q0[0] = case.q0[0] * (1.0 + 0.1 * rng.random(case.q0[0].shape[:2]))[..., None]
+    a, b = _increments(case, 1, 1)[0], _increments(case, 0, 1)[0]
+    scale = np.max(np.abs(b), axis=(0, 1))
+    assert np.all(scale > 0.0)
+    assert np.all(np.max(np.abs(a - b), axis=(0, 1)) <= 16 * (31 + 33) * np.finfo(float).eps * scale)
