@@ -292,11 +292,12 @@ __global__ void __launch_bounds__(64) k_chem0d(const shcfd_mech* __restrict__ m,
     template __global__ void k_thermo_chem<NS>(DevCtx, const Tile*, const shcfd_mech*);                         \
     template __global__ void k_reaction<NS, SHCFD_REACTION_CHEMEQ2>(DevCtx, const Tile*, const shcfd_mech*,     \
                                                                     double*, int);                              \
-    template __global__ void k_reaction<NS, SHCFD_REACTION_POINT_IMPLICIT>(DevCtx, const Tile*,                 \
-                                                                           const shcfd_mech*, double*, int);    \
     template __global__ void k_reaction_dvode<NS>(DevCtx, const shcfd_mech*, const double*, int);
 #define SHCFD_CHEM_LDS_INST(NS) \
     template __global__ void k_reaction_lds<NS>(DevCtx, const Tile*, int, const shcfd_mech*);
+#define SHCFD_CHEM_REG_INST(NS)                                                                             \
+    template __global__ void k_reaction<NS, SHCFD_REACTION_POINT_IMPLICIT>(DevCtx, const Tile*,             \
+                                                                           const shcfd_mech*, double*, int);
 #define SHCFD_CHEM0D_OP(NS, OP) \
     template __global__ void k_chem0d<NS, OP>(const shcfd_mech*, int, const double*, int, double*, int, int*, double);
 #define SHCFD_CHEM0D_INST(NS)                                                                     \
@@ -305,6 +306,7 @@ __global__ void __launch_bounds__(64) k_chem0d(const shcfd_mech* __restrict__ m,
     SHCFD_CHEM0D_OP(NS, CHEM_OP_POINT_IMPLICIT) SHCFD_CHEM0D_OP(NS, CHEM_OP_DVODE)
 SHCFD_FOR_EACH_FLOW_NS(SHCFD_CHEM_FLOW_INST)
 SHCFD_FOR_EACH_LDS_NS(SHCFD_CHEM_LDS_INST)
+SHCFD_FOR_EACH_REG_NS(SHCFD_CHEM_REG_INST)
 SHCFD_FOR_EACH_NS(SHCFD_CHEM0D_INST)
 
 }  // namespace shcfd

@@ -36,8 +36,10 @@
 #define SHCFD_LDS_NEWTON_MAX_NS 10
 #if SHCFD_INST_GROUP <= 2  // the counts up to SHCFD_LDS_NEWTON_MAX_NS
 #define SHCFD_FOR_EACH_LDS_NS(X) SHCFD_FOR_EACH_NY(X)
+#define SHCFD_FOR_EACH_REG_NS(X)
 #else
 #define SHCFD_FOR_EACH_LDS_NS(X)
+#define SHCFD_FOR_EACH_REG_NS(X) SHCFD_FOR_EACH_NY(X)
 #endif
 
 namespace shcfd {
