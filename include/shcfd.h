@@ -137,7 +137,8 @@ int shcfd_check_error(shcfd_ctx *ctx);
 int shcfd_mech_parse(const char *chem_inp, const char *mw_inp, const char *trans_inp, shcfd_mech *out, char *errbuf,
                      int errlen);
 /* make mech the context's mechanism (the reference's module chem state, set
- * up by init_therm); mech->ns must equal nY */
+ * up by init_therm); mech->ns must equal nY.  SHCFD_E_ARG for a table with more
+ * transport entries than species or with an index of no species. */
 int shcfd_set_mechanism(shcfd_ctx *ctx, const shcfd_mech *mech);
 /* init_therm of the reactive model (store/therm_lib/chemkin/flow/reactive/
  * main.part_init.f90 -> read_cheminp, set_trans_data, control_chem.inp
@@ -197,7 +198,9 @@ int shcfd_chem_boundary_state(const shcfd_mech *mech, double p, double T, const 
  *   SHCFD_CHEM_DVODE    in vrho(ns),T       out vrho(ns)   reaction (DVODE over dt), sub_chem.f90:1236-1315
  * status[i] (may be NULL): Newton iterations / CHEMEQ2 attempts (11: DVODE
  * finished the interval) / DVODE steps, or -code.
- * Synchronous; allocates and frees its own device buffers. */
+ * SHCFD_E_ARG for a table with an index of no species; a species may have more
+ * than one transport entry.  Synchronous; allocates and frees its own device
+ * buffers. */
 int shcfd_chem_eval(const shcfd_mech *mech, int op, int nstates, const double *in, double *out, int *status,
                     double dt);
 /* No counterpart in the reference.  For callers that cannot allocate device

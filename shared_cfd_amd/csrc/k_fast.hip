@@ -310,9 +310,10 @@ __device__ inline int col_off(int col) { return (col + HOFF) * 32; }
 //
 // What bounds the sweep is the issue of the compute wave: 9 FP64 operations
 // (about 8 cycles each), 8 DPP moves and 7 LDS accesses per step, 148 cycles
-// in isolation and 170 beside the loader, against a dependent chain of about
-// 105 (v -> quad rotations -> four multiply-adds -> the neighbour row's lanes
-// -> next v).  So the operator rows are stored rotated (own component first:
+// in isolation and 170 (74 ns) beside the loader, against 86 (35.8 ns) for the
+// same step with all operands in registers and 78 for its dependent chain alone
+// (v -> quad rotations -> four multiply-adds -> the neighbour row's lanes -> next
+// v).  So the operator rows are stored rotated (own component first:
 // 6 moves instead of 8 broadcasts), the next right-hand side opens the chain
 // of a, and the neighbour value is read before the operators, which the step
 // after next needs.  Within a 16-lane row of the wavefront (four grid rows)
@@ -322,8 +323,8 @@ __device__ inline int col_off(int col) { return (col + HOFF) * 32; }
 // DPP moves per step.
 //
 // Measured, forward / backward us per launch: 258,048-cell forward step 167 /
-// 152 -> 135 / 122; 512x128 C-mesh 84 / 87 -> 65 / 66; 400x4 tube 47 / 47 ->
-// 29 / 33 (one strip: 112 -> 75 ns per step).  A hop between strips costs 18
+// 152 -> 133 to 140 / 124; 512x128 C-mesh 84 / 87 -> 64 / 67; 400x4 tube 47 / 47 ->
+// 30 / 33 (one strip: 112 -> 75 ns per step).  A hop between strips costs 18
 // steps of skew, up to 5 of chunk granularity and 1.3 us from the producer's
 // store to the consumer's look.
 constexpr int CS = 4;                                   // steps per LDS chunk
@@ -585,7 +586,8 @@ __device__ inline void courier_in(double* ring, __amdgpu_buffer_rsrc_t rin, bool
 
 // wave 3: the strip's outgoing columns (lanes at `edge` of the ring) to its
 // hand-off row after chunk j's barrier (late_out: up to the step before the
-// chunk's last, whose terms follow with the next chunk's).  Step e gives column col0 + e (forward) or col0 - e (backward).
+// chunk's last, whose terms follow with the next chunk's).  Step e gives column
+// col0 + e (forward) or col0 - e (backward).
 template <int RS, bool BWD>
 __device__ inline void courier_out(const double* ring, __amdgpu_buffer_rsrc_t rout, bool present, int col0, int edge,
                                    int nck, int L) {

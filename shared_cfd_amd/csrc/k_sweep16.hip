@@ -95,8 +95,8 @@ __device__ inline void load_ops(const double* __restrict__ base, StepIn<DQ>& in)
 // Bound by the chain of one step, 240 ns: 17 FP64 operations (about 8 cycles
 // each from one wave), the DPP moves and two LDS round trips, beside 5 loads of
 // 64 x 16 bytes per wave; then by the hand-off, a strip running 18 steps plus
-// about 4 us behind its neighbour.  Measured at nY = 9: 575 us forward and
-// 545 us backward on 1024 x 512 (before 1285 and 986), 109 and 110 us on
+// about 4 us behind its neighbour.  Measured at nY = 9: 571 us forward and
+// 542 us backward on 1024 x 512 (before 1285 and 986), 108 and 109 us on
 // 223 x 99 (before 200 and 210); forming the records and the right-hand side
 // in one pass, 195 us on 1024 x 512 (before, cell data 104 us and right-hand
 // side 78 us in two), the update 56 us.  Before, dq was read and written in
@@ -454,8 +454,8 @@ k_sweep16j(DevCtx d, const Strip16* strips, int nstrips, double* hand, long long
 //
 // Bound by the matrix rows: 43 KB per step at nY = 9 through one CU's 64 bytes
 // per cycle (280 ns of the 400 ns of a step), beside 48 dependent FP64
-// operations; then by the hand-off.  Measured at nY = 9 on 223 x 99: 249 us
-// forward and 245 us backward (before, dq and q read and written in place and
+// operations; then by the hand-off.  Measured at nY = 9 on 223 x 99: 239 us
+// forward and 243 us backward (before, dq and q read and written in place and
 // the hand-off polled by the computing waves, 327 and 447 us); prefetching
 // four steps instead of three 260 us, since the rows then pass through
 // accumulation registers.

@@ -31,8 +31,10 @@
 #define SHCFD_FOR_EACH_FLOW_NS(X) SHCFD_FOR_EACH_NY(X)
 // the point-implicit kernels keep each lane's (NS+1)^2 Newton matrix, but for
 // two columns, in LDS up to this species count (64 lanes x 99 doubles = 51 KB,
-// three waves per CU; 11 species would leave two); above it the register
-// kernel runs
+// three waves per CU); above it the register kernel runs.  Six steps on 223 x
+// 99, LDS / registers in ms: ten species 3.1 / 5.3, eleven (two waves per CU) 3.3
+// / 6.2, twelve 3.6 / 7.3: the line lies where it was drawn from the waves alone,
+// and could move up.
 #define SHCFD_LDS_NEWTON_MAX_NS 10
 #if SHCFD_INST_GROUP <= 2  // the counts up to SHCFD_LDS_NEWTON_MAX_NS
 #define SHCFD_FOR_EACH_LDS_NS(X) SHCFD_FOR_EACH_NY(X)
